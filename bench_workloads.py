@@ -144,14 +144,26 @@ def sweep_small(checker):
 
 
 def grad_executed_flops(n):
-    """Flops the single-sweep gradient executes per n x n matrix: per Gray step of a group of
-    G columns a row flip (2n), n + 2G - 5 complex multiplies (6 each), G running sums (2
-    each) and G corrector FMAs (4 each), 8n + 18G - 30 flops, over 2^(n-1) steps; groups of
-    8 columns, the last 1..4 columns (n mod 8) in one group of 4, else ceil(n/8) groups of 8
-    (the last overlapping its predecessor)."""
+    """Flops of the gradient as one Gray sweep per group of G columns: per step a row flip
+    (2n), n + 2G - 5 complex multiplies (6 each), G running sums (2 each) and G corrector FMAs
+    (4 each), 8n + 18G - 30 flops, over 2^(n-1) steps; groups of 8 columns, the last 1..4
+    columns (n mod 8) in one group of 4, else ceil(n/8) groups of 8 (the last overlapping its
+    predecessor). The kernel shares one sweep among all columns and executes fewer
+    (grad_sweep_flops)."""
     full, rest = divmod(n, 8)
     groups = [8] * full + ([4] if 0 < rest <= 4 else [8] if rest else [])
     return 2 ** (n - 1) * sum(8 * n + 18 * g - 30 for g in groups)
+
+
+def grad_sweep_flops(n):
+    """Flops the gradient sweep executes per n x n matrix (n >= 6): per Gray code, on L lanes
+    of C = ceil(n / L) columns each (padding included), a row flip, a running sum and a
+    corrector FMA per column (8 flops) and 3C - 3 complex multiplies per lane, with L = 4 two
+    more for the product of the other lanes (6 flops each)."""
+    lanes = 4 if n <= 8 or n > 18 else 2
+    cols = -(-n // lanes)
+    mults = 3 * cols - 3 + (2 if lanes == 4 else 0)
+    return 2 ** (n - 1) * lanes * (8 * cols + 6 * mults)
 
 
 def glynn_flops(n):
@@ -360,7 +372,7 @@ def grad(checker, cpu=True, tune=True):
     # All n^2 minors by one sweep: 2^(n-1) (2n^2 + 20n) (n column adds, ~3n multiplies for
     # leave-one-out products, n^2 signed accumulations per step).
     f_grad = B * 2 ** (n - 1) * (2 * n * n + 20 * n)
-    f_bwd_exec = B * grad_executed_flops(n)
+    f_bwd_exec = B * grad_sweep_flops(n)
     return {"workload": "permanent + gradient, 64 x n=20",
             "autograd_fwd_bwd_ms": t_pass * 1e3,
             "cpu_baseline": cpu_rec,
@@ -374,12 +386,11 @@ def grad(checker, cpu=True, tune=True):
             "flops_executed": f_bwd_exec, "flops_effective": f_fwd + f_grad,
             "note": "autograd pass: the forward of permanent() on a tensor that requires grad "
                     "runs the gradient launch, which returns perm and all n^2 minors (one Gray "
-                    "sweep per group of 8 columns); the backward scales the kept minors. "
-                    "executed: the flops the sweeps perform, per matrix 2^(n-1) (8n + 114) for "
-                    "each group of 8 columns and 2^(n-1) (8n + 42) for the group of 4 that takes "
-                    "the last n mod 8 <= 4 columns (n = 20: 2 of 8 and 1 of 4) "
-                    "(the FLOP counter reads ~1.2x this: FMAs with a +-1 or +-2 operand "
-                    "count 2); _kernels: over the gradient launches alone, without the autograd "
+                    "sweep per matrix); the backward scales the kept minors. executed: the "
+                    "flops the sweep performs (n = 20: 496 per Gray code; row flips, running "
+                    "sums and correctors 8 per column, 14 complex multiplies on each of 4 "
+                    "lanes of 5 columns); _kernels: over the gradient launches alone, without "
+                    "the autograd "
                     "host work. effective: algorithm-equivalent flops, a Glynn forward (8n - 4) 2^(n-1) "
                     "plus the all-minors count 2^(n-1)(2n^2 + 20n) per matrix, which charges "
                     "more than the single sweep executes (not a roofline fraction)"}

@@ -76,7 +76,7 @@ int32_t tb_device_count(void);
  * waves per permanent -- from this table when a call does not set one:
  *   TB_TUNE_SWEEP  C&C minors sweep, size = k (also the steps of tb_gccb_sample)
  *   TB_TUNE_GLYNN  tb_glynn_batch, size = n
- *   TB_TUNE_GRAD   single-sweep gradient of tb_perm_grad_batch, size = n
+ *   TB_TUNE_GRAD   gradient sweep of tb_perm_grad_batch, size = n
  * Entries are kept per batch bucket: the batch of a launch (matrices, sweep items, or
  * samples of tb_gccb_sample) falls in bucket ceil(log2(batch)), i.e. 1 | 2 | 3-4 | 5-8 |
  * ... | above 2^(TB_TUNE_BATCH_BUCKETS - 2), because the best chunk for one permanent is
@@ -203,10 +203,9 @@ int32_t tb_sweep_minors_batch(const tb_complex128 *Vt, int32_t k, int32_t ldv,
  * Permanent and its gradient d perm(A) / d A[i][j] = perm(A without row i, column j)
  * for a batch of n x n matrices. No reference counterpart (the reference has no
  * differentiation); row i of the gradient is what the C&C submatrices calculator returns
- * with row i deleted. For 14 <= n <= 26 one Gray sweep per group of 8 columns yields
- * all n rows of those columns (leave-one-out products and per-row correctors); other n
- * run one C&C minors sweep per deleted row. Both recompute instead of storing
- * per-subset sums.
+ * with row i deleted. From n = 6 on one Gray sweep per matrix yields all n rows and columns
+ * (leave-one-out products over lanes that share the columns, and per-row correctors); up to
+ * n = 5 the minors are expanded directly. Nothing is stored per subset.
  *   perm_out   batch permanents (Laplace expansion of the gradient along row 0)
  *   grad_out   batch x n x n
  * ------------------------------------------------------------------------------- */
@@ -215,6 +214,12 @@ int32_t tb_perm_grad_batch(const tb_complex128 *A, int32_t n, int32_t batch,
                            int64_t matrix_stride, tb_complex128 *perm_out,
                            tb_complex128 *grad_out, void *workspace, size_t workspace_bytes,
                            void *stream);
+/* The same with every entry of grad_out conjugated (the factor that a gradient in the
+ * conjugate-Wirtinger convention multiplies by); perm_out is not conjugated. */
+int32_t tb_perm_grad_conj_batch(const tb_complex128 *A, int32_t n, int32_t batch,
+                                int64_t matrix_stride, tb_complex128 *perm_out,
+                                tb_complex128 *grad_out, void *workspace, size_t workspace_bytes,
+                                void *stream);
 
 /* ---------------------------------------------------------------------------------
  * Batched generalized Clifford & Clifford (GCC-B) sampler.

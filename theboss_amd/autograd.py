@@ -4,10 +4,11 @@ forward:  perm(A) for a batch of n x n complex128 matrices. When A requires grad
           gradient launch (tb_perm_grad_batch) yields the permanents and all n^2 minors
           d perm / d A_ij = perm(A without row i and column j); the minors (B x n x n) are
           kept for the backward pass. Otherwise the Glynn kernel computes perm alone.
-backward: grad_out times the kept minors. Per-subset sums are recomputed inside the
-          sweep, never stored.
+backward: grad_out times the kept minors, one pass over them. Per-subset sums are
+          recomputed inside the sweep, never stored.
 The permanent is holomorphic, so in PyTorch's conjugate-Wirtinger convention the
-incoming gradient g maps to g * conj(d perm / d A).
+incoming gradient g maps to g * conj(d perm / d A); the gradient launch writes the minors
+conjugated, so that the backward does not conjugate them in a pass of its own.
 """
 from . import _device as D
 from . import ops
@@ -24,15 +25,15 @@ def _make_function():
         @staticmethod
         def forward(ctx, A):
             if ctx.needs_input_grad[0]:
-                perm, G = ops.perm_grad_batch(A.detach())
-                ctx.save_for_backward(G)
+                perm, Gc = ops.perm_grad_batch(A.detach(), conj=True)
+                ctx.save_for_backward(Gc)
                 return perm
             return ops.glynn_batch(A.detach())
 
         @staticmethod
         def backward(ctx, grad_out):
-            (G,) = ctx.saved_tensors
-            return grad_out.reshape(-1, 1, 1) * G.conj()
+            (Gc,) = ctx.saved_tensors
+            return grad_out.reshape(-1, 1, 1) * Gc
 
     return _Permanent
 

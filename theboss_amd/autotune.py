@@ -121,33 +121,33 @@ def glynn_builtin(n: int, batch: int) -> int:
 
 
 def grad_columns(n: int) -> int:
-    """Columns per sweep of the gradient kernel at n (8 for 14 <= n <= 26)."""
-    return 8 if 14 <= n <= 26 else 4
+    """Columns whose minors one sweep of the gradient kernel yields: all of them."""
+    return n
+
+
+def _grad_lane_bits(n: int) -> int:
+    """log2 of the lane groups of a wave that walk codes of their own (groups of 4 or 2)."""
+    return 4 if n <= 8 or n > 18 else 5
 
 
 def grad_static_bits(n: int) -> int:
-    return 2 if grad_columns(n) == 8 else (4 if n <= 19 else 3)
+    lanes = _grad_lane_bits(n)
+    u = (4 if n <= 16 else 3) if lanes == 5 else 4 if 8 < n <= 32 else 2
+    return min(u, n - 1 - lanes)
 
 
 def grad_builtin(n: int, batch: int) -> int:
-    """The gradient's built-in chunk: ~8192 waves, then up to two sizes larger while the
-    main launch's rounds of 2 x 1024 waves stay as full, scored by round fill times the
-    share of a chunk left after seeding, 4n(n - 1) / ((8n + 18G - 30) 2^c)."""
-    nb = n - 1
-    g = grad_columns(n)
-    groups = (n + g - 1) // g
-    main = n // g if g == 8 and 0 < n % 8 <= 4 else groups  # the 4-column tail apart
-    want = 0
-    while (batch * groups << want) < 8192 and want < 30:
-        want += 1
-    low = grad_static_bits(n)
-    if main != groups:  # the tail launch's 4-column groups need their static bits too
-        low = max(low, 4 if n <= 19 else 3)
-    c0 = min(max(min(nb - 6 - want, 11), low), nb - 7)
-    best, best_c = -1.0, c0
-    for c in range(c0, min(c0 + 2, 11, nb - 7) + 1):
-        rounds = batch * main * 2.0 ** (nb - c - 6) / 2048
-        score = rounds / math.ceil(rounds) * (1 - 4.0 * n * (n - 1) / ((8 * n + 18 * g - 30) * 2.0 ** c))
+    """The gradient's built-in chunk (n >= 6): the best product of the SIMDs' fill, the issue
+    rate that so many waves per SIMD reach and the share of a chunk left after its seed and
+    end (about 10 steps)."""
+    nb, u, lanes = n - 1, grad_static_bits(n), _grad_lane_bits(n)
+    top = min(max(11, u), nb - lanes)
+    best, best_c = -1.0, top
+    for c in range(top, u - 1, -1):
+        w = batch * 2.0 ** (nb - c - lanes) / 1024.0
+        up = math.ceil(w)
+        rate = 0.83 if up < 2 else 0.97 if up < 3 else 1.0
+        score = w / up * rate / (1 + 10.0 / 2.0 ** c)
         if score > best + 1e-9:
             best, best_c = score, c
     return best_c
@@ -235,16 +235,17 @@ def tune_glynn(ns: Iterable[int], batch: int, spread: int = 2, reps: int = 2,
 
 def tune_grad(ns: Iterable[int], batch: int, spread: int = 2, reps: int = 3,
               seed: int = 0) -> Dict[int, dict]:
-    """Single-sweep gradient (14 <= n <= 26) over a batch of `batch` matrices."""
+    """Gradient sweep (n >= 14; smaller ones are sub-millisecond launches) over a batch of
+    `batch` matrices."""
     out = {}
     for n in ns:
-        if not 14 <= n <= 26:
+        if not 14 <= n <= L.TB_SWEEP_MAX_K:
             continue
         A = D.to_device_c128(np.stack([_haar_block(2 * n, 2 * n, seed + 37 * n + b)[:n, :n]
                                        for b in range(batch)]))
         u = grad_static_bits(n)
         c0 = grad_builtin(n, batch)
-        cands = _candidates(c0, u, min(11, n - 8), spread)
+        cands = _candidates(c0, u, min(11, n - 7), spread)
         out[n] = _pick("grad", n, batch, cands, c0, lambda: ops.perm_grad_batch(A), reps)
     return out
 

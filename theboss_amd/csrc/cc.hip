@@ -11,10 +11,9 @@ int32_t run_sweep(int k, const tb::cd *Vt, int ldv, int64_t item_stride, const i
                   tb::cd *minors, hipStream_t s);
 }  // namespace tbs
 namespace tbgr {
-bool grad_supported(int n);
-size_t grad_partial_bytes(int n, int batch, int c_pref);
-int32_t run_grad(int n, const tb::cd *A, int64_t mstride, int batch, int c_pref, tb::cd *partial,
-                 tb::cd *grad, hipStream_t s);
+size_t grad_workspace(int n, int batch, int c_pref);
+int32_t run_grad(int n, const tb::cd *A, int64_t mstride, int batch, int c_pref, int conj,
+                 tb::cd *partial, tb::cd *grad, tb::cd *perm, hipStream_t s);
 }  // namespace tbgr
 namespace tbg {
 int32_t run_guan(const tb::cd *U, int ldu, const int *out_modes, const int *out_mult, int out_max,
@@ -79,36 +78,6 @@ __global__ void cc_scatter_kernel(const cd *__restrict__ compact, const int *__r
 __global__ void cc_single_kernel(const int *__restrict__ in_mult, int n, cd *__restrict__ minors) {
   const int idx = blockIdx.x * blockDim.x + threadIdx.x;
   if (idx < n) minors[idx] = {(double)in_mult[idx], 0.0};
-}
-
-// Gradient items (b, r): Vt[nu][j'] = A[b][row j' (skipping r)][nu].
-__global__ void grad_gather_kernel(const cd *__restrict__ A, int n, int batch, int64_t mstride,
-                                   cd *__restrict__ Vt) {
-  const int R = n - 1;
-  const int64_t per_item = (int64_t)n * R;
-  const int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (idx >= (int64_t)batch * n * per_item) return;
-  const int64_t item = idx / per_item;
-  const int rem = (int)(idx - item * per_item);
-  const int nu = rem / R, jp = rem - nu * R;
-  const int b = (int)(item / n), r = (int)(item - (int64_t)b * n);
-  const int row = jp < r ? jp : jp + 1;
-  Vt[idx] = A[(size_t)b * mstride + (size_t)row * n + nu];
-}
-
-// perm[b] = sum_nu A[b][0][nu] * G[b][0][nu] (Laplace expansion along row 0).
-__global__ void grad_perm_kernel(const cd *__restrict__ A, int n, int batch, int64_t mstride,
-                                 const cd *__restrict__ G, cd *__restrict__ perm) {
-  const int b = blockIdx.x * blockDim.x + threadIdx.x;
-  if (b >= batch) return;
-  double re = 0.0, im = 0.0;
-  for (int nu = 0; nu < n; ++nu) {
-    const cd a = A[(size_t)b * mstride + nu];
-    const cd g = G[(size_t)b * n * n + nu];
-    re += a.re * g.re - a.im * g.im;
-    im += a.re * g.im + a.im * g.re;
-  }
-  perm[b] = {re, im};
 }
 
 __global__ void grad_small_kernel(const cd *__restrict__ A, int n, int batch, int64_t mstride,
@@ -200,32 +169,15 @@ extern "C" int32_t tb_cc_submatrices_batch(const tb_complex128 *U, int32_t ldu,
   return tbh::check_hip(hipGetLastError(), "cc_scatter_kernel");
 }
 
-namespace {
-// c: the tuning entry of the path that n takes (single-sweep gradient over the batch, or
-// n sweeps per matrix over batch * n sweep items).
-int grad_tuned(int n, int batch) {
-  if (tbgr::grad_supported(n)) return tbh::tuned(TB_TUNE_GRAD, n, batch);
-  return tbh::tuned(TB_TUNE_SWEEP, n, (int64_t)batch * n);
-}
-
-size_t grad_workspace_bytes(int n, int batch, int c) {
-  if (n < 2 || batch <= 0 || n > TB_SWEEP_MAX_K) return 0;
-  if (tbgr::grad_supported(n)) return tbgr::grad_partial_bytes(n, batch, c);
-  const int items = batch * n;
-  return align256((size_t)items * n * (n - 1) * sizeof(tb::cd)) +
-         tbs::sweep_partial_bytes(n, items, c);
-}
-}  // namespace
-
 extern "C" size_t tb_perm_grad_workspace_size(int32_t n, int32_t batch) {
   if (n < 2 || n > TB_SWEEP_MAX_K) return 0;
-  return grad_workspace_bytes(n, batch, grad_tuned(n, batch));
+  return tbgr::grad_workspace(n, batch, tbh::tuned(TB_TUNE_GRAD, n, batch));
 }
 
-extern "C" int32_t tb_perm_grad_batch(const tb_complex128 *A, int32_t n, int32_t batch,
-                                      int64_t matrix_stride, tb_complex128 *perm_out,
-                                      tb_complex128 *grad_out, void *workspace,
-                                      size_t workspace_bytes, void *stream) {
+namespace {
+int32_t perm_grad(const tb_complex128 *A, int32_t n, int32_t batch, int64_t matrix_stride,
+                  int conj, tb_complex128 *perm_out, tb_complex128 *grad_out, void *workspace,
+                  size_t workspace_bytes, void *stream) {
   hipStream_t s = (hipStream_t)stream;
   if (batch < 0) return tbh::fail(TB_EINVAL, "grad: batch=%d < 0", batch);
   if (batch == 0) return TB_OK;
@@ -241,31 +193,28 @@ extern "C" int32_t tb_perm_grad_batch(const tb_complex128 *A, int32_t n, int32_t
                        (tb::cd *)grad_out);
     return tbh::check_hip(hipGetLastError(), "grad_small_kernel");
   }
-  const int c = grad_tuned(n, batch);  // read once: size check and launch agree
-  const size_t need = grad_workspace_bytes(n, batch, c);
-  if (!workspace || workspace_bytes < need)
+  const int c = tbh::tuned(TB_TUNE_GRAD, n, batch);  // read once: size check and launch agree
+  const size_t need = tbgr::grad_workspace(n, batch, c);
+  if (need > 0 && (!workspace || workspace_bytes < need))
     return tbh::fail(TB_EWORKSPACE, "grad: workspace %zu bytes < required %zu", workspace_bytes,
                      need);
-  if (tbgr::grad_supported(n)) {  // one sweep per group of 4 or 8 columns
-    int32_t rc = tbgr::run_grad(n, (const tb::cd *)A, matrix_stride, batch, c,
-                                (tb::cd *)workspace, (tb::cd *)grad_out, s);
-    if (rc) return rc;
-  } else {  // one C&C minors sweep per deleted row
-    const int items = batch * n;
-    tb::cd *Vt = (tb::cd *)workspace;
-    tb::cd *partial =
-        (tb::cd *)((char *)workspace + align256((size_t)items * n * (n - 1) * sizeof(tb::cd)));
-    const int64_t total = (int64_t)items * n * (n - 1);
-    hipLaunchKernelGGL(tb::grad_gather_kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0,
-                       s, (const tb::cd *)A, n, batch, matrix_stride, Vt);
-    int32_t rc = tbh::check_hip(hipGetLastError(), "grad_gather_kernel");
-    if (rc) return rc;
-    rc = tbs::run_sweep(n, Vt, n - 1, (int64_t)n * (n - 1), nullptr, nullptr, items, c, partial,
-                        (tb::cd *)grad_out, s);
-    if (rc) return rc;
-  }
-  hipLaunchKernelGGL(tb::grad_perm_kernel, dim3((batch + 255) / 256), dim3(256), 0, s,
-                     (const tb::cd *)A, n, batch, matrix_stride, (const tb::cd *)grad_out,
-                     (tb::cd *)perm_out);
-  return tbh::check_hip(hipGetLastError(), "grad_perm_kernel");
+  return tbgr::run_grad(n, (const tb::cd *)A, matrix_stride, batch, c, conj, (tb::cd *)workspace,
+                        (tb::cd *)grad_out, (tb::cd *)perm_out, s);
+}
+}  // namespace
+
+extern "C" int32_t tb_perm_grad_batch(const tb_complex128 *A, int32_t n, int32_t batch,
+                                      int64_t matrix_stride, tb_complex128 *perm_out,
+                                      tb_complex128 *grad_out, void *workspace,
+                                      size_t workspace_bytes, void *stream) {
+  return perm_grad(A, n, batch, matrix_stride, 0, perm_out, grad_out, workspace, workspace_bytes,
+                   stream);
+}
+
+extern "C" int32_t tb_perm_grad_conj_batch(const tb_complex128 *A, int32_t n, int32_t batch,
+                                           int64_t matrix_stride, tb_complex128 *perm_out,
+                                           tb_complex128 *grad_out, void *workspace,
+                                           size_t workspace_bytes, void *stream) {
+  return perm_grad(A, n, batch, matrix_stride, 1, perm_out, grad_out, workspace, workspace_bytes,
+                   stream);
 }

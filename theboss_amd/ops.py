@@ -111,8 +111,9 @@ def sweep_minors_batch(Vt, k: int):
     return minors
 
 
-def perm_grad_batch(A) -> Tuple["object", "object"]:
-    """perm(A[b]) and d perm / d A[b][i][j] = perm(A[b] without row i, column j)."""
+def perm_grad_batch(A, conj: bool = False) -> Tuple["object", "object"]:
+    """perm(A[b]) and d perm / d A[b][i][j] = perm(A[b] without row i, column j); with conj
+    the minors come conjugated (and the permanents do not)."""
     T = D.require_gpu()
     if A.dim() != 3 or A.shape[1] != A.shape[2]:
         raise ValueError(f"perm_grad_batch expects B x n x n, got {tuple(A.shape)}")
@@ -123,9 +124,9 @@ def perm_grad_batch(A) -> Tuple["object", "object"]:
     lib = L.load()
     need = lib.tb_perm_grad_workspace_size(n, B)
     ws = D.workspace(need, A.device) if need else None
-    L.check(lib.tb_perm_grad_batch(D.ptr(A), n, B, n * n, D.ptr(perm), D.ptr(grad),
-                                   D.ptr(ws) if ws is not None else None, need,
-                                   D.stream_ptr(A.device)))
+    fn = lib.tb_perm_grad_conj_batch if conj else lib.tb_perm_grad_batch
+    L.check(fn(D.ptr(A), n, B, n * n, D.ptr(perm), D.ptr(grad),
+               D.ptr(ws) if ws is not None else None, need, D.stream_ptr(A.device)))
     return perm, grad
 
 
