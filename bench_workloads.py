@@ -74,7 +74,8 @@ class GuanFlops:
     tb_guan_perm_batch and tb_guan_perm_outer launch the calculators make: per item (pair)
     prod_d (e_d + 1) Guan codes, each costing 2|T| + 6(sum t - 1) + 2 (|T| complex adds
     into the sums of the product side's distinct modes, sum t - 1 complex multiplies, the
-    accumulation), with e the enumerated side's multiplicities and t the product side's.
+    accumulation), with e the enumerated side's multiplicities and t the product side's. Calls
+    that take the subset recurrence are charged the same, the walk they replace.
     The count is summed on the device and read once at the end."""
 
     def __enter__(self):
@@ -95,7 +96,8 @@ class GuanFlops:
 
         self._orig_outer = ops.guan_perm_outer
 
-        def counted_outer(U, out_modes, out_mult, in_modes, in_mult, formula=L.TB_FORMULA_RYSER):
+        def counted_outer(U, out_modes, out_mult, in_modes, in_mult, formula=L.TB_FORMULA_RYSER,
+                          common=None):
             # pair (j, i) enumerates the T row j when it has fewer codes than the S row i
             f64 = T.float64
             codes_t, codes_s = (out_mult.to(f64) + 1).prod(dim=1), (in_mult.to(f64) + 1).prod(dim=1)
@@ -106,7 +108,7 @@ class GuanFlops:
             self._acc += T.where(codes_t[:, None] < codes_s[None, :], enum_t, enum_s).sum()
             self.launches += 1
             self.items += int(out_mult.shape[0]) * int(in_mult.shape[0])
-            return self._orig_outer(U, out_modes, out_mult, in_modes, in_mult, formula)
+            return self._orig_outer(U, out_modes, out_mult, in_modes, in_mult, formula, common)
 
         ops.guan_perm_batch = counted
         ops.guan_perm_outer = counted_outer

@@ -164,6 +164,22 @@ int32_t tb_guan_perm_outer(const tb_complex128 *U, int32_t ldu, const int32_t *o
                            const int32_t *in_modes, const int32_t *in_mult, int32_t in_max,
                            int32_t n_in, int32_t formula, tb_complex128 *out, void *stream);
 
+/* tb_guan_perm_outer with a workspace (of tb_guan_outer_workspace_size bytes; 0 = none is
+ * used), which lets it compute all pairs of an output row in one pass: where the input rows lie
+ * below one state of at most 12 modes and 4096 substates (GCC-A's layers, the lossy inputs of
+ * an exact distribution) and hold at most 12 particles, by expansion along the output
+ * particles over that state's substates; the other calls and rows are walked pair by pair.
+ * Same values up to rounding, whatever the formula. The size is 0 for calls too small to gain.
+ * A caller that knows its input rows have no such state passes no workspace: finding that out
+ * on the device takes about 7 us. */
+size_t tb_guan_outer_workspace_size(int32_t ldu, int32_t out_max, int32_t n_out, int32_t in_max,
+                                    int32_t n_in);
+int32_t tb_guan_perm_outer_ws(const tb_complex128 *U, int32_t ldu, const int32_t *out_modes,
+                              const int32_t *out_mult, int32_t out_max, int32_t n_out,
+                              const int32_t *in_modes, const int32_t *in_mult, int32_t in_max,
+                              int32_t n_in, int32_t formula, tb_complex128 *out, void *workspace,
+                              size_t workspace_bytes, void *stream);
+
 /* ---------------------------------------------------------------------------------
  * Clifford & Clifford submatrices permanents: all input-particle-deleted minors in one
  * sweep. Replaces BSCCRyserSubmatricesPermanentCalculator.compute_permanents

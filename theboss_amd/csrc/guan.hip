@@ -225,21 +225,26 @@ __device__ __forceinline__ void guan_item_run(const GuanItemLds &it, int D, int 
 // choose per item on the host: perm(U[t, s]) = perm(U^T[s, t]), so a transposed item
 // swaps the two rows' roles and reads U with swapped strides. Its slots then hold up to
 // max(in_max, out_max) entries on either side.
-template <int JB, int IPW, bool OUTER = false>
-__global__ __launch_bounds__(64) void guan_kernel(const cd *__restrict__ U, int ldu,
-                                                  const int *__restrict__ out_modes,
-                                                  const int *__restrict__ out_mult, int out_max,
-                                                  const int *__restrict__ in_modes,
-                                                  const int *__restrict__ in_mult, int in_max,
-                                                  int batch, int n_in, int formula, int mode,
-                                                  cd *__restrict__ out) {
+template <int JB, int IPW, bool OUTER>
+__device__ __forceinline__ void guan_items(const cd *__restrict__ U, int ldu,
+                                           const int *__restrict__ out_modes,
+                                           const int *__restrict__ out_mult, int out_max,
+                                           const int *__restrict__ in_modes,
+                                           const int *__restrict__ in_mult, int in_max, int batch,
+                                           int n_in, int formula, int mode, int b0,
+                                           const int *__restrict__ done, char *smem,
+                                           cd *__restrict__ out) {
   constexpr int W = 64 / IPW;  // lanes per item in a packed wave
-  extern __shared__ char smem[];
   const int lane = threadIdx.x;
   const int g = lane / W, l = lane % W;
-  const int b0 = blockIdx.x * IPW;
   const int b = b0 + g;
-  const bool live = b < batch;
+  bool live = b < batch;
+  if constexpr (OUTER) {  // rows the subset recurrence has already written
+    if (done != nullptr) {
+      if (live) live = done[b / n_in] == 0;
+      if (!__any(live)) return;
+    }
+  }
   // Slot capacities of the enumerated (columns) and product (rows) sides: wave-uniform.
   const int cap = OUTER ? max(in_max, out_max) : in_max;
   const int pcap = OUTER ? cap : out_max;
@@ -345,7 +350,7 @@ __global__ __launch_bounds__(64) void guan_kernel(const cd *__restrict__ U, int 
   // A large item among the wave's items: walk them one after another with all lanes.
   for (int q = 0; q < IPW; ++q) {
     const int bq = b0 + q;
-    if (bq >= batch) break;
+    if (!__shfl((int)live, q * W, 64)) continue;
     const int Dq = __shfl(D, q * W, 64), Jq = __shfl(J, q * W, 64);
     const int ssq = __shfl(ss, q * W, 64), stq = __shfl(st, q * W, 64);
     const GuanItemLds itq = guan_item_at(items + q * stride, pcap, cap);
@@ -353,6 +358,40 @@ __global__ __launch_bounds__(64) void guan_kernel(const cd *__restrict__ U, int 
     for (int d = 0; d < Dq; ++d) totq *= (uint64_t)(itq.s[d] + 1);
     guan_item_run<JB, 64>(itq, Dq, Jq, ssq, stq, totq, bq, in_max, lane, lane, formula, mode,
                           Macc, rr, uu, out);
+  }
+}
+
+template <int JB, int IPW>
+__global__ __launch_bounds__(64) void guan_kernel(const cd *__restrict__ U, int ldu,
+                                                  const int *__restrict__ out_modes,
+                                                  const int *__restrict__ out_mult, int out_max,
+                                                  const int *__restrict__ in_modes,
+                                                  const int *__restrict__ in_mult, int in_max,
+                                                  int batch, int formula, int mode,
+                                                  cd *__restrict__ out) {
+  extern __shared__ char smem[];
+  guan_items<JB, IPW, false>(U, ldu, out_modes, out_mult, out_max, in_modes, in_mult, in_max, batch,
+                             1, formula, mode, (int)blockIdx.x * IPW, nullptr, smem, out);
+}
+
+// All-pairs form. AFTER: the launch follows the subset recurrence, which has usually done every
+// row, so its grid is bounded and each block loops over its share of the items.
+template <int JB, int IPW, bool AFTER>
+__global__ __launch_bounds__(64) void guan_outer_kernel(
+    const cd *__restrict__ U, int ldu, const int *__restrict__ out_modes,
+    const int *__restrict__ out_mult, int out_max, const int *__restrict__ in_modes,
+    const int *__restrict__ in_mult, int in_max, int batch, int n_in, int formula,
+    const int *__restrict__ done, cd *__restrict__ out) {
+  extern __shared__ char smem[];
+  if constexpr (!AFTER) {
+    guan_items<JB, IPW, true>(U, ldu, out_modes, out_mult, out_max, in_modes, in_mult, in_max,
+                              batch, n_in, formula, 0, (int)blockIdx.x * IPW, nullptr, smem, out);
+  } else {
+    for (int64_t b0 = (int64_t)blockIdx.x * IPW; b0 < batch; b0 += (int64_t)gridDim.x * IPW) {
+      guan_items<JB, IPW, true>(U, ldu, out_modes, out_mult, out_max, in_modes, in_mult, in_max,
+                                batch, n_in, formula, 0, (int)b0, done, smem, out);
+      __syncthreads();  // the next items reuse the LDS blocks
+    }
   }
 }
 
@@ -371,10 +410,14 @@ size_t guan_lds_bytes(int out_max, int in_max, int mode, int ipw) {
   return bytes;
 }
 
-// n_in > 0: the all-pairs form over batch = n_out * n_in items (mode 0 only).
+// n_in > 0: the all-pairs form over batch = n_out * n_in items (mode 0 only); done (may be
+// null): output rows already written. Those launches use a bounded grid, since the walk is
+// then the exception (1.0M pairs all done: 126,000 one-wave blocks that only read their flag
+// take 15 us longer than 4096; nothing done: the bounded grid takes 350 us instead of 356).
+constexpr int kGuanAfterRecurrenceBlocks = 4096;
 int32_t run_guan(const tb::cd *U, int ldu, const int *out_modes, const int *out_mult, int out_max,
                  const int *in_modes, const int *in_mult, int in_max, int batch, int formula,
-                 int mode, tb::cd *out, hipStream_t s, int n_in = 0) {
+                 int mode, tb::cd *out, hipStream_t s, int n_in = 0, const int *done = nullptr) {
   const bool outer = n_in > 0;
   // slot capacities: an all-pairs item may enumerate either side
   const int ecap = outer ? std::max(in_max, out_max) : in_max;
@@ -395,14 +438,20 @@ int32_t run_guan(const tb::cd *U, int ldu, const int *out_modes, const int *out_
   const bool pack8 = outer && pack && ecap <= 8 && lds8 <= 32 * 1024;
 #define TB_GUAN_LAUNCH(JB, IPW, LDS)                                                          \
   do {                                                                                        \
-    if (outer)                                                                                \
-      hipLaunchKernelGGL((tb::guan_kernel<JB, IPW, true>), dim3((batch + IPW - 1) / IPW),     \
-                         dim3(64), LDS, s, U, ldu, out_modes, out_mult, out_max, in_modes,    \
-                         in_mult, in_max, batch, n_in, formula, 0, out);                      \
+    const int blocks = (batch + IPW - 1) / IPW;                                               \
+    if (outer && done)                                                                        \
+      hipLaunchKernelGGL((tb::guan_outer_kernel<JB, IPW, true>),                              \
+                         dim3(std::min(blocks, kGuanAfterRecurrenceBlocks)), dim3(64), LDS, s, \
+                         U, ldu, out_modes, out_mult, out_max, in_modes, in_mult, in_max,     \
+                         batch, n_in, formula, done, out);                                    \
+    else if (outer)                                                                           \
+      hipLaunchKernelGGL((tb::guan_outer_kernel<JB, IPW, false>), dim3(blocks), dim3(64),     \
+                         LDS, s, U, ldu, out_modes, out_mult, out_max, in_modes, in_mult,     \
+                         in_max, batch, n_in, formula, nullptr, out);                         \
     else                                                                                      \
-      hipLaunchKernelGGL((tb::guan_kernel<JB, IPW, false>), dim3((batch + IPW - 1) / IPW),    \
-                         dim3(64), LDS, s, U, ldu, out_modes, out_mult, out_max, in_modes,    \
-                         in_mult, in_max, batch, 0, formula, mode, out);                      \
+      hipLaunchKernelGGL((tb::guan_kernel<JB, IPW>), dim3(blocks), dim3(64), LDS, s, U, ldu,  \
+                         out_modes, out_mult, out_max, in_modes, in_mult, in_max, batch,      \
+                         formula, mode, out);                                                 \
   } while (0)
   if (pack8) {
     if (pcap <= 8)
@@ -449,11 +498,34 @@ extern "C" int32_t tb_guan_perm_batch(const tb_complex128 *U, int32_t ldu,
                        in_max, batch, formula, 0, (tb::cd *)out, (hipStream_t)stream);
 }
 
+namespace tbsub {
+bool attempt(int ldu, int out_max, int n_out, int in_max, int n_in);
+size_t workspace(int n_out);
+int32_t run(const tb::cd *U, int ldu, const int *out_modes, const int *out_mult, int out_max,
+            int n_out, const int *in_modes, const int *in_mult, int in_max, int n_in, int *done,
+            tb::cd *out, hipStream_t s);
+}  // namespace tbsub
+
+extern "C" size_t tb_guan_outer_workspace_size(int32_t ldu, int32_t out_max, int32_t n_out,
+                                               int32_t in_max, int32_t n_in) {
+  return tbsub::attempt(ldu, out_max, n_out, in_max, n_in) ? tbsub::workspace(n_out) : 0;
+}
+
 extern "C" int32_t tb_guan_perm_outer(const tb_complex128 *U, int32_t ldu,
                                       const int32_t *out_modes, const int32_t *out_mult,
                                       int32_t out_max, int32_t n_out, const int32_t *in_modes,
                                       const int32_t *in_mult, int32_t in_max, int32_t n_in,
                                       int32_t formula, tb_complex128 *out, void *stream) {
+  return tb_guan_perm_outer_ws(U, ldu, out_modes, out_mult, out_max, n_out, in_modes, in_mult,
+                               in_max, n_in, formula, out, nullptr, 0, stream);
+}
+
+extern "C" int32_t tb_guan_perm_outer_ws(const tb_complex128 *U, int32_t ldu,
+                                         const int32_t *out_modes, const int32_t *out_mult,
+                                         int32_t out_max, int32_t n_out, const int32_t *in_modes,
+                                         const int32_t *in_mult, int32_t in_max, int32_t n_in,
+                                         int32_t formula, tb_complex128 *out, void *workspace,
+                                         size_t workspace_bytes, void *stream) {
   if (n_out < 0 || n_in < 0) return tbh::fail(TB_EINVAL, "guan_outer: n_out=%d n_in=%d < 0", n_out, n_in);
   if (n_out == 0 || n_in == 0) return TB_OK;
   if ((int64_t)n_out * n_in > INT32_MAX)
@@ -471,6 +543,19 @@ extern "C" int32_t tb_guan_perm_outer(const tb_complex128 *U, int32_t ldu,
     return tbh::fail(TB_ERANGE, "guan_outer: out_max=%d, in_max=%d: either side may be "
                      "enumerated, so both must be <= %d", out_max, in_max,
                      std::min(TB_GUAN_MAX_ROWS, TB_GUAN_MAX_COLS));
+  int *done = nullptr;
+  if (workspace != nullptr && tbsub::attempt(ldu, out_max, n_out, in_max, n_in)) {
+    const size_t need = tbsub::workspace(n_out);
+    if (workspace_bytes < need)
+      return tbh::fail(TB_EWORKSPACE, "guan_outer: workspace %zu bytes < required %zu",
+                       workspace_bytes, need);
+    done = (int *)workspace;
+    const int32_t rc = tbsub::run((const tb::cd *)U, ldu, out_modes, out_mult, out_max, n_out,
+                                  in_modes, in_mult, in_max, n_in, done, (tb::cd *)out,
+                                  (hipStream_t)stream);
+    if (rc) return rc;
+  }
   return tbg::run_guan((const tb::cd *)U, ldu, out_modes, out_mult, out_max, in_modes, in_mult,
-                       in_max, n_out * n_in, formula, 0, (tb::cd *)out, (hipStream_t)stream, n_in);
+                       in_max, n_out * n_in, formula, 0, (tb::cd *)out, (hipStream_t)stream, n_in,
+                       done);
 }

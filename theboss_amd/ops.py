@@ -59,19 +59,34 @@ def guan_perm_batch(U, out_modes, out_mult, in_modes, in_mult, formula: int = L.
     return out
 
 
-def guan_perm_outer(U, out_modes, out_mult, in_modes, in_mult, formula: int = L.TB_FORMULA_RYSER):
-    """All pairs of output rows j and input rows i in one launch: an (n_out, n_in) tensor
-    holding perm(U[t_j, s_i]); each pair enumerates the row with fewer Guan codes."""
+# Pairs x 2^in_max from which on guan_perm_outer tries the subset recurrence without being
+# told that the input rows allow it (trying in vain adds about 7 us to the walk's 50).
+_OUTER_TRY_CODES = 1 << 22
+
+
+def guan_perm_outer(U, out_modes, out_mult, in_modes, in_mult, formula: int = L.TB_FORMULA_RYSER,
+                    common: Optional[bool] = None):
+    """All pairs of output rows j and input rows i in one call: an (n_out, n_in) tensor
+    holding perm(U[t_j, s_i]), by the subset recurrence over the input rows' common state where
+    that is small enough, else pair by pair over the row with fewer Guan codes. `common` says
+    whether the input rows are known to have such a state (states.has_small_common_state);
+    None leaves it to the device, for calls large enough."""
     T = D.require_gpu()
     U = _c128(U, "U")
     out_modes, out_mult = _i32(out_modes, "out_modes"), _i32(out_mult, "out_mult")
     in_modes, in_mult = _i32(in_modes, "in_modes"), _i32(in_mult, "in_mult")
     n_out, n_in = out_modes.shape[0], in_modes.shape[0]
     out = T.empty((n_out, n_in), dtype=T.complex128, device=U.device)
-    L.check(L.load().tb_guan_perm_outer(
-        D.ptr(U), U.shape[1], D.ptr(out_modes), D.ptr(out_mult), out_modes.shape[1], n_out,
-        D.ptr(in_modes), D.ptr(in_mult), in_modes.shape[1], n_in, formula, D.ptr(out),
-        D.stream_ptr(U.device)))
+    lib = L.load()
+    ldu, out_max, in_max = U.shape[1], out_modes.shape[1], in_modes.shape[1]
+    need = 0
+    if common or (common is None and (n_out * n_in) << min(in_max, 32) >= _OUTER_TRY_CODES):
+        need = lib.tb_guan_outer_workspace_size(ldu, out_max, n_out, in_max, n_in)
+    ws = D.workspace(need, U.device) if need else None
+    L.check(lib.tb_guan_perm_outer_ws(
+        D.ptr(U), ldu, D.ptr(out_modes), D.ptr(out_mult), out_max, n_out,
+        D.ptr(in_modes), D.ptr(in_mult), in_max, n_in, formula, D.ptr(out),
+        D.ptr(ws) if ws is not None else None, need, D.stream_ptr(U.device)))
     return out
 
 

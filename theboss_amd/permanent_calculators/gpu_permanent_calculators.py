@@ -21,7 +21,8 @@ from numpy import complex128
 from .. import _device as D
 from .. import _lib as L
 from .. import ops
-from ..states import as_occupation, compact_batch, effective_matrix, layer_rows
+from ..states import (as_occupation, compact_batch, effective_matrix, has_small_common_state,
+                      layer_rows)
 from .bs_permanent_calculator_interface import BSPermanentCalculatorInterface
 
 
@@ -208,8 +209,9 @@ class _GuanGPUCalculator(BSPermanentCalculatorBase):
         """All pairs at once: a (len(Tm), len(S)) complex128 device tensor holding
         perm(U[Tm[j], S[i]]) at [j, i], for S and Tm rows that all hold the same number
         k >= 1 of particles. The S side is compacted once (cached by content), the Tm side
-        on the device, and one tb_guan_perm_outer launch walks every pair, each over the
-        side with fewer Guan codes (as compute_permanent_batch_arrays chooses). None when
+        on the device, and one tb_guan_perm_outer_ws call computes every pair, by the subset
+        recurrence where the S rows have a small common state, else each over the side with
+        fewer Guan codes (as compute_permanent_batch_arrays chooses). None when
         a side needs the Glynn fallback."""
         S = np.asarray(S, dtype=np.int64)
         Tm = np.asarray(Tm, dtype=np.int64)
@@ -218,9 +220,9 @@ class _GuanGPUCalculator(BSPermanentCalculatorBase):
             raise AttributeError("outer batch needs rows with one common particle number >= 1")
         T = D.require_gpu()
         dev = D.device()
-        codes_s, cs = _cached(_content_key("S", dev, S), lambda: (
+        codes_s, cs, common = _cached(_content_key("S", dev, S), lambda: (
             np.prod(S.astype(np.float64) + 1, axis=1),
-            [D.to_device_i32(a, dev) for a in compact_batch(S)]))
+            [D.to_device_i32(a, dev) for a in compact_batch(S)], has_small_common_state(S)))
         codes_t = np.prod(Tm.astype(np.float64) + 1, axis=1)
         ct = _compact_on_device(T, Tm, dev)
         if max(cs[0].shape[1], ct[0].shape[1]) > min(L.TB_GUAN_MAX_COLS, L.TB_GUAN_MAX_ROWS) \
@@ -228,15 +230,15 @@ class _GuanGPUCalculator(BSPermanentCalculatorBase):
             return None
         U = np.asarray(self._matrix, dtype=np.complex128)
         Ud = _cached(_content_key("U", dev, U), lambda: D.to_device_c128(U, dev))
-        return ops.guan_perm_outer(Ud, ct[0], ct[1], cs[0], cs[1], self.formula)
+        return ops.guan_perm_outer(Ud, ct[0], ct[1], cs[0], cs[1], self.formula, common)
 
     def compute_permanent_layer(self, S: np.ndarray, prefixes: np.ndarray):
         """A GCC-A layer's pairs: a (len(prefixes) * m, len(S)) complex128 device tensor
         holding perm(U[prefix_p + e_o, S[i]]) at [p * m + o, i], for S rows of k >= 1
         particles and prefixes of k - 1. The output rows are built in compact form from the
         compacted prefixes (each prefix's modes, then mode o: one more particle where the
-        prefix holds o, else a new slot), uploaded once, and walked by one
-        tb_guan_perm_outer launch. A row's slots are then not in mode order, which changes
+        prefix holds o, else a new slot), uploaded once, and computed by one
+        tb_guan_perm_outer_ws call. A row's slots are then not in mode order, which changes
         the walk's rounding only. None when a side needs the Glynn fallback."""
         S = np.asarray(S, dtype=np.int64)
         Pf = np.asarray(prefixes, dtype=np.int64)
@@ -246,9 +248,9 @@ class _GuanGPUCalculator(BSPermanentCalculatorBase):
             raise AttributeError("a layer needs S rows of k >= 1 particles and prefixes of k - 1")
         D.require_gpu()
         dev = D.device()
-        codes_s, cs = _cached(_content_key("S", dev, S), lambda: (
+        codes_s, cs, common = _cached(_content_key("S", dev, S), lambda: (
             np.prod(S.astype(np.float64) + 1, axis=1),
-            [D.to_device_i32(a, dev) for a in compact_batch(S)]))
+            [D.to_device_i32(a, dev) for a in compact_batch(S)], has_small_common_state(S)))
         rows = layer_rows(Pf)  # modes, multiplicities: 2 x (P m) x (W + 1)
         codes_t = np.prod(rows[1].astype(np.float64) + 1, axis=1)
         if max(cs[0].shape[1], rows.shape[2]) > min(L.TB_GUAN_MAX_COLS, L.TB_GUAN_MAX_ROWS) \
@@ -257,7 +259,7 @@ class _GuanGPUCalculator(BSPermanentCalculatorBase):
         td = D.to_device_i32(rows, dev)
         U = np.asarray(self._matrix, dtype=np.complex128)
         Ud = _cached(_content_key("U", dev, U), lambda: D.to_device_c128(U, dev))
-        return ops.guan_perm_outer(Ud, td[0], td[1], cs[0], cs[1], self.formula)
+        return ops.guan_perm_outer(Ud, td[0], td[1], cs[0], cs[1], self.formula, common)
 
     def compute_permanent(self) -> complex128:
         s, t = self._checked_states()

@@ -48,6 +48,18 @@ def compact_batch(states: np.ndarray) -> Tuple[np.ndarray, np.ndarray]:
     return modes, mult
 
 
+def has_small_common_state(states: np.ndarray) -> bool:
+    """Whether the rows (B x m occupations) are substates of one state of at most 12 modes and
+    4096 substates and hold at most 12 particles each: the inputs for which the all-pairs
+    permanents come from one recurrence over that state's substates."""
+    states = np.asarray(states)
+    if states.size == 0 or int(states.sum(axis=1).max()) > 12:
+        return False
+    top = states.max(axis=0)
+    top = top[top > 0].astype(np.int64)
+    return len(top) <= 12 and math.prod((top + 1).tolist()) <= 4096
+
+
 def layer_rows(prefixes: np.ndarray) -> np.ndarray:
     """The occupations prefix_p + e_o (o < m) of a GCC-A layer in compact form, built from
     the compacted prefixes: rows[0] modes, rows[1] multiplicities, row p * m + o of shape
