@@ -38,8 +38,8 @@ struct TreeProdT<F, LO, LO + 1> {
   static __device__ __forceinline__ cpx<F> run(const F *re, const F *im) { return {re[LO], im[LO]}; }
 };
 
-// h += row (add) or h -= row; `row` is a wave-uniform LDS row (broadcast reads) or a
-// per-lane global row (NARROW mode). The row is consumed in groups of G complex values
+// h += row (add) or h -= row; `row` is an LDS row shared by the lanes of a matrix (broadcast
+// reads). The row is consumed in groups of G complex values
 // with the reads of group g+1 issued before the adds of group g, and a scheduling
 // barrier per group, so at most 2*G loaded values are live at once.
 #ifndef TB_FLIP_GROUP

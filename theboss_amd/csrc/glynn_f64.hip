@@ -45,7 +45,8 @@ bool runs_fp32(int n, int precision) {
 size_t glynn_workspace_bytes(int n, int batch, int precision, int c_pref) {
   if (n <= 1 || batch <= 0 || n > TB_GLYNN_MAX_N) return 0;
   size_t bytes = tbgl_partial_bytes(n, batch, c_pref);
-  if (runs_fp32(n, precision)) bytes += align256((size_t)batch * n * n * sizeof(tb::cpx<float>));
+  if (n >= tbgl::kWideMinN && runs_fp32(n, precision))
+    bytes += align256((size_t)batch * n * n * sizeof(tb::cpx<float>));
   return bytes;
 }
 }  // namespace
@@ -92,6 +93,9 @@ extern "C" int32_t tb_glynn_batch(const tb_complex128 *A, int32_t n, int32_t bat
   const int wpm_cap = n >= tbgl::kWideMinN ? tbgl_partial_wpm(n, batch, c_pref) : 0;
   if (!runs_fp32(n, precision))
     return tbgl::glynn_dispatch_f64(n, (const tb::cpx<double> *)A, matrix_stride, batch, o,
+                                    partial, handled, wpm_cap, c_pref, s);
+  if (n < tbgl::kWideMinN)  // the SMALL kernel converts as it stages
+    return tbgl::glynn_dispatch_f32(n, nullptr, 0, (const tb::cd *)A, matrix_stride, batch, o,
                                     partial, handled, wpm_cap, c_pref, s);
   // FP32 column sums: convert once into the tail of the workspace.
   float *A32 = (float *)(ws + tbgl_partial_bytes(n, batch, c_pref));

@@ -39,6 +39,10 @@ namespace tb {
 #define TB_GLYNN_SROW 20
 #endif
 
+// FP64 SMALL kernels from this n on give a matrix at least 16 lanes and hold its rows in
+// broadcast form.
+constexpr int kSmallBcastMinN = 7;
+
 // Rows 0..R0-1 (the most frequently flipped: row i flips on 2^-(i+1) of all steps) are
 // held in VGPRs; the rest are read from memory at each flip.
 template <int N, int R0, typename F>
@@ -778,17 +782,145 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE))) void
   }
 }
 
-// NARROW: one lane per matrix, whole enumeration in the lane (small n), global rows.
+// One row of a matrix in LDS in broadcast form, each 16-lane row of the wave from its own M.
+template <int N>
+__device__ __forceinline__ Bcast<N> row_bcast(const cpx<double> *M, int i) {
+  const int lane = threadIdx.x & 15;
+  Bcast<N> b;
+#pragma unroll
+  for (int p = 0; p < Bcast<N>::P; ++p) {
+    const int t = 16 * p + lane;
+    b.v[p] = ((const double *)(M + i * N))[t < 2 * N ? t : 2 * N - 1];
+  }
+  return b;
+}
+// Two wait states between whatever wrote the row's registers and its DPP reads (N <= 16).
+template <int N>
+__device__ __forceinline__ void bcast_ready(Bcast<N> &b) {
+  asm volatile("s_nop 1" : "+v"(b.v[0]), "+v"(b.v[Bcast<N>::P - 1]));
+}
+
+// glynn_lane with every row in broadcast form, for matrices that own whole 16-lane rows: the
+// U static rows stay in registers, the others are loaded (2 values per lane instead of N
+// complex ones) a row ahead of the flip that adds them.
+template <int N, int U>
+__device__ __forceinline__ void glynn_bcast_lane(const cpx<double> *M, int C, uint32_t q,
+                                                 double &acc_re, double &acc_im) {
+  constexpr int NB = N - 1;
+  const uint32_t t0 = q << C, g0 = t0 ^ (t0 >> 1);
+  const bool q_odd = (q & 1u) != 0;  // the Gray bit above the chunk
+  Bcast<N> rows[U];
+#pragma unroll
+  for (int u = 0; u < U; ++u) rows[u] = row_bcast<N>(M, u);
+  const double one = vgpr_one();
+  double hr[N], hi[N];
+#pragma unroll
+  for (int j = 0; j < N; ++j) {
+    hr[j] = 0.0;
+    hi[j] = 0.0;
+  }
+  Bcast<N> next = row_bcast<N>(M, NB);
+#pragma unroll 1
+  for (int i = NB; i >= 0; --i) {  // half column sums at t0, the fixed row first
+    Bcast<N> row = next;
+    next = row_bcast<N>(M, i > 0 ? i - 1 : (U < NB ? U : 0));
+    const double d = (i < NB && ((g0 >> i) & 1u)) ? -0.5 : 0.5;
+    bcast_ready(row);
+    flip_bcast<0, N, 0>(hr, hi, row, d);
+  }
+#pragma unroll
+  for (int u = 0; u < U; ++u) bcast_ready(rows[u]);
+  const cd p0 = TreeProd<0, N>::run(hr, hi);
+  double cre = p0.re, cim = p0.im;
+  const int nblocks = 1 << (C - U);
+  auto static_steps = [&](int blk) {
+#pragma unroll
+    for (int j = 1; j < (1 << U); ++j) {
+      const int i = __builtin_ctz(j);
+      if (i + 1 < U) {
+        if ((j >> (i + 1)) & 1)
+          flip_bcast<0, N, 1>(hr, hi, rows[i], one);
+        else
+          flip_bcast<0, N, -1>(hr, hi, rows[i], one);
+      } else {
+        const bool add = (U < C) ? (blk & 1) != 0 : q_odd;
+        flip_bcast<0, N, 0>(hr, hi, rows[i], add ? 1.0 : -1.0);
+      }
+      if (j & 1)
+        tree_prod_acc<-1, 0, N>(cre, cim, hr, hi);
+      else
+        tree_prod_acc<1, 0, N>(cre, cim, hr, hi);
+      TB_STEP_FENCE();
+    }
+  };
+  static_steps(0);
+  for (int blk = 1; blk < nblocks; ++blk) {
+    const int i = U + __builtin_ctz(blk);
+    const bool add = i + 1 < C ? ((blk >> (i + 1 - U)) & 1) != 0 : q_odd;
+    Bcast<N> row = next;
+    next = row_bcast<N>(M, U + __builtin_ctz(blk + 1 < nblocks ? blk + 1 : 1));
+    bcast_ready(row);
+    flip_bcast<0, N, 0>(hr, hi, row, add ? 1.0 : -1.0);
+    tree_prod_acc<1, 0, N>(cre, cim, hr, hi);
+    TB_STEP_FENCE();
+    static_steps(blk);
+  }
+  acc_re += cre;
+  acc_im += cim;
+}
+
+// SMALL (n < kWideMinN): 2^(N-1-C) lanes per matrix, each walking one chunk of 2^C ranks, 256
+// lanes per workgroup; the matrices are staged in LDS (one complex value of padding each, so
+// that the groups of a wave read different banks) and the lanes' sums added up by shuffles,
+// beyond a wave through LDS. One launch, no partial sums in memory.
+// What bounds it: latency and, in large batches, VALU issue. Against one lane per matrix with
+// its rows in global memory (n <= 10) and 4 waves per matrix, an idle fallback launch and a
+// finishing one (n = 11..13), times from Python, where an empty call takes 9 us: one n = 10
+// matrix 76 -> 9 us, 20,000 of them 140 -> 29; one n = 12 matrix 14 -> 9, 20,000: 203 -> 112.
+// From LDS rows instead of broadcast ones, 1000 n = 13 matrices took 28 us (15; 21 before):
+// the seeds' N^2 16-byte broadcast reads per lane held the LDS return path.
 template <int N, int U, typename F>
-__global__ __launch_bounds__(256) void glynn_narrow_kernel(const cpx<F> *__restrict__ A,
-                                                           int64_t mstride, int batch,
-                                                           cd *__restrict__ out) {
-  const int b = blockIdx.x * blockDim.x + threadIdx.x;
-  if (b >= batch) return;
-  const cpx<F> *M = A + (size_t)b * mstride;
+__global__ __launch_bounds__(256) void glynn_small_kernel(const cd *__restrict__ A, int64_t mstride,
+                                                          int batch, int C, cd *__restrict__ out) {
+  constexpr int NB = N - 1, MS = N * N + 1;
+  extern __shared__ char small_lds[];
+  cpx<F> *Ms = (cpx<F> *)small_lds;
+  __shared__ double wave_re[4], wave_im[4];
+  const int tid = threadIdx.x;
+  const int wbits = NB - C, W = 1 << wbits;  // lanes per matrix, 1..256
+  const int mats = 256 >> wbits;
+  const int b0 = blockIdx.x * mats;
+  const int here = min(mats, batch - b0);
+  for (int e = tid; e < here * N * N; e += 256) {
+    const int k = e / (N * N), r = e - k * (N * N);
+    const cd v = A[(size_t)(b0 + k) * mstride + r];
+    Ms[k * MS + r] = {(F)v.re, (F)v.im};
+  }
+  __syncthreads();
+  const int g = min(tid >> wbits, here - 1);  // idle groups repeat the last matrix
+  const int q = tid & (W - 1);
   double are = 0.0, aim = 0.0;
-  glynn_lane<N, U, 0, F>(M, N - 1, 0, 0, 1, are, aim);
-  out[b] = {2.0 * are, 2.0 * aim};
+  if constexpr (sizeof(F) == 8 && N >= kSmallBcastMinN)
+    glynn_bcast_lane<N, U>((const cpx<double> *)(Ms + g * MS), C, (uint32_t)q, are, aim);
+  else
+    glynn_lane<N, U, 1, F>((const cpx<F> *)(Ms + g * MS), C, (uint64_t)q, 0, 1, are, aim);
+  for (int off = min(W, 64) >> 1; off >= 1; off >>= 1) {
+    are += __shfl_xor(are, off, 64);
+    aim += __shfl_xor(aim, off, 64);
+  }
+  if (W > 64) {  // uniform over the launch
+    if ((tid & 63) == 0) {
+      wave_re[tid >> 6] = are;
+      wave_im[tid >> 6] = aim;
+    }
+    __syncthreads();
+    if (q == 0)
+      for (int w = 1; w < W >> 6; ++w) {
+        are += wave_re[(tid >> 6) + w];
+        aim += wave_im[(tid >> 6) + w];
+      }
+  }
+  if (q == 0 && (tid >> wbits) < here) out[b0 + g] = {2.0 * are, 2.0 * aim};
 }
 
 namespace {  // internal linkage: each translation unit keeps its own copy
@@ -902,7 +1034,7 @@ inline int glynn_u_max(int n) {
   return std::max({2, n >= 25 ? TB_GLYNN_U_LARGE : 2, u32});
 }
 
-constexpr int kWideMinN = 11;  // below this a lane owns a whole matrix
+constexpr int kWideMinN = 14;  // below this the SMALL kernel
 
 // FP64 sizes that run the paired walk first (the plain WIDE kernel then takes the
 // matrices it left): from where a chunk holds the static block plus one bit up to the
@@ -1041,6 +1173,27 @@ inline GlynnPlan glynn_plan(int n, int batch, int c_pref, int u = 2, int wave_sl
   return p;
 }
 
+// SMALL plan: the longest chunk (less seeding) that still gives the launch a wave per SIMD (2
+// or 4 measured up to 10% slower, 12 and 13 columns, 1000 to 4000 matrices), at least U bits,
+// at most 256 lanes per matrix and 48 KiB of matrices per workgroup; 16 lanes or more where the
+// rows are in broadcast form.
+#ifndef TB_SMALL_WAVES
+#define TB_SMALL_WAVES 1024
+#endif
+inline size_t glynn_small_lds(int n, int C, size_t elem) {
+  return (size_t)(256 >> (n - 1 - C)) * (n * n + 1) * elem;
+}
+inline int glynn_small_plan(int n, int batch, int c_pref, int u, size_t elem) {
+  const int nb = n - 1;
+  const int lo = std::max(u, nb - 8);
+  int hi = elem == sizeof(tb::cpx<double>) && n >= tb::kSmallBcastMinN ? nb - 4 : nb;
+  while (hi > lo && glynn_small_lds(n, hi, elem) > 48 * 1024) --hi;
+  if (c_pref > 0) return std::min(std::max(c_pref, lo), hi);
+  int C = hi;
+  while (C > lo && ((int64_t)batch << (nb - C)) < TB_SMALL_WAVES * 64) --C;
+  return C;
+}
+
 // A: the matrices in the kernel's precision; A64 / mstride64: the same matrices in FP64
 // (the paired FP32 kernel forms its quotients from them).
 // wpm_cap: partials per matrix the workspace holds; a plan that needs more fails with
@@ -1051,15 +1204,16 @@ inline int32_t launch_glynn_n(const tb::cpx<F> *A, int64_t mstride, const tb::cd
                               int *handled, int wpm_cap, int c_pref, hipStream_t s) {
   if constexpr (N < kWideMinN) {
     constexpr int U = (N - 1) < 2 ? (N - 1) : 2;
-    hipLaunchKernelGGL((tb::glynn_narrow_kernel<N, U, F>), dim3((batch + 255) / 256), dim3(256), 0,
-                       s, A, mstride, batch, out);
+    const int C = glynn_small_plan(N, batch, c_pref, U, sizeof(tb::cpx<F>));
+    const int mats = 256 >> (N - 1 - C);
+    hipLaunchKernelGGL((tb::glynn_small_kernel<N, U, F>), dim3((batch + mats - 1) / mats), dim3(256),
+                       glynn_small_lds(N, C, sizeof(tb::cpx<F>)), s, A64, mstride64, batch, C, out);
+    (void)A;
+    (void)mstride;
     (void)partial;
     (void)handled;
     (void)wpm_cap;
-    (void)c_pref;
-    (void)A64;
-    (void)mstride64;
-    return tbh::check_hip(hipGetLastError(), "glynn_narrow_kernel");
+    return tbh::check_hip(hipGetLastError(), "glynn_small_kernel");
   } else {
     constexpr int U = glynn_u<N, F>();
     constexpr int CMIN = glynn_min_c<N, F>();
