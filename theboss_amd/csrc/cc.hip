@@ -1,14 +1,13 @@
-// Entry points built on the binary C&C sweep: the submatrices calculator and the
-// permanent gradient. The mixed-radix fallback lives in guan.hip.
+// Entry points of the submatrices calculator (the binary C&C sweep, gathered from U as it stages;
+// the mixed-radix fallback lives in guan.hip) and of the permanent gradient.
 #include <algorithm>
 
-#include "tb_common.hpp"
+#include "sweep_impl.hpp"
 
 namespace tbs {
 size_t sweep_partial_bytes(int k, int items, int c_override);
-int32_t run_sweep(int k, const tb::cd *Vt, int ldv, int64_t item_stride, const int *item_map,
-                  const int *item_count, int items, int c_override, tb::cd *partial,
-                  tb::cd *minors, hipStream_t s);
+int32_t run_sweep(int k, const tb::SweepSource &src, int items, int c_override, tb::cd *partial,
+                  const int *in_mult, int in_max, tb::cd *minors, hipStream_t s);
 }  // namespace tbs
 namespace tbgr {
 size_t grad_workspace(int n, int batch, int c_pref);
@@ -22,57 +21,6 @@ int32_t run_guan(const tb::cd *U, int ldu, const int *out_modes, const int *out_
 }  // namespace tbg
 
 namespace tb {
-
-// Vt[b][nu][j] = U[out row j][in particle nu]: particles are the input slots with
-// multiplicity 1 in slot order, output rows expand each slot's multiplicity.
-__global__ void cc_gather_kernel(const cd *__restrict__ U, int ldu, const int *__restrict__ out_modes,
-                                 const int *__restrict__ out_mult, int out_max,
-                                 const int *__restrict__ in_modes, const int *__restrict__ in_mult,
-                                 int in_max, int batch, int k, cd *__restrict__ Vt) {
-  const int R = k - 1;
-  const int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (idx >= (int64_t)batch * k * R) return;
-  const int b = (int)(idx / ((int64_t)k * R));
-  const int rem = (int)(idx - (int64_t)b * k * R);
-  const int nu = rem / R, j = rem - nu * R;
-  int col = -1, cnt = 0;
-  for (int d = 0; d < in_max; ++d) {
-    if (in_mult[(size_t)b * in_max + d] > 0) {
-      if (cnt == nu) {
-        col = in_modes[(size_t)b * in_max + d];
-        break;
-      }
-      ++cnt;
-    }
-  }
-  int row = -1, acc = 0;
-  for (int q = 0; q < out_max; ++q) {
-    acc += out_mult[(size_t)b * out_max + q];
-    if (j < acc) {
-      row = out_modes[(size_t)b * out_max + q];
-      break;
-    }
-  }
-  cd v = {0.0, 0.0};
-  if (row >= 0 && col >= 0) v = U[(size_t)row * ldu + col];
-  Vt[idx] = v;
-}
-
-// minors[b][slot] = compact[b][nu(slot)] for occupied slots, 0 elsewhere.
-__global__ void cc_scatter_kernel(const cd *__restrict__ compact, const int *__restrict__ in_mult,
-                                  int in_max, int batch, int k, cd *__restrict__ minors) {
-  const int idx = blockIdx.x * blockDim.x + threadIdx.x;
-  if (idx >= batch * in_max) return;
-  const int b = idx / in_max, d = idx - b * in_max;
-  cd v = {0.0, 0.0};
-  if (in_mult[idx] > 0) {
-    int nu = 0;
-    for (int e = 0; e < d; ++e)
-      if (in_mult[(size_t)b * in_max + e] > 0) ++nu;
-    if (nu < k) v = compact[(size_t)b * k + nu];
-  }
-  minors[idx] = v;
-}
 
 // k == 1: bs_submatrices_permanent_calculator_base.py:156-158 returns s itself.
 __global__ void cc_single_kernel(const int *__restrict__ in_mult, int n, cd *__restrict__ minors) {
@@ -94,22 +42,11 @@ __global__ void grad_small_kernel(const cd *__restrict__ A, int n, int batch, in
 
 }  // namespace tb
 
-namespace {
-inline size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
-
-size_t cc_workspace_bytes(int k, int batch, int c) {
-  if (k < 2 || batch <= 0 || k > TB_SWEEP_MAX_K) return 0;
-  const size_t vt = align256((size_t)batch * k * (k - 1) * sizeof(tb::cd));
-  const size_t compact = align256((size_t)batch * k * sizeof(tb::cd));
-  return vt + compact + tbs::sweep_partial_bytes(k, batch, c);
-}
-}  // namespace
-
 extern "C" size_t tb_cc_workspace_size(int32_t k, int32_t out_max, int32_t in_max, int32_t batch) {
   (void)out_max;
   (void)in_max;
   if (k < 2 || k > TB_SWEEP_MAX_K) return 0;
-  return cc_workspace_bytes(k, batch, tbh::tuned(TB_TUNE_SWEEP, k, batch));
+  return tbs::sweep_partial_bytes(k, batch, tbh::tuned(TB_TUNE_SWEEP, k, batch));
 }
 
 extern "C" int32_t tb_cc_submatrices_batch(const tb_complex128 *U, int32_t ldu,
@@ -144,29 +81,20 @@ extern "C" int32_t tb_cc_submatrices_batch(const tb_complex128 *U, int32_t ldu,
   if (k > TB_SWEEP_MAX_K)
     return tbh::fail(TB_ERANGE, "cc: k=%d exceeds TB_SWEEP_MAX_K=%d", k, TB_SWEEP_MAX_K);
   const int c = tbh::tuned(TB_TUNE_SWEEP, k, batch);  // read once: size check and launch agree
-  const size_t need = cc_workspace_bytes(k, batch, c);
+  const size_t need = tbs::sweep_partial_bytes(k, batch, c);
   if (!workspace || workspace_bytes < need)
     return tbh::fail(TB_EWORKSPACE, "cc: workspace %zu bytes < required %zu", workspace_bytes,
                      need);
-  char *ws = (char *)workspace;
-  tb::cd *Vt = (tb::cd *)ws;
-  ws += align256((size_t)batch * k * (k - 1) * sizeof(tb::cd));
-  tb::cd *compact = (tb::cd *)ws;
-  ws += align256((size_t)batch * k * sizeof(tb::cd));
-  tb::cd *partial = (tb::cd *)ws;
-  const int64_t total = (int64_t)batch * k * (k - 1);
-  hipLaunchKernelGGL(tb::cc_gather_kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, s,
-                     (const tb::cd *)U, ldu, out_modes, out_mult, out_max, in_modes, in_mult,
-                     in_max, batch, k, Vt);
-  int32_t rc = tbh::check_hip(hipGetLastError(), "cc_gather_kernel");
-  if (rc) return rc;
-  rc = tbs::run_sweep(k, Vt, k - 1, (int64_t)k * (k - 1), nullptr, nullptr, batch, c, partial,
-                      compact, s);
-  if (rc) return rc;
-  const int n = batch * in_max;
-  hipLaunchKernelGGL(tb::cc_scatter_kernel, dim3((n + 255) / 256), dim3(256), 0, s, compact,
-                     in_mult, in_max, batch, k, mo);
-  return tbh::check_hip(hipGetLastError(), "cc_scatter_kernel");
+  tb::SweepSource src{};
+  src.U = (const tb::cd *)U;
+  src.ldu = ldu;
+  src.out_modes = out_modes;
+  src.out_mult = out_mult;
+  src.out_max = out_max;
+  src.in_modes = in_modes;
+  src.in_mult = in_mult;
+  src.in_max = in_max;
+  return tbs::run_sweep(k, src, batch, c, (tb::cd *)workspace, in_mult, in_max, mo, s);
 }
 
 extern "C" size_t tb_perm_grad_workspace_size(int32_t n, int32_t batch) {

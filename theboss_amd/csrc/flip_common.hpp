@@ -264,6 +264,80 @@ __device__ __forceinline__ void prod_half_scaled(const cd *v, int J, cd &mant, i
   e2 = ke;
 }
 
+// ------------------------------------------------------------------------------------
+// Sums of several values over 2^LB lanes (LB = 4: each row of 16 lanes; 5: the rows 0, 1 and
+// 2, 3; 6: the wave), transposed: every stage halves the number of values a lane carries, so
+// CNT sums cost about CNT additions and swaps in all instead of CNT LB shuffles, and use no
+// LDS (permlane swaps for lane distances 32 and 16, DPP inside a row).
+// ------------------------------------------------------------------------------------
+__device__ __forceinline__ double select_f64(bool c, double a, double b) { return c ? a : b; }
+
+template <int CTRL>
+__device__ __forceinline__ double dpp_perm(double v) {
+  const uint64_t u = __builtin_bit_cast(uint64_t, v);
+  const uint32_t lo = (uint32_t)__builtin_amdgcn_mov_dpp((int)(uint32_t)u, CTRL, 0xf, 0xf, true);
+  const uint32_t hi = (uint32_t)__builtin_amdgcn_mov_dpp((int)(uint32_t)(u >> 32), CTRL, 0xf, 0xf, true);
+  return join64(lo, hi);
+}
+
+// (a, b) -> lanes < 32: a + a[lane ^ 32]; lanes >= 32: b + b[lane ^ 32].
+__device__ __forceinline__ double swap32_pair_sum(double a, double b) {
+  const uint64_t ua = __builtin_bit_cast(uint64_t, a), ub = __builtin_bit_cast(uint64_t, b);
+  const auto lo = __builtin_amdgcn_permlane32_swap((uint32_t)ua, (uint32_t)ub, false, false);
+  const auto hi =
+      __builtin_amdgcn_permlane32_swap((uint32_t)(ua >> 32), (uint32_t)(ub >> 32), false, false);
+  return join64(lo[0], hi[0]) + join64(lo[1], hi[1]);
+}
+// (a, b) -> rows 0, 2: a + a[lane ^ 16]; rows 1, 3: b + b[lane ^ 16].
+__device__ __forceinline__ double swap16_pair_sum(double a, double b) {
+  const uint64_t ua = __builtin_bit_cast(uint64_t, a), ub = __builtin_bit_cast(uint64_t, b);
+  const auto lo = __builtin_amdgcn_permlane16_swap((uint32_t)ua, (uint32_t)ub, false, false);
+  const auto hi =
+      __builtin_amdgcn_permlane16_swap((uint32_t)(ua >> 32), (uint32_t)(ub >> 32), false, false);
+  return join64(lo[0], hi[0]) + join64(lo[1], hi[1]);
+}
+// (a, b) -> lanes with `odd` clear: a + a[partner], set: b + b[partner].
+template <int CTRL>
+__device__ __forceinline__ double dpp_pair_sum(double a, double b, bool odd) {
+  const double keep = select_f64(odd, b, a), send = select_f64(odd, a, b);
+  return keep + dpp_perm<CTRL>(send);
+}
+// Halves `x` (CNT values) by one stage.
+template <int CTRL, int CNT>
+__device__ __forceinline__ void dpp_stage(double *x, bool odd) {
+#pragma unroll
+  for (int k = 0; k < CNT / 2; ++k) x[k] = dpp_pair_sum<CTRL>(x[2 * k], x[2 * k + 1], odd);
+  if (CNT & 1) x[CNT / 2] = x[CNT - 1] + dpp_perm<CTRL>(x[CNT - 1]);
+}
+
+// Ends with ceil(CNT / 2^LB) values in x: value v of a lane is the total of input
+// lane_sums_index(lane) + v 2^LB (meaningless where that is CNT or more).
+template <int LB, int CNT>
+__device__ __forceinline__ void lane_sums(double *x, int lane) {
+  constexpr int H32 = LB == 6 ? (CNT + 1) / 2 : CNT, H16 = LB >= 5 ? (H32 + 1) / 2 : H32;
+  if constexpr (LB == 6) {
+#pragma unroll
+    for (int k = 0; k < CNT / 2; ++k) x[k] = swap32_pair_sum(x[2 * k], x[2 * k + 1]);
+    if (CNT & 1) x[CNT / 2] = swap32_pair_sum(x[CNT - 1], x[CNT - 1]);
+  }
+  if constexpr (LB >= 5) {
+#pragma unroll
+    for (int k = 0; k < H32 / 2; ++k) x[k] = swap16_pair_sum(x[2 * k], x[2 * k + 1]);
+    if (H32 & 1) x[H32 / 2] = swap16_pair_sum(x[H32 - 1], x[H32 - 1]);
+  }
+  constexpr int H8 = (H16 + 1) / 2, H4 = (H8 + 1) / 2, H2 = (H4 + 1) / 2;
+  dpp_stage<0x128, H16>(x, (lane & 8) != 0);  // row_ror:8
+  dpp_stage<0x141, H8>(x, (lane & 4) != 0);   // row_half_mirror
+  dpp_stage<0x4E, H4>(x, (lane & 2) != 0);    // quad_perm [2,3,0,1]
+  dpp_stage<0xB1, H2>(x, (lane & 1) != 0);    // quad_perm [1,0,3,2]
+}
+template <int LB>
+__device__ __forceinline__ int lane_sums_index(int lane) {
+  const int a = ((lane & 1) << 3) | ((lane & 2) << 1) | ((lane & 4) >> 1) | ((lane & 8) >> 3);
+  const int b = 2 * a + ((lane >> 4) & 1);
+  return LB == 4 ? a : LB == 5 ? b : 2 * b + ((lane >> 5) & 1);
+}
+
 // 1.0 in a VGPR the compiler cannot fold away (second operand of fixed-direction flips).
 __device__ __forceinline__ double vgpr_one() {
   double one = 1.0;

@@ -72,16 +72,6 @@ constexpr int grad_wbits(int n) {
   return w;
 }
 
-__device__ __forceinline__ double select_f64(bool c, double a, double b) { return c ? a : b; }
-
-template <int CTRL>
-__device__ __forceinline__ double dpp_perm(double v) {
-  const uint64_t u = __builtin_bit_cast(uint64_t, v);
-  const uint32_t lo = (uint32_t)__builtin_amdgcn_mov_dpp((int)(uint32_t)u, CTRL, 0xf, 0xf, true);
-  const uint32_t hi = (uint32_t)__builtin_amdgcn_mov_dpp((int)(uint32_t)(u >> 32), CTRL, 0xf, 0xf, true);
-  return join64(lo, hi);
-}
-
 // v of lane ^ 16 and of lane ^ 32, over the LDS crossbar: no VALU issue slots, which the
 // FP64 work needs (permlane swaps and their selects: 24 32-bit instructions per code).
 __device__ __forceinline__ double xor16_lane(double v) {
@@ -95,53 +85,6 @@ __device__ __forceinline__ double xor32_lane(double v, int addr) {
   const int lo = __builtin_amdgcn_ds_bpermute(addr, (int)(uint32_t)u);
   const int hi = __builtin_amdgcn_ds_bpermute(addr, (int)(uint32_t)(u >> 32));
   return join64((uint32_t)lo, (uint32_t)hi);
-}
-
-// (a, b) -> rows 0, 2: a + a[lane ^ 16]; rows 1, 3: b + b[lane ^ 16].
-__device__ __forceinline__ double swap16_pair_sum(double a, double b) {
-  const uint64_t ua = __builtin_bit_cast(uint64_t, a), ub = __builtin_bit_cast(uint64_t, b);
-  const auto lo = __builtin_amdgcn_permlane16_swap((uint32_t)ua, (uint32_t)ub, false, false);
-  const auto hi =
-      __builtin_amdgcn_permlane16_swap((uint32_t)(ua >> 32), (uint32_t)(ub >> 32), false, false);
-  return join64(lo[0], hi[0]) + join64(lo[1], hi[1]);
-}
-
-// (a, b) -> lanes with `odd` clear: a + a[partner], set: b + b[partner].
-template <int CTRL>
-__device__ __forceinline__ double dpp_pair_sum(double a, double b, bool odd) {
-  const double keep = select_f64(odd, b, a), send = select_f64(odd, a, b);
-  return keep + dpp_perm<CTRL>(send);
-}
-
-// Halves `x` (CNT values) by one transposed stage.
-template <int CTRL, int CNT>
-__device__ __forceinline__ void dpp_stage(double *x, bool odd) {
-#pragma unroll
-  for (int k = 0; k < CNT / 2; ++k) x[k] = dpp_pair_sum<CTRL>(x[2 * k], x[2 * k + 1], odd);
-  if (CNT & 1) x[CNT / 2] = x[CNT - 1] + dpp_perm<CTRL>(x[CNT - 1]);
-}
-
-// Sums of x[0..CNT) over the code lanes (the 64 / L lanes that share a column block):
-// ends with V = grad_sum_regs values in x; value v of a lane is the total of input
-// grad_sum_index(lane) + v * 2^lb.
-template <int L, int CNT>
-__device__ __forceinline__ void code_lane_sums(double *x, int lane) {
-  constexpr int H0 = (L == 4) ? CNT : (CNT + 1) / 2;
-  if constexpr (L == 2) {
-#pragma unroll
-    for (int k = 0; k < CNT / 2; ++k) x[k] = swap16_pair_sum(x[2 * k], x[2 * k + 1]);
-    if (CNT & 1) x[CNT / 2] = swap16_pair_sum(x[CNT - 1], x[CNT - 1]);
-  }
-  constexpr int H1 = (H0 + 1) / 2, H2 = (H1 + 1) / 2, H3 = (H2 + 1) / 2;
-  dpp_stage<0x128, H0>(x, (lane & 8) != 0);  // row_ror:8
-  dpp_stage<0x141, H1>(x, (lane & 4) != 0);  // row_half_mirror
-  dpp_stage<0x4E, H2>(x, (lane & 2) != 0);   // quad_perm [2,3,0,1]
-  dpp_stage<0xB1, H3>(x, (lane & 1) != 0);   // quad_perm [1,0,3,2]
-}
-template <int L>
-__device__ __forceinline__ int grad_sum_index(int lane) {
-  const int b = ((lane & 1) << 3) | ((lane & 2) << 1) | ((lane & 4) >> 1) | ((lane & 8) >> 3);
-  return L == 4 ? b : 2 * b + ((lane >> 4) & 1);
 }
 
 // Product tree over columns LO..HI-1 of a lane; inner products are kept in P by the
@@ -251,11 +194,11 @@ __attribute__((amdgpu_waves_per_eu(2))) void grad_kernel(
   const int far = (lane ^ 32) << 2;         // ds_bpermute address of lane ^ 32
   const int blk_col = (lane >> LB) * C;     // first column of the lane's block
   const cd *M = Ms + blk_col;
-  const int sum_ix = grad_sum_index<L>(lane);
+  const int sum_ix = lane_sums_index<LB>(lane);
   double *acc_l = (double *)(acc + blk_col) + sum_ix;  // + row * 2 NP
   // x (2C values per lane) summed over the code lanes and added to row i of the wave's sums.
   auto row_add = [&](double (&x)[2 * C], int i, double coef) {
-    code_lane_sums<L, 2 * C>(x, lane);
+    lane_sums<LB, 2 * C>(x, lane);
 #pragma unroll
     for (int v = 0; v << LB < 2 * C; ++v)
       if (sum_ix + (v << LB) < 2 * C) {
@@ -409,7 +352,7 @@ __attribute__((amdgpu_waves_per_eu(2))) void grad_kernel(
         x[2 * k] = Tr[k];
         x[2 * k + 1] = Ti[k];
       }
-      code_lane_sums<L, 2 * C>(x, lane);
+      lane_sums<LB, 2 * C>(x, lane);
       const uint64_t gw = gend;  // rows outside the lane range: the same in every lane
       for (int i = U; i < N; ++i) {
         if (i >= lo_lane && i < hi_lane) continue;

@@ -408,6 +408,7 @@ __global__ __launch_bounds__(64) void gccb_step_kernel(
 #define TB_GCCB_SMALL_K 12
 #endif
 constexpr int kSmallK = TB_GCCB_SMALL_K;
+static_assert(2 * kSmallK <= 64, "a lane of the small kernel holds one minor component");
 struct SmallPlan {
   int c[kSmallK + 1], wpi[kSmallK + 1], iters[kSmallK + 1];
 };
@@ -433,13 +434,11 @@ __device__ __forceinline__ void gccb_small_sweep(const cd *Vl, cd *Vs, cd *Ed, c
     Vs[e] = Vl[nu * kSmallK + j];
   }
   __syncthreads();
-  double re = 0.0, im = 0.0;
-  for (int w = 0; w < pl.wpi[K]; ++w) {
-    const cd acc = sweep_wave<K, U, R0>(Vs, Ed, lane, pl.c[K], w, pl.wpi[K], pl.iters[K]);
-    re += acc.re;
-    im += acc.im;
-  }
-  if (lane < K) mi[lane] = {re, im};
+  double sum = 0.0;  // 2K <= 64: one value per lane
+  for (int w = 0; w < pl.wpi[K]; ++w)
+    sum += sweep_wave<K, U, R0>(Vs, Ed, lane, pl.c[K], w, pl.wpi[K], pl.iters[K]).v[0];
+  const int e = lane_sums_index<6>(lane);
+  if (e < 2 * K) ((double *)mi)[e] = sum;
   __syncthreads();
 }
 

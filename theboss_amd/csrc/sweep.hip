@@ -4,6 +4,54 @@
 
 namespace tb {
 
+// Stages item `item` as Vs[nu][j] = V[nu][j]: copied from gathered columns, or gathered from U
+// by the item's slots (particles: the occupied input slots in order; rows: the output slots,
+// repeated by multiplicity; entries past either list are 0). lists: 2K - 1 ints of LDS.
+template <int K>
+__device__ __forceinline__ void sweep_stage(const SweepSource &src, int item, cd *Vs, int *lists,
+                                            int lane) {
+  constexpr int R = K - 1;
+  if (src.U == nullptr) {
+    const cd *v = src.Vt + (size_t)item * src.item_stride;
+    for (int e = lane; e < K * R; e += 64) {
+      const int nu = e / R, j = e - nu * R;
+      Vs[e] = v[(size_t)nu * src.ldv + j];
+    }
+    return;
+  }
+  int *cols = lists, *rows = lists + K;
+  for (int e = lane; e < K + R; e += 64) lists[e] = -1;
+  __syncthreads();
+  int base = 0;
+  for (int q0 = 0; q0 < src.in_max; q0 += 64) {
+    const size_t q = (size_t)item * src.in_max + q0 + lane;
+    const bool on = q0 + lane < src.in_max && src.in_mult[q] > 0;
+    const uint64_t bal = __ballot(on);
+    const int at = base + __popcll(bal & ((1ull << lane) - 1ull));
+    if (on && at < K) cols[at] = src.in_modes[q];
+    base += __popcll(bal);
+  }
+  base = 0;
+  for (int q0 = 0; q0 < src.out_max; q0 += 64) {
+    const size_t q = (size_t)item * src.out_max + q0 + lane;
+    const int m = q0 + lane < src.out_max ? min(max(src.out_mult[q], 0), R) : 0;
+    int incl = m;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+      const int v = __shfl_up(incl, off, 64);
+      if (lane >= off) incl += v;
+    }
+    for (int e = base + incl - m; e < min(base + incl, R); ++e) rows[e] = src.out_modes[q];
+    base = min(base + __shfl(incl, 63, 64), R);
+  }
+  __syncthreads();
+  for (int e = lane; e < K * R; e += 64) {
+    const int nu = e / R, j = e - nu * R;
+    const int row = rows[j], col = cols[nu];
+    Vs[e] = row >= 0 && col >= 0 ? src.U[(size_t)row * src.ldu + col] : cd{0.0, 0.0};
+  }
+}
+
 // Persistent grid: G one-wave blocks loop over the tasks (slot, w), slot < active
 // items, w < wpi. Blocks are dispatched round-robin over the 8 XCDs (each with its own
 // L2); XCD x takes the contiguous task range [x T/8, (x+1) T/8) so that the waves of one
@@ -12,13 +60,13 @@ namespace tb {
 // any number of active items and idle tasks cost nothing.
 template <int K, int U, int R0>
 __global__ __launch_bounds__(64) TB_SWEEP_ATTR(K) void sweep_kernel(
-    const cd *__restrict__ Vt, int ldv, int64_t item_stride, const int *__restrict__ item_map,
-    const int *__restrict__ item_count, int items, int c, int wpi, int iters,
-    cd *__restrict__ partial) {
+    SweepSource src, const int *__restrict__ item_map, const int *__restrict__ item_count,
+    int items, int c, int wpi, int iters, cd *__restrict__ partial) {
   constexpr int R = K - 1;
   extern __shared__ cd smem[];
   cd *Vs = smem;          // K*R
   cd *Ed = smem + K * R;  // (c - U) * 64 corrector slots
+  int *lists = (int *)(Ed + (size_t)(c > U ? c - U : 0) * 64);  // 2K - 1
   const int lane = threadIdx.x;
   int nitems = items;
   if (item_count) nitems = min(items, *item_count);
@@ -33,39 +81,77 @@ __global__ __launch_bounds__(64) TB_SWEEP_ATTR(K) void sweep_kernel(
   for (int64_t task = lo + bi; task < hi; task += nblk_x) {
     const int slot = (int)(task / wpi);
     const int w = (int)(task - (int64_t)slot * wpi);
-    const int item = item_map ? item_map[slot] : slot;
-    const cd *src = Vt + (size_t)item * item_stride;
     __syncthreads();  // previous task's reads of Vs are done
-    for (int e = lane; e < K * R; e += 64) {
-      const int nu = e / R, j = e - nu * R;
-      Vs[e] = src[(size_t)nu * ldv + j];
-    }
+    sweep_stage<K>(src, item_map ? item_map[slot] : slot, Vs, lists, lane);
     __syncthreads();
-    const cd acc = sweep_wave<K, U, R0>(Vs, Ed, lane, c, w, wpi, iters);
-    if (lane < K) partial[((size_t)slot * wpi + w) * K + lane] = acc;
+    const SweepSums<K> acc = sweep_wave<K, U, R0>(Vs, Ed, lane, c, w, wpi, iters);
+    double *dst = (double *)(partial + ((size_t)slot * wpi + w) * K);
+#pragma unroll
+    for (int v = 0; v < SweepSums<K>::V; ++v) {
+      const int e = lane_sums_index<6>(lane) + 64 * v;
+      if (e < 2 * K) dst[e] = acc.v[v];
+    }
   }
+}
+
+__device__ __forceinline__ double wave_allmax(double v) {
+  const uint64_t u = __builtin_bit_cast(uint64_t, v);
+  const auto l32 = __builtin_amdgcn_permlane32_swap((uint32_t)u, (uint32_t)u, false, false);
+  const auto h32 = __builtin_amdgcn_permlane32_swap((uint32_t)(u >> 32), (uint32_t)(u >> 32), false, false);
+  v = fmax(join64(l32[0], h32[0]), join64(l32[1], h32[1]));
+  const uint64_t t = __builtin_bit_cast(uint64_t, v);
+  const auto l16 = __builtin_amdgcn_permlane16_swap((uint32_t)t, (uint32_t)t, false, false);
+  const auto h16 = __builtin_amdgcn_permlane16_swap((uint32_t)(t >> 32), (uint32_t)(t >> 32), false, false);
+  v = fmax(join64(l16[0], h16[0]), join64(l16[1], h16[1]));
+  v = fmax(v, dpp_perm<0x128>(v));
+  v = fmax(v, dpp_perm<0x124>(v));
+  v = fmax(v, dpp_perm<0x122>(v));
+  return fmax(v, dpp_perm<0x121>(v));
+}
+
+// Both halves' value of a lane pair at distance 32: {low lane's, high lane's}, in both.
+__device__ __forceinline__ void both32(double v, double &lo, double &hi) {
+  const uint64_t u = __builtin_bit_cast(uint64_t, v);
+  const auto a = __builtin_amdgcn_permlane32_swap((uint32_t)u, (uint32_t)u, false, false);
+  const auto b = __builtin_amdgcn_permlane32_swap((uint32_t)(u >> 32), (uint32_t)(u >> 32), false, false);
+  lo = join64(a[0], b[0]);
+  hi = join64(a[1], b[1]);
+}
+
+// Product of one complex value per lane over the wave (wave-uniform).
+__device__ __forceinline__ cd wave_prod(cd v) {
+  cd a, b;
+  both32(v.re, a.re, b.re);
+  both32(v.im, a.im, b.im);
+  v = cmul(a, b);
+  v = cmul(v, {__shfl_xor(v.re, 16, 64), __shfl_xor(v.im, 16, 64)});
+  v = cmul(v, {dpp_perm<0x128>(v.re), dpp_perm<0x128>(v.im)});
+  v = cmul(v, {dpp_perm<0x124>(v.re), dpp_perm<0x124>(v.im)});
+  v = cmul(v, {dpp_perm<0x122>(v.re), dpp_perm<0x122>(v.im)});
+  v = cmul(v, {dpp_perm<0x121>(v.re), dpp_perm<0x121>(v.im)});
+  return {uniform_value(v.re), uniform_value(v.im)};
 }
 
 // Paired variant of sweep_kernel (same grid, tasks and partial layout). Per task the wave
 // stages the item, picks the particle whose smallest column entry is largest (relative to
 // the item's largest entry, at least 2^-16), swaps it into particle 1, divides the other
 // columns by it and runs the paired walk; an item without such a particle takes the plain
-// walk. The swap is undone when the minors are written. LDS: Vs | Ed | inv[R] | pmin[K] |
-// pmax[K] | Kc, exponent, pick.
+// walk. The swap is undone when the minors are written. The pick, the column product and the
+// sums of the minors are wave operations without LDS round trips (one lane multiplying the 19
+// entries one after the other, one lane scanning the particles and 6 shuffles per minor
+// component took 7 of the 34 us of one k = 20 item on 256 waves; the k = 13..16 sweeps of the
+// sampler are 2-8% faster and its fused steps 1..12 260 -> 200 us).
+// LDS: Vs | Ed | inv[R] | lists.
 template <int K, int U>
 __global__ __launch_bounds__(64) TB_SWEEP_PAIR_ATTR(K) void sweep_pair_kernel(
-    const cd *__restrict__ Vt, int ldv, int64_t item_stride, const int *__restrict__ item_map,
-    const int *__restrict__ item_count, int items, int c, int wpi, int iters,
-    cd *__restrict__ partial) {
+    SweepSource src, const int *__restrict__ item_map, const int *__restrict__ item_count,
+    int items, int c, int wpi, int iters, cd *__restrict__ partial) {
   constexpr int R = K - 1;
   extern __shared__ cd smem[];
   cd *Vs = smem;                                       // K*R
   cd *Ed = smem + K * R;                               // (c - U) * 64
   cd *inv = Ed + (size_t)(c > U ? c - U : 0) * 64;     // R
-  double *pmin = (double *)(inv + R);                  // K
-  double *pmax = pmin + K;                             // K
-  cd *kc = (cd *)(pmax + K);                           // 1 (2K doubles keep 16-byte alignment)
-  int *ke = (int *)(kc + 1);                           // exponent, pick
+  int *lists = (int *)(inv + R);                       // 2K - 1
   const int lane = threadIdx.x;
   int nitems = items;
   if (item_count) nitems = min(items, *item_count);
@@ -80,41 +166,25 @@ __global__ __launch_bounds__(64) TB_SWEEP_PAIR_ATTR(K) void sweep_pair_kernel(
   for (int64_t task = lo + bi; task < hi; task += nblk_x) {
     const int slot = (int)(task / wpi);
     const int w = (int)(task - (int64_t)slot * wpi);
-    const int item = item_map ? item_map[slot] : slot;
-    const cd *src = Vt + (size_t)item * item_stride;
     __syncthreads();  // previous task's reads of LDS are done
-    for (int e = lane; e < K * R; e += 64) {
-      const int nu = e / R, j = e - nu * R;
-      Vs[e] = src[(size_t)nu * ldv + j];
-    }
+    sweep_stage<K>(src, item_map ? item_map[slot] : slot, Vs, lists, lane);
     __syncthreads();
+    double mn = -1.0, mx = 0.0;  // squared magnitudes of particle `lane`'s entries
     if (lane < K) {
-      double mn = INFINITY, mx = 0.0;
+      mn = INFINITY;
       for (int j = 0; j < R; ++j) {
         const cd v = Vs[lane * R + j];
         const double a = fma(v.re, v.re, v.im * v.im);
         mn = fmin(mn, a);
         mx = fmax(mx, a);
       }
-      pmin[lane] = mn;
-      pmax[lane] = mx;
     }
-    __syncthreads();
-    if (lane == 0) {
-      int best = 0;
-      double mx = 0.0;
-      for (int nu = 0; nu < K; ++nu) {
-        if (pmin[nu] > pmin[best]) best = nu;
-        mx = fmax(mx, pmax[nu]);
-      }
-      const bool ok = mx > 0.0 && mx <= 1.7976931348623157e308 && pmin[best] >= kPairMinRel2 * mx;
-      ke[1] = ok ? best : -1;
-    }
-    __syncthreads();
-    const int pick = ke[1];
-    cd acc;
-    int dst = lane;  // minor slot this lane's result belongs to
-    if (pick < 0) {
+    const double top = wave_allmax(mx), best = wave_allmax(mn);
+    const bool ok = top > 0.0 && top <= 1.7976931348623157e308 && best >= kPairMinRel2 * top;
+    const int pick = __ffsll((unsigned long long)__ballot(mn == best)) - 1;  // the first such particle
+    SweepSums<K> acc;
+    double *dst = (double *)(partial + ((size_t)slot * wpi + w) * K);
+    if (!ok) {
       acc = sweep_wave<K, U, 3>(Vs, Ed, lane, c, w, wpi, iters);
     } else {
       if (pick != 1 && lane < R) {
@@ -122,50 +192,111 @@ __global__ __launch_bounds__(64) TB_SWEEP_PAIR_ATTR(K) void sweep_pair_kernel(
         Vs[R + lane] = Vs[pick * R + lane];
         Vs[pick * R + lane] = t;
       }
-      __syncthreads();
-      if (lane < R) inv[lane] = cinv_scaled(Vs[R + lane]);
-      if (lane == 63) {
-        cd m;
-        int e2;
-        prod_half_scaled(Vs + R, R, m, e2);
-        kc[0] = m;
-        ke[0] = e2;
+      // Per lane < R the reciprocal of particle 1's entry, scaled by a power of two so that
+      // its square stays in range, and the entry's mantissa of magnitude 1 to 2 sqrt 2.
+      cd m = {1.0, 0.0};
+      double e = 0.0;
+      if (lane < R) {
+        const cd v = Vs[R + lane];
+        const int ex = ilogb(fmax(fabs(v.re), fabs(v.im)));
+        m = {ldexp(v.re, -ex), ldexp(v.im, -ex)};
+        const double d = fma(m.re, m.re, m.im * m.im);
+        inv[lane] = {ldexp(m.re / d, -ex), ldexp(-m.im / d, -ex)};
+        e = (double)ex;
       }
       __syncthreads();
-      for (int e = lane; e < K * R; e += 64) {
-        const int nu = e / R, j = e - nu * R;
+      for (int q = lane; q < K * R; q += 64) {
+        const int nu = q / R, j = q - nu * R;
         if (nu != 1) {
-          const cd v = cmul(Vs[e], inv[j]);
-          Vs[e] = {2.0 * v.re, 2.0 * v.im};
+          const cd v = cmul(Vs[q], inv[j]);
+          Vs[q] = {2.0 * v.re, 2.0 * v.im};
         }
       }
+      // K = prod_j V[1][j] / 2 as mantissa (below 2^60) and power of two
+      const cd km = wave_prod(m);
+      const int ke = (int)uniform_value(wave_allsum(e)) - R;
       __syncthreads();
-      const cd a = sweep_pair_wave<K, U>(Vs, Ed, lane, c, w, wpi, iters);
-      const cd m = kc[0];
-      const int e2 = ke[0];
-      acc = {ldexp(m.re * a.re - m.im * a.im, e2), ldexp(m.re * a.im + m.im * a.re, e2)};
-      if (lane == 1) dst = pick;
-      else if (lane == pick) dst = 1;
+      acc = sweep_pair_wave<K, U>(Vs, Ed, lane, c, w, wpi, iters);
+#pragma unroll
+      for (int v = 0; v < SweepSums<K>::V; ++v) {
+        double re, im;  // lanes < 32 hold real parts, their partners the imaginary ones
+        both32(acc.v[v], re, im);
+        acc.v[v] = ldexp(lane < 32 ? km.re * re - km.im * im : km.re * im + km.im * re, ke);
+      }
     }
-    if (lane < K) partial[((size_t)slot * wpi + w) * K + dst] = acc;
+#pragma unroll
+    for (int v = 0; v < SweepSums<K>::V; ++v) {
+      const int q = lane_sums_index<6>(lane) + 64 * v;
+      int i = q >> 1;
+      if (ok && i == 1)
+        i = pick;
+      else if (ok && i == pick)
+        i = 1;
+      if (q < 2 * K) dst[2 * i + (q & 1)] = acc.v[v];
+    }
   }
 }
 
-// minors[slot*K + nu] = sum_w partial[(slot*wpi + w)*K + nu], fixed order.
+// Output d of item b: minor nu of the item, nu = d, or with in_mult the rank of slot d among the
+// occupied slots (0 where it is empty).
+__device__ __forceinline__ int sweep_output_minor(const int *in_mult, int in_max, int b, int d,
+                                                  int K) {
+  if (in_mult == nullptr) return d;
+  if (in_mult[(size_t)b * in_max + d] <= 0) return -1;
+  int nu = 0;
+  for (int e = 0; e < d; ++e) nu += in_mult[(size_t)b * in_max + e] > 0;
+  return nu < K ? nu : -1;
+}
+
+// minors[b*in_max + d] = sum_w partial[(b*wpi + w)*K + nu(d)], in w order.
 __global__ void sweep_reduce_kernel(const cd *__restrict__ partial, int K, int wpi, int items,
-                                    const int *__restrict__ item_count, cd *__restrict__ minors) {
+                                    const int *__restrict__ in_mult, int in_max,
+                                    cd *__restrict__ minors) {
   const int idx = blockIdx.x * blockDim.x + threadIdx.x;
-  if (idx >= items * K) return;
-  const int b = idx / K, nu = idx - b * K;
-  if (item_count && b >= *item_count) return;
+  if (idx >= items * in_max) return;
+  const int b = idx / in_max;
+  const int nu = sweep_output_minor(in_mult, in_max, b, idx - b * in_max, K);
   double re = 0.0, im = 0.0;
+  if (nu >= 0) {
 #pragma unroll 8
-  for (int w = 0; w < wpi; ++w) {  // unrolled: the loads are in flight together
-    const cd v = partial[((size_t)b * wpi + w) * K + nu];
-    re += v.re;
-    im += v.im;
+    for (int w = 0; w < wpi; ++w) {  // unrolled: the loads are in flight together
+      const cd v = partial[((size_t)b * wpi + w) * K + nu];
+      re += v.re;
+      im += v.im;
+    }
   }
   minors[idx] = {re, im};
+}
+
+// The same for many partials per item, one block per item: 256 / K slices of w, then the
+// slices in order (one thread per minor took 11 us over the 256 partials of a single item).
+__global__ __launch_bounds__(256) void sweep_reduce_wide_kernel(
+    const cd *__restrict__ partial, int K, int wpi, const int *__restrict__ in_mult, int in_max,
+    cd *__restrict__ minors) {
+  __shared__ cd part[256];
+  const int b = blockIdx.x;
+  const int slices = 256 / K, sl = threadIdx.x / K, nu = threadIdx.x - sl * K;
+  if (sl < slices) {
+    double re = 0.0, im = 0.0;
+#pragma unroll 4
+    for (int w = sl; w < wpi; w += slices) {
+      const cd v = partial[((size_t)b * wpi + w) * K + nu];
+      re += v.re;
+      im += v.im;
+    }
+    part[threadIdx.x] = {re, im};
+  }
+  __syncthreads();
+  if (threadIdx.x < K) {
+    cd v = part[threadIdx.x];
+    for (int s = 1; s < slices; ++s) v = cadd(v, part[s * K + threadIdx.x]);
+    part[threadIdx.x] = v;
+  }
+  __syncthreads();
+  for (int d = threadIdx.x; d < in_max; d += 256) {
+    const int i = sweep_output_minor(in_mult, in_max, b, d, K);
+    minors[(size_t)b * in_max + d] = i >= 0 ? part[i] : cd{0.0, 0.0};
+  }
 }
 
 }  // namespace tb
@@ -221,16 +352,15 @@ inline SweepPlan sweep_plan(int k, int64_t items, int c_override) {
   return p;
 }
 
-// LDS per wave: the item's k(k-1) columns plus 64 lanes x (c - U) corrector slots; the
-// paired kernel adds the quotients' reciprocals, the particles' extreme magnitudes and the
-// column product.
+// LDS per wave: the item's k(k-1) columns, 64 lanes x (c - U) corrector slots and the particle
+// and row lists; the paired kernel adds the quotients' reciprocals.
 inline size_t sweep_lds_bytes(int k, int c) {
   const int u = std::min(tb::kSweepU, k - 1);
-  return sizeof(tb::cd) * ((size_t)k * (k - 1) + (size_t)std::max(c - u, 0) * 64);
+  return sizeof(tb::cd) * ((size_t)k * (k - 1) + (size_t)std::max(c - u, 0) * 64) +
+         sizeof(int) * (size_t)(2 * k);
 }
 inline size_t sweep_pair_lds_bytes(int k, int c) {
-  return sweep_lds_bytes(k, c) + sizeof(tb::cd) * (size_t)(k - 1) +
-         sizeof(double) * (size_t)(2 * k) + sizeof(tb::cd) + 2 * sizeof(int);
+  return sweep_lds_bytes(k, c) + sizeof(tb::cd) * (size_t)(k - 1);
 }
 // Sizes that run the paired sweep (with a chunk holding the static block plus the pair
 // bit), at 2 waves per SIMD: up to k = 21 with five particles in broadcast form, from
@@ -247,8 +377,8 @@ constexpr bool sweep_paired() {
 }
 
 template <int K>
-int32_t launch_sweep_k(const tb::cd *Vt, int ldv, int64_t item_stride, const int *item_map,
-                       const int *item_count, int items, const SweepPlan &p, tb::cd *partial,
+int32_t launch_sweep_k(const tb::SweepSource &src, const int *item_map, const int *item_count,
+                       int items, const SweepPlan &p, tb::cd *partial,
                        hipStream_t s) {
   // Persistent grid: enough one-wave blocks to fill every SIMD a few times over.
   const int64_t tasks = (int64_t)items * p.wpi;
@@ -258,28 +388,26 @@ int32_t launch_sweep_k(const tb::cd *Vt, int ldv, int64_t item_stride, const int
   if constexpr (sweep_paired<K>()) {
     if (p.c >= U + 1) {
       hipLaunchKernelGGL((tb::sweep_pair_kernel<K, U>), dim3(grid), dim3(64),
-                         sweep_pair_lds_bytes(K, p.c), s, Vt, ldv, item_stride, item_map,
-                         item_count, items, p.c, p.wpi, p.iters, partial);
+                         sweep_pair_lds_bytes(K, p.c), s, src, item_map, item_count, items,
+                         p.c, p.wpi, p.iters, partial);
       return tbh::check_hip(hipGetLastError(), "sweep_pair_kernel");
     }
   }
   hipLaunchKernelGGL((tb::sweep_kernel<K, U, R0>), dim3(grid), dim3(64), sweep_lds_bytes(K, p.c), s,
-                     Vt, ldv, item_stride, item_map, item_count, items, p.c, p.wpi, p.iters,
+                     src, item_map, item_count, items, p.c, p.wpi, p.iters,
                      partial);
   return tbh::check_hip(hipGetLastError(), "sweep_kernel");
 }
 
 template <int K = 2>
-int32_t dispatch_sweep(int k, const tb::cd *Vt, int ldv, int64_t item_stride, const int *item_map,
+int32_t dispatch_sweep(int k, const tb::SweepSource &src, const int *item_map,
                        const int *item_count, int items, const SweepPlan &p, tb::cd *partial,
                        hipStream_t s) {
   if constexpr (K > TB_SWEEP_MAX_K) {
     return tbh::fail(TB_ERANGE, "sweep: k=%d exceeds TB_SWEEP_MAX_K=%d", k, TB_SWEEP_MAX_K);
   } else {
-    if (k == K) return launch_sweep_k<K>(Vt, ldv, item_stride, item_map, item_count, items, p,
-                                         partial, s);
-    return dispatch_sweep<K + 1>(k, Vt, ldv, item_stride, item_map, item_count, items, p, partial,
-                                 s);
+    if (k == K) return launch_sweep_k<K>(src, item_map, item_count, items, p, partial, s);
+    return dispatch_sweep<K + 1>(k, src, item_map, item_count, items, p, partial, s);
   }
 }
 
@@ -298,26 +426,41 @@ void sweep_plan_of(int k, int items, int c_override, int *c, int *wpi, int *iter
   *iters = p.iters;
 }
 
+tb::SweepSource gathered(const tb::cd *Vt, int ldv, int64_t item_stride) {
+  tb::SweepSource src{};
+  src.Vt = Vt;
+  src.ldv = ldv;
+  src.item_stride = item_stride;
+  return src;
+}
+
 // Partial sums only: partial[(item * wpi + w) * k + nu], w < *wpi. A consumer that sums
-// them in w order gets the same minors as run_sweep.
+// them in w order gets the same minors as run_sweep with up to kReduceInOrder of them.
 int32_t run_sweep_partial(int k, const tb::cd *Vt, int ldv, int64_t item_stride,
                           const int *item_map, const int *item_count, int items, int c_override,
                           tb::cd *partial, int *wpi, hipStream_t s) {
   const SweepPlan p = sweep_plan(k, items, c_override);
   *wpi = p.wpi;
-  return dispatch_sweep(k, Vt, ldv, item_stride, item_map, item_count, items, p, partial, s);
+  return dispatch_sweep(k, gathered(Vt, ldv, item_stride), item_map, item_count, items, p, partial, s);
 }
 
-// Full sweep: partial sums then the fixed-order reduction into minors[items][k].
-int32_t run_sweep(int k, const tb::cd *Vt, int ldv, int64_t item_stride, const int *item_map,
-                  const int *item_count, int items, int c_override, tb::cd *partial,
-                  tb::cd *minors, hipStream_t s) {
+// Full sweep: partial sums then the fixed-order reduction into minors[items][k], or with
+// in_mult into minors[items][in_max] by input slot (0 at empty ones).
+constexpr int kReduceInOrder = 32;
+int32_t run_sweep(int k, const tb::SweepSource &src, int items, int c_override, tb::cd *partial,
+                  const int *in_mult, int in_max, tb::cd *minors, hipStream_t s) {
   const SweepPlan p = sweep_plan(k, items, c_override);
-  int32_t rc = dispatch_sweep(k, Vt, ldv, item_stride, item_map, item_count, items, p, partial, s);
+  int32_t rc = dispatch_sweep(k, src, nullptr, nullptr, items, p, partial, s);
   if (rc) return rc;
-  const int total = items * k;
-  hipLaunchKernelGGL(tb::sweep_reduce_kernel, dim3((total + 255) / 256), dim3(256), 0, s, partial,
-                     k, p.wpi, items, item_count, minors);
+  const int outs = in_mult ? in_max : k;
+  if (p.wpi > kReduceInOrder) {
+    hipLaunchKernelGGL(tb::sweep_reduce_wide_kernel, dim3(items), dim3(256), 0, s, partial, k, p.wpi,
+                       in_mult, outs, minors);
+  } else {
+    const int total = items * outs;
+    hipLaunchKernelGGL(tb::sweep_reduce_kernel, dim3((total + 255) / 256), dim3(256), 0, s, partial,
+                       k, p.wpi, items, in_mult, outs, minors);
+  }
   return tbh::check_hip(hipGetLastError(), "sweep_reduce_kernel");
 }
 
@@ -347,6 +490,6 @@ extern "C" int32_t tb_sweep_minors_batch(const tb_complex128 *Vt, int32_t k, int
   if (!workspace || workspace_bytes < need)
     return tbh::fail(TB_EWORKSPACE, "sweep: workspace %zu bytes < required %zu", workspace_bytes,
                      need);
-  return tbs::run_sweep(k, (const tb::cd *)Vt, ldv, item_stride, nullptr, nullptr, batch, c,
-                        (tb::cd *)workspace, (tb::cd *)minors, s);
+  return tbs::run_sweep(k, tbs::gathered((const tb::cd *)Vt, ldv, item_stride), batch, c,
+                        (tb::cd *)workspace, nullptr, 0, (tb::cd *)minors, s);
 }

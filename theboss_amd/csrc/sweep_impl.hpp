@@ -67,6 +67,20 @@ namespace tb {
 constexpr int kSweepU = TB_SWEEP_U;  // Gray bits unrolled per block (static flip rows)
 constexpr int kSweepMaxC = 16;  // largest chunk (bits); sizes the LDS corrector store
 
+// Where a sweep's items come from: gathered columns V[nu][j] at Vt + item item_stride + nu ldv +
+// j, or (U set) the submatrix of U that an item's output and input slots name.
+struct SweepSource {
+  const cd *Vt;
+  int ldv;
+  int64_t item_stride;
+  const cd *U;
+  int ldu;
+  const int *out_modes, *out_mult;
+  int out_max;
+  const int *in_modes, *in_mult;
+  int in_max;
+};
+
 // h += sg * column (sg = +-1 per lane, or a compile-time sign).
 constexpr int kSweepG = 4;  // column values per LDS group
 
@@ -293,10 +307,33 @@ __device__ __forceinline__ void sweep_chunk(const cd *Vs, const Col0<K - 1, R0> 
   }
 }
 
+// One wave's result for K minors: value v of a lane is component c (0 real, 1 imaginary) of
+// minor i with 2 i + c = lane_sums_index<6>(lane) + 64 v (nothing when i >= K).
+template <int K>
+struct SweepSums {
+  static constexpr int V = (2 * K + 63) / 64;
+  double v[V];
+};
+
+// acc += the sums of mi over the wave's lanes.
+template <int K>
+__device__ __forceinline__ void sweep_add_sums(SweepSums<K> &acc, const cd (&mi)[K], bool live,
+                                               int lane) {
+  double x[2 * K];
+#pragma unroll
+  for (int i = 0; i < K; ++i) {
+    x[2 * i] = live ? mi[i].re : 0.0;
+    x[2 * i + 1] = live ? mi[i].im : 0.0;
+  }
+  lane_sums<6, 2 * K>(x, lane);
+#pragma unroll
+  for (int v = 0; v < SweepSums<K>::V; ++v) acc.v[v] += x[v];
+}
+
 // One wave's share of an item whose columns are in Vs: chunks q = (w + it * wpi) * 64 + lane
-// for it < iters. Lane i returns the sum over those chunks of minor i (in it order).
+// for it < iters, their sums added in it order.
 template <int K, int U, int R0>
-__device__ __forceinline__ cd sweep_wave(const cd *Vs, cd *Ed, int lane, int c, int w, int wpi,
+__device__ __forceinline__ SweepSums<K> sweep_wave(const cd *Vs, cd *Ed, int lane, int c, int w, int wpi,
                                          int iters) {
   constexpr int R = K - 1;
   const uint64_t nchunks = (uint64_t)1 << (K - 1 - c);
@@ -310,7 +347,7 @@ __device__ __forceinline__ cd sweep_wave(const cd *Vs, cd *Ed, int lane, int c, 
     c1.one = vgpr_one();
     asm volatile("s_nop 4");  // VALU writes of the store before its first DPP read
   }
-  cd acc = {0.0, 0.0};
+  SweepSums<K> acc{};
   for (int it = 0; it < iters; ++it) {
     const uint64_t q = ((uint64_t)w + (uint64_t)it * wpi) * 64 + lane;
     cd mi[K];
@@ -318,19 +355,7 @@ __device__ __forceinline__ cd sweep_wave(const cd *Vs, cd *Ed, int lane, int c, 
     // (the broadcast flips read other lanes' registers).
     const bool live = q < nchunks;
     sweep_chunk<K, U, R0>(Vs, c1, Ed + lane, c, live ? q : (q & (nchunks - 1)), mi);
-    if (!live) {
-#pragma unroll
-      for (int i = 0; i < K; ++i) mi[i] = {0.0, 0.0};
-    }
-#pragma unroll
-    for (int i = 0; i < K; ++i) {
-      const double re = wave_sum(mi[i].re);
-      const double im = wave_sum(mi[i].im);
-      if (lane == i) {
-        acc.re += re;
-        acc.im += im;
-      }
-    }
+    sweep_add_sums<K>(acc, mi, live, lane);
   }
   return acc;
 }
@@ -490,10 +515,10 @@ __device__ __forceinline__ void sweep_pair_chunk(const cd *S2, const ColP<K - 1>
 }
 
 // One wave's share of an item whose scaled columns are in S2, chunk c of codes (c - 1
-// super-step bits per lane): the chunk and lane mapping of sweep_wave. Lane i returns
-// minor i's sum without Kc.
+// super-step bits per lane): the chunk and lane mapping of sweep_wave. The sums come
+// without Kc.
 template <int K, int U>
-__device__ __forceinline__ cd sweep_pair_wave(const cd *S2, cd *Ed, int lane, int c, int w,
+__device__ __forceinline__ SweepSums<K> sweep_pair_wave(const cd *S2, cd *Ed, int lane, int c, int w,
                                               int wpi, int iters) {
   constexpr int R = K - 1;
   const uint64_t nchunks = (uint64_t)1 << (K - 1 - c);
@@ -502,25 +527,13 @@ __device__ __forceinline__ cd sweep_pair_wave(const cd *S2, cd *Ed, int lane, in
   for (int u = 0; u < ColP<R>::NU; ++u) load_bcast(cp.b[u], (const double *)(S2 + (u + 2) * R), lane);
   cp.one = vgpr_one();
   asm volatile("s_nop 4");  // VALU writes of the store before its first DPP read
-  cd acc = {0.0, 0.0};
+  SweepSums<K> acc{};
   for (int it = 0; it < iters; ++it) {
     const uint64_t q = ((uint64_t)w + (uint64_t)it * wpi) * 64 + lane;
     cd mi[K];
     const bool live = q < nchunks;
     sweep_pair_chunk<K, U>(S2, cp, Ed + lane, c - 1, live ? q : (q & (nchunks - 1)), mi);
-    if (!live) {
-#pragma unroll
-      for (int i = 0; i < K; ++i) mi[i] = {0.0, 0.0};
-    }
-#pragma unroll
-    for (int i = 0; i < K; ++i) {
-      const double re = wave_sum(mi[i].re);
-      const double im = wave_sum(mi[i].im);
-      if (lane == i) {
-        acc.re += re;
-        acc.im += im;
-      }
-    }
+    sweep_add_sums<K>(acc, mi, live, lane);
   }
   return acc;
 }
