@@ -299,11 +299,20 @@ int32_t tb_gccb_status(const void *workspace, void *stream);
  *   counts             uint32 per outcome, incremented (the caller zeroes them)
  *   outside            optional uint32 counter of samples not in the list (other particle
  *                      numbers, negative entries); NULL = not counted
+ * tb_outcome_histogram64 sets 64-bit counts and outside (optional) instead; they need no
+ * clearing. The workspace, of tb_outcome_histogram64_workspace_size bytes (0: none needed;
+ * at most 32 MiB of ranks and the table of their runs), lets a large call count without
+ * atomics on memory; without it (NULL, or fewer bytes) the counts are the same, slower.
  * ------------------------------------------------------------------------------- */
 int64_t tb_outcome_count(int32_t n, int32_t m, int32_t losses);
 int32_t tb_outcome_histogram(const int32_t *samples, int32_t ld, int32_t samples_n, int32_t m,
                              int32_t n, int32_t losses, uint32_t *counts, uint32_t *outside,
                              void *stream);
+size_t tb_outcome_histogram64_workspace_size(int32_t samples_n, int32_t m, int32_t n,
+                                             int32_t losses);
+int32_t tb_outcome_histogram64(const int32_t *samples, int32_t ld, int32_t samples_n, int32_t m,
+                               int32_t n, int32_t losses, int64_t *counts, int64_t *outside,
+                               void *workspace, size_t workspace_bytes, void *stream);
 
 /* ---------------------------------------------------------------------------------
  * Clock probe (measurement only; no reference counterpart). tb_clock_probe launches one

@@ -88,6 +88,8 @@ SIGNATURES = {
     "tb_perm_grad_conj_batch": (_i32, [_vp, _i32, _i32, _i64, _vp, _vp, _vp, _sz, _vp]),
     "tb_outcome_count": (_i64, [_i32, _i32, _i32]),
     "tb_outcome_histogram": (_i32, [_vp, _i32, _i32, _i32, _i32, _i32, _vp, _vp, _vp]),
+    "tb_outcome_histogram64_workspace_size": (_sz, [_i32, _i32, _i32, _i32]),
+    "tb_outcome_histogram64": (_i32, [_vp, _i32, _i32, _i32, _i32, _i32, _vp, _vp, _vp, _sz, _vp]),
     "tb_gccb_workspace_size": (_sz, [ctypes.POINTER(GccbConfig)]),
     "tb_gccb_sample": (
         _i32,

@@ -247,9 +247,13 @@ def outcome_histogram(samples, particles_number: int, losses: bool = False):
         raise ValueError(f"samples must be S x m, got {tuple(samples.shape)}")
     S, m = samples.shape
     count = outcome_count(particles_number, m, losses)
-    counts = T.zeros(count, dtype=T.int32, device=samples.device)  # uint32 counters
-    outside = T.zeros(1, dtype=T.int32, device=samples.device)
-    L.check(L.load().tb_outcome_histogram(D.ptr(samples), m, S, m, int(particles_number),
-                                          1 if losses else 0, D.ptr(counts), D.ptr(outside),
-                                          D.stream_ptr(samples.device)))
-    return counts.to(T.int64), int(outside.item())
+    n, losses = int(particles_number), 1 if losses else 0
+    counts = T.empty(count, dtype=T.int64, device=samples.device)
+    outside = T.empty(1, dtype=T.int64, device=samples.device)
+    lib = L.load()
+    need = lib.tb_outcome_histogram64_workspace_size(S, m, n, losses)
+    ws = T.empty(need, dtype=T.uint8, device=samples.device) if need else None
+    L.check(lib.tb_outcome_histogram64(D.ptr(samples), m, S, m, n, losses, D.ptr(counts),
+                                       D.ptr(outside), D.ptr(ws) if need else None, need,
+                                       D.stream_ptr(samples.device)))
+    return counts, int(outside.item())
