@@ -180,6 +180,23 @@ int32_t tb_guan_perm_outer_ws(const tb_complex128 *U, int32_t ldu, const int32_t
                               int32_t n_in, int32_t formula, tb_complex128 *out, void *workspace,
                               size_t workspace_bytes, void *stream);
 
+/* The layers of GCC-A sampling (generalized_cliffords_simulation_strategy.py:136-247) for
+ * prefixes_n prefixes (rows of m occupations):
+ *   pmf[p*m + o] = sum_i weights[i] |perm(U[prefix_p + e_o, s_i])|^2
+ * over the n_in input rows (in_modes, in_mult) of tb_guan_perm_outer_ws, each of one particle
+ * more than the prefixes; U is m x m.
+ *   width      at least the most modes a prefix occupies, >= 1 (width + 1 and in_max as
+ *              out_max and in_max of tb_guan_perm_outer)
+ *   common     nonzero: the input rows are known to have a small common state (as above)
+ *   workspace  tb_gcca_layer_workspace_size bytes (holds the permanents; 0 = sizes refused) */
+size_t tb_gcca_layer_workspace_size(int32_t m, int32_t prefixes_n, int32_t width, int32_t in_max,
+                                    int32_t n_in, int32_t common);
+int32_t tb_gcca_layer_pmfs(const tb_complex128 *U, int32_t m, const int32_t *prefixes,
+                           int32_t prefixes_n, int32_t width, const int32_t *in_modes,
+                           const int32_t *in_mult, int32_t in_max, int32_t n_in,
+                           const double *weights, int32_t formula, int32_t common, double *pmf,
+                           void *workspace, size_t workspace_bytes, void *stream);
+
 /* ---------------------------------------------------------------------------------
  * Clifford & Clifford submatrices permanents: all input-particle-deleted minors in one
  * sweep. Replaces BSCCRyserSubmatricesPermanentCalculator.compute_permanents

@@ -78,6 +78,9 @@ SIGNATURES = {
     "tb_guan_outer_workspace_size": (_sz, [_i32, _i32, _i32, _i32, _i32]),
     "tb_guan_perm_outer_ws": (
         _i32, [_vp, _i32, _vp, _vp, _i32, _i32, _vp, _vp, _i32, _i32, _i32, _vp, _vp, _sz, _vp]),
+    "tb_gcca_layer_workspace_size": (_sz, [_i32, _i32, _i32, _i32, _i32, _i32]),
+    "tb_gcca_layer_pmfs": (_i32, [_vp, _i32, _vp, _i32, _i32, _vp, _vp, _i32, _i32, _vp, _i32,
+                                  _i32, _vp, _vp, _sz, _vp]),
     "tb_cc_workspace_size": (_sz, [_i32, _i32, _i32, _i32]),
     "tb_cc_submatrices_batch": (
         _i32, [_vp, _i32, _vp, _vp, _i32, _vp, _vp, _i32, _i32, _i32, _i32, _vp, _vp, _sz, _vp]),

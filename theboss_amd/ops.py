@@ -90,6 +90,32 @@ def guan_perm_outer(U, out_modes, out_mult, in_modes, in_mult, formula: int = L.
     return out
 
 
+def gcca_layer_pmfs(U, prefixes, width: int, in_modes, in_mult, weights,
+                    formula: int = L.TB_FORMULA_RYSER, common: bool = False):
+    """The layers of P prefixes (P x m occupations, int32) on the m x m matrix U: a (P, m)
+    tensor of sum_i weights[i] |perm(U[prefix_p + e_o, s_i])|^2 over the input rows s_i of
+    guan_perm_outer. `width` is the most modes a prefix occupies (at least 1); `common` as in
+    guan_perm_outer."""
+    T = D.require_gpu()
+    U, prefixes = _c128(U, "U"), _i32(prefixes, "prefixes")
+    in_modes, in_mult = _i32(in_modes, "in_modes"), _i32(in_mult, "in_mult")
+    P, m = prefixes.shape
+    n_in, in_max = in_modes.shape
+    if tuple(U.shape) != (m, m) or in_mult.shape != in_modes.shape or tuple(weights.shape) != (n_in,) \
+            or weights.dtype != T.float64 or not weights.is_contiguous():
+        raise ValueError("gcca_layer_pmfs needs U m x m, prefixes P x m and a float64 weight per "
+                         "input row")
+    pmf = T.empty((P, m), dtype=T.float64, device=U.device)
+    lib = L.load()
+    need = lib.tb_gcca_layer_workspace_size(m, P, width, in_max, n_in, 1 if common else 0)
+    ws = T.empty(max(need, 1), dtype=T.uint8, device=U.device)
+    L.check(lib.tb_gcca_layer_pmfs(
+        D.ptr(U), m, D.ptr(prefixes), P, width, D.ptr(in_modes), D.ptr(in_mult), in_max, n_in,
+        D.ptr(weights), formula, 1 if common else 0, D.ptr(pmf), D.ptr(ws), need,
+        D.stream_ptr(U.device)))
+    return pmf
+
+
 def cc_submatrices_batch(U, out_modes, out_mult, in_modes, in_mult, k: int,
                          collision_free: bool):
     """All input-deleted minors per item: result[b, d] = perm(U[t_b, s_b - e_d])."""

@@ -261,6 +261,45 @@ class _GuanGPUCalculator(BSPermanentCalculatorBase):
         Ud = _cached(_content_key("U", dev, U), lambda: D.to_device_c128(U, dev))
         return ops.guan_perm_outer(Ud, td[0], td[1], cs[0], cs[1], self.formula, common)
 
+    def layer_inputs(self, S: np.ndarray, weights: np.ndarray):
+        """The input side of GCC-A layers of k particles, on the device: S rows of k >= 1
+        particles and a weight for each. What compute_layer_pmfs takes, or None when the rows
+        need the Glynn fallback (as compute_permanent_layer; with at most 28 particles a row
+        has at most 2^28 Guan codes)."""
+        S = np.asarray(S, dtype=np.int64)
+        k = int(S[0].sum()) if len(S) else 0
+        if k < 1 or k > 28 or np.any(S.sum(axis=1) != k):
+            return None
+        T = D.require_gpu()
+        modes, mult = compact_batch(S)
+        n_in, W = modes.shape
+        if W > min(L.TB_GUAN_MAX_COLS, L.TB_GUAN_MAX_ROWS):
+            return None
+        host = np.empty(n_in * (1 + W), dtype=np.float64)  # weights, modes, multiplicities
+        host[:n_in] = weights
+        rows = host[n_in:].view(np.int32).reshape(2, n_in, W)
+        rows[0], rows[1] = modes, mult
+        dev = T.from_numpy(host).to(D.device())
+        rows = dev[n_in:].view(T.int32).view(2, n_in, W)
+        return k, rows[0], rows[1], dev[:n_in], has_small_common_state(S)
+
+    def compute_layer_pmfs(self, inputs, prefixes: np.ndarray):
+        """A (len(prefixes), m) float64 device tensor: the weighted sums over `inputs`
+        (layer_inputs) of |perm(U[prefix_p + e_o, S[i]])|^2, for prefixes of one particle less,
+        by one tb_gcca_layer_pmfs call. None when a prefix needs the Glynn fallback."""
+        k, modes, mult, weights, common = inputs
+        Pf = np.ascontiguousarray(prefixes, dtype=np.int32)
+        U = np.asarray(self._matrix, dtype=np.complex128)
+        if Pf.ndim != 2 or U.shape != (Pf.shape[1],) * 2 or np.any(Pf.sum(axis=1) != k - 1):
+            return None
+        width = max(1, int(np.count_nonzero(Pf, axis=1).max(initial=0)))
+        if max(modes.shape[1], width + 1) > min(L.TB_GUAN_MAX_COLS, L.TB_GUAN_MAX_ROWS):
+            return None
+        dev = modes.device
+        Ud = _cached(_content_key("U", dev, U), lambda: D.to_device_c128(U, dev))
+        return ops.gcca_layer_pmfs(Ud, D.to_device_i32(Pf, dev), width, modes, mult, weights,
+                                   self.formula, common)
+
     def compute_permanent(self) -> complex128:
         s, t = self._checked_states()
         if len(s) == 0:

@@ -75,8 +75,8 @@ class GeneralizedCliffordsUniformLossesSimulationStrategy(GeneralizedCliffordsSi
     def _particles_kept(self, samples: int) -> np.ndarray:
         return self._rng.random(samples) < self._transmissivity
 
-    def _calculate_layers(self, keys) -> None:
-        super()._calculate_layers(keys)
+    def _calculate_layers(self, keys, rows=None) -> None:
+        super()._calculate_layers(keys, rows)
         n = self.number_of_input_photons
         for key in keys:
             for output, p in zip(self.possible_outputs[key], self.pmfs[key]):
