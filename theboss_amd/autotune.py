@@ -97,27 +97,39 @@ def sweep_builtin(k: int, items: int) -> int:
 
 
 def glynn_builtin(n: int, batch: int) -> int:
-    """The FP64 kernels' built-in chunk (two waves per SIMD): ~8192 waves, then up to two
-    sizes larger while the rounds of 2 x 1024 waves stay as full, scored by round fill
-    times the share of a chunk left after seeding, (n - 2) 2 / (5 2^c)."""
+    """The FP64 kernels' built-in chunk. Bound: ~8192 waves, then up to two sizes larger while
+    the rounds of 2 x 1024 waves stay as full, scored by round fill times the share of a chunk
+    left after seeding, (n - 2) 2 / (5 2^c). Below it, the least ceil(waves / 1024) (2^c + 1.1 n),
+    a launch of at most 1024 waves counting 1.02 rounds."""
     nb = n - 1
     want = 0
     while (batch << want) < 8192 and want < 30:
         want += 1
+    low = min(max(2, glynn_paired_min_c(n)), nb - 8)
 
     def clamp(c):
-        return max(2, min(c, 12, nb - 8))
+        return min(max(low, min(c, 12)), nb - 8)
 
     c0 = clamp(max(nb - 6 - want, min(7, nb - 8)))
-    best, best_c = -1.0, c0
+    best, top = -1.0, c0
     for c in (c0, c0 + 1, c0 + 2):
         if clamp(c) != c:
             continue
         rounds = batch * 2.0 ** (nb - c - 6) / 2048
         score = rounds / math.ceil(rounds) * (1 - (n - 2) * 2.0 / (5 * 2.0 ** c))
         if score > best + 1e-9:
-            best, best_c = score, c
+            best, top = score, c
+    least, best_c = math.inf, top
+    for c in range(top, low - 1, -1):
+        rounds = max(math.ceil(batch * 2.0 ** (nb - c - 6) / 1024), 1.02)
+        if rounds * (2.0 ** c + 1.1 * n) < least:
+            least, best_c = rounds * (2.0 ** c + 1.1 * n), c
     return best_c
+
+
+def glynn_paired_min_c(n: int) -> int:
+    """Least chunk of the FP64 walk: its static bits, 3 and the pair bit for n = 14..39."""
+    return 4 if 14 <= n <= 39 else (3 if n >= 25 else 2)
 
 
 def grad_columns(n: int) -> int:

@@ -345,4 +345,43 @@ __device__ __forceinline__ double vgpr_one() {
   return one;
 }
 
+// Largest of one value per lane, in every lane.
+__device__ __forceinline__ double wave_allmax(double v) {
+  const uint64_t u = __builtin_bit_cast(uint64_t, v);
+  const auto l32 = __builtin_amdgcn_permlane32_swap((uint32_t)u, (uint32_t)u, false, false);
+  const auto h32 = __builtin_amdgcn_permlane32_swap((uint32_t)(u >> 32), (uint32_t)(u >> 32), false, false);
+  v = fmax(join64(l32[0], h32[0]), join64(l32[1], h32[1]));
+  const uint64_t t = __builtin_bit_cast(uint64_t, v);
+  const auto l16 = __builtin_amdgcn_permlane16_swap((uint32_t)t, (uint32_t)t, false, false);
+  const auto h16 = __builtin_amdgcn_permlane16_swap((uint32_t)(t >> 32), (uint32_t)(t >> 32), false, false);
+  v = fmax(join64(l16[0], h16[0]), join64(l16[1], h16[1]));
+  v = fmax(v, dpp_perm<0x128>(v));
+  v = fmax(v, dpp_perm<0x124>(v));
+  v = fmax(v, dpp_perm<0x122>(v));
+  return fmax(v, dpp_perm<0x121>(v));
+}
+
+// Both halves' value of a lane pair at distance 32: {low lane's, high lane's}, in both.
+__device__ __forceinline__ void both32(double v, double &lo, double &hi) {
+  const uint64_t u = __builtin_bit_cast(uint64_t, v);
+  const auto a = __builtin_amdgcn_permlane32_swap((uint32_t)u, (uint32_t)u, false, false);
+  const auto b = __builtin_amdgcn_permlane32_swap((uint32_t)(u >> 32), (uint32_t)(u >> 32), false, false);
+  lo = join64(a[0], b[0]);
+  hi = join64(a[1], b[1]);
+}
+
+// Product of one complex value per lane over the wave (wave-uniform).
+__device__ __forceinline__ cd wave_prod(cd v) {
+  cd a, b;
+  both32(v.re, a.re, b.re);
+  both32(v.im, a.im, b.im);
+  v = cmul(a, b);
+  v = cmul(v, {__shfl_xor(v.re, 16, 64), __shfl_xor(v.im, 16, 64)});
+  v = cmul(v, {dpp_perm<0x128>(v.re), dpp_perm<0x128>(v.im)});
+  v = cmul(v, {dpp_perm<0x124>(v.re), dpp_perm<0x124>(v.im)});
+  v = cmul(v, {dpp_perm<0x122>(v.re), dpp_perm<0x122>(v.im)});
+  v = cmul(v, {dpp_perm<0x121>(v.re), dpp_perm<0x121>(v.im)});
+  return {uniform_value(v.re), uniform_value(v.im)};
+}
+
 }  // namespace tb

@@ -5,27 +5,28 @@
 #include "glynn_impl.hpp"
 
 namespace tbgl {
-int32_t glynn_dispatch_f64(int n, const tb::cpx<double> *A, int64_t mstride, int batch,
-                           tb::cd *out, tb::cd *partial, int *handled, int wpm_cap, int c_pref,
-                           hipStream_t s) {
-  return dispatch_glynn<double>(n, A, mstride, (const tb::cd *)A, mstride, batch, out, partial,
-                                handled, wpm_cap, c_pref, s);
+int32_t glynn_dispatch_f64(int n, const tb::cd *A, int64_t mstride, int batch, tb::cd *out,
+                           tb::cd *partial, int *handled, int wpm_cap, int c_pref, hipStream_t s) {
+  return dispatch_glynn<double>(n, A, mstride, batch, out, partial, handled, wpm_cap, c_pref, s);
 }
 }  // namespace tbgl
 
 namespace {
 size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
 
-// The "handled" flags of the paired walk (one int per matrix) ahead of the partials.
+// The "handled" flags of the paired FP32 walk (one int per matrix) ahead of the partials.
 size_t tbgl_flag_bytes(int batch) { return align256((size_t)batch * sizeof(int)); }
 
 // Partials per matrix the workspace holds: the largest over every plan a launch of n can
 // make, i.e. every lower bound on C (the static bits, 2..4, and the paired walks' static
-// bits plus one) and every residency the plan may count (2, 3 or 4 waves per SIMD).
+// bits plus one), every residency the plan may count (2, 3 or 4 waves per SIMD) and both kinds
+// of column sums.
 int tbgl_partial_wpm(int n, int batch, int c_pref) {
   int wpm = 0;
   for (int u : {2, 3, 4, tbgl::glynn_u_max(n)})
-    for (int slots : {2, 3, 4}) wpm = std::max(wpm, tbgl::glynn_plan(n, batch, c_pref, u, slots).wpm);
+    for (int slots : {2, 3, 4})
+      for (int grow : {0, 2})
+        wpm = std::max(wpm, tbgl::glynn_plan(n, batch, c_pref, u, slots, grow).wpm);
   return wpm;
 }
 
@@ -45,6 +46,8 @@ bool runs_fp32(int n, int precision) {
 size_t glynn_workspace_bytes(int n, int batch, int precision, int c_pref) {
   if (n <= 1 || batch <= 0 || n > TB_GLYNN_MAX_N) return 0;
   size_t bytes = tbgl_partial_bytes(n, batch, c_pref);
+  // room for an FP32 copy of the matrices, which callers may rely on; the kernels convert as
+  // they stage
   if (n >= tbgl::kWideMinN && runs_fp32(n, precision))
     bytes += align256((size_t)batch * n * n * sizeof(tb::cpx<float>));
   return bytes;
@@ -91,27 +94,14 @@ extern "C" int32_t tb_glynn_batch(const tb_complex128 *A, int32_t n, int32_t bat
   int *handled = (int *)ws;
   tb::cd *partial = ws ? (tb::cd *)(ws + tbgl_flag_bytes(batch)) : nullptr;
   const int wpm_cap = n >= tbgl::kWideMinN ? tbgl_partial_wpm(n, batch, c_pref) : 0;
-  if (!runs_fp32(n, precision))
-    return tbgl::glynn_dispatch_f64(n, (const tb::cpx<double> *)A, matrix_stride, batch, o,
-                                    partial, handled, wpm_cap, c_pref, s);
-  if (n < tbgl::kWideMinN)  // the SMALL kernel converts as it stages
-    return tbgl::glynn_dispatch_f32(n, nullptr, 0, (const tb::cd *)A, matrix_stride, batch, o,
-                                    partial, handled, wpm_cap, c_pref, s);
-  // FP32 column sums: convert once into the tail of the workspace.
-  float *A32 = (float *)(ws + tbgl_partial_bytes(n, batch, c_pref));
-  const int64_t total = (int64_t)batch * n * n;
-  hipLaunchKernelGGL(tb::to_fp32_kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, s,
-                     (const tb::cd *)A, matrix_stride, n, batch, A32);
-  int32_t rc = tbh::check_hip(hipGetLastError(), "to_fp32_kernel");
-  if (rc) return rc;
-  return tbgl::glynn_dispatch_f32(n, (const tb::cpx<float> *)A32, (int64_t)n * n,
-                                  (const tb::cd *)A, matrix_stride, batch, o, partial, handled,
-                                  wpm_cap, c_pref, s);
+  const auto dispatch =
+      runs_fp32(n, precision) ? tbgl::glynn_dispatch_f32 : tbgl::glynn_dispatch_f64;
+  return dispatch(n, (const tb::cd *)A, matrix_stride, batch, o, partial, handled, wpm_cap, c_pref, s);
 }
 
 // ------------------------------------------------------------------------------------
 // tb_glynn_batch_noalloc: the same launches with their scratch memory (per-wave partial
-// sums, the FP32 copy of the matrices) in a static device array instead of a caller's
+// sums, flags) in a static device array instead of a caller's
 // workspace, for callers that cannot allocate. `scratch` is the array's host-side name
 // only; its address on a device comes from hipGetSymbolAddress, taken once per device
 // with that device current, and that address is what the launches receive.

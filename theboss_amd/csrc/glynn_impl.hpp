@@ -220,25 +220,15 @@ __device__ __forceinline__ void glynn_lane(P M, int C, uint64_t q0, uint64_t qst
   }
 }
 
-// WIDE: the 4 waves of a workgroup share one matrix, staged once into LDS; every flip is
-// a broadcast LDS read. Grid: batch * (wpm/4) workgroups; wave wq of matrix b covers
-// chunks q = (wq + it*wpm)*64 + lane. Strides count complex elements.
-// `handled` (may be null): matrices whose partials the paired kernel already wrote.
+// Wave of the workgroup, in an SGPR.
+__device__ __forceinline__ int wave_in_block() {
+  return __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+}
+
+// The plain walk of one wave (wq of wpm) over the matrix in LDS.
 template <int N, int U, int R0, typename F>
-__global__ __launch_bounds__(256) TB_WIDE_ATTR(N) void glynn_wide_kernel(const cpx<F> *__restrict__ A,
-                                                         int64_t mstride, int C, int wpm, int iters,
-                                                         cd *__restrict__ partial,
-                                                         const int *__restrict__ handled) {
-  __shared__ cpx<F> Ms[N * N];
-  const int lane = threadIdx.x & 63;
-  const int wgs_per_matrix = wpm >> 2;
-  const int b = blockIdx.x / wgs_per_matrix;
-  if (handled != nullptr && handled[b] != 0) return;
-  const int wq = (blockIdx.x - b * wgs_per_matrix) * 4 + (threadIdx.x >> 6);
-  const cpx<F> *src = A + (size_t)b * mstride;
-  for (int e = threadIdx.x; e < N * N; e += 256) Ms[e] = src[e];
-  __syncthreads();
-  double are = 0.0, aim = 0.0;
+__device__ __forceinline__ void glynn_wide_walk(const cpx<F> *Ms, int C, int wq, int wpm, int iters,
+                                                double &are, double &aim) {
   // R0 = 0: row 0's first values in SGPRs; 1: row 0 in VGPRs; 2 (FP64): rows 0..U+1
   // (n <= TB_GLYNN_BCAST_WIDE_MAX_N) or 0..U-1 in broadcast form; 3: rows 0..U-1 (every
   // static flip) in VGPRs.
@@ -247,10 +237,49 @@ __global__ __launch_bounds__(256) TB_WIDE_ATTR(N) void glynn_wide_kernel(const c
   constexpr int B = (R0 == 2) ? (BW < N - 1 ? BW : N - 1) : 0;
   constexpr int RR = (R0 == 2) ? 0 : (R0 == 3 ? U : R0);  // rows in plain VGPRs
   glynn_lane<N, U, RR, F, const cpx<F> *, (S < N ? S : N), B>(
-      (const cpx<F> *)Ms, C, (uint64_t)wq * 64 + lane, (uint64_t)wpm * 64, iters, are, aim);
-  are = wave_sum(are);
-  aim = wave_sum(aim);
-  if (lane == 0) partial[(size_t)b * wpm + wq] = {are, aim};
+      Ms, C, (uint64_t)wq * 64 + (threadIdx.x & 63), (uint64_t)wpm * 64, iters, are, aim);
+}
+
+// A wave's sum goes to its partial; a matrix of one workgroup (wpm = 4) is summed here and
+// needs no second launch. With the matrices that the paired walk cannot take walked in the same
+// kernel that is one launch instead of three: 256 matrices of n = 14 take 14 us, not 28.
+__device__ __forceinline__ void glynn_store(double re, double im, int b, int wq, int wpm, cd *sums,
+                                            cd *__restrict__ partial, cd *__restrict__ out) {
+  const bool first = (threadIdx.x & 63) == 0;
+  if (wpm > 4) {
+    if (first) partial[(size_t)b * wpm + wq] = {re, im};
+    return;
+  }
+  if (first) sums[wq & 3] = {re, im};
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    const cd t = cadd(cadd(sums[0], sums[1]), cadd(sums[2], sums[3]));
+    out[b] = {2.0 * t.re, 2.0 * t.im};
+  }
+}
+
+// WIDE: the 4 waves of a workgroup share one matrix, staged once into LDS (and converted on
+// the way for FP32 column sums); every flip is a broadcast LDS read. Grid: batch * (wpm/4)
+// workgroups; wave wq of matrix b covers chunks q = (wq + it*wpm)*64 + lane. Strides count
+// complex elements. `handled` (may be null): matrices the paired kernel already did.
+template <int N, int U, int R0, typename F>
+__global__ __launch_bounds__(256) TB_WIDE_ATTR(N) void glynn_wide_kernel(const cd *__restrict__ A,
+                                                         int64_t mstride, int C, int wpm, int iters,
+                                                         cd *__restrict__ partial,
+                                                         const int *__restrict__ handled,
+                                                         cd *__restrict__ out) {
+  __shared__ cpx<F> Ms[N * N];
+  __shared__ cd sums[4];
+  const int wgs_per_matrix = wpm >> 2;
+  const int b = blockIdx.x / wgs_per_matrix;
+  if (handled != nullptr && handled[b] != 0) return;
+  const int wq = (blockIdx.x - b * wgs_per_matrix) * 4 + wave_in_block();
+  const cd *src = A + (size_t)b * mstride;
+  for (int e = threadIdx.x; e < N * N; e += 256) Ms[e] = {(F)src[e].re, (F)src[e].im};
+  __syncthreads();
+  double are = 0.0, aim = 0.0;
+  glynn_wide_walk<N, U, R0, F>(Ms, C, wq, wpm, iters, are, aim);
+  glynn_store(wave_sum(are), wave_sum(aim), b, wq, wpm, sums, partial, out);
 }
 
 // ------------------------------------------------------------------------------------
@@ -391,82 +420,104 @@ __device__ __forceinline__ void glynn_pair_lane(const cpx<double> *S2, int C, ui
   }
 }
 
-// PAIRED WIDE kernel: grid, chunks and partial layout of glynn_wide_kernel with C Gray
-// bits per chunk of codes (C - 1 super-step bits). Writes handled[b] (1: this kernel wrote
-// matrix b's partials; 0: left to the plain kernel).
-template <int N, int U, int B>
-__global__ __launch_bounds__(256) TB_WIDE_ATTR(N) void glynn_pair_kernel(
-    const cpx<double> *__restrict__ A, int64_t mstride, int C, int wpm, int iters,
-    cd *__restrict__ partial, int *__restrict__ handled) {
-  __shared__ cpx<double> Ms[N * N];
-  __shared__ cd inv0[N];
-  __shared__ double rmin[N], rmax[N];
-  __shared__ int pick, Ke;
-  __shared__ cd Km;
-  const int lane = threadIdx.x & 63;
-  const int wgs_per_matrix = wpm >> 2;
-  const int b = blockIdx.x / wgs_per_matrix;
-  const int wg = blockIdx.x - b * wgs_per_matrix;
-  const int wq = wg * 4 + (threadIdx.x >> 6);
-  const cpx<double> *src = A + (size_t)b * mstride;
-  for (int e = threadIdx.x; e < N * N; e += 256) Ms[e] = src[e];
-  __syncthreads();
-  if (threadIdx.x < N) {
-    double lo = INFINITY, hi = 0.0;
-    for (int j = 0; j < N; ++j) {
-      const cpx<double> v = Ms[threadIdx.x * N + j];
+// The pair row of the matrix in Ms (its row with the largest smallest entry, row r), or -1
+// where that is too small against the largest entry of all: the same value in every wave.
+// Four lanes look at each row, and every wave then compares the rows itself. rmin, rmax: N
+// values each. Ends with the barrier between the looks and the compare only.
+template <int N>
+__device__ __forceinline__ int pair_row(const cd *Ms, double *rmin, double *rmax) {
+  if (threadIdx.x < 4 * N) {
+    const int row = threadIdx.x >> 2;
+    double lo = INFINITY, hi = 0.0;  // of the squared magnitudes
+    for (int j = threadIdx.x & 3; j < N; j += 4) {
+      const cd v = Ms[row * N + j];
       const double a = fma(v.re, v.re, v.im * v.im);
       lo = fmin(lo, a);
       hi = fmax(hi, a);
     }
-    rmin[threadIdx.x] = lo;
-    rmax[threadIdx.x] = hi;
-  }
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    int best = 0;
-    double mx = 0.0;
-    for (int i = 0; i < N; ++i) {
-      if (rmin[i] > rmin[best]) best = i;
-      mx = fmax(mx, rmax[i]);
+    lo = fmin(lo, dpp_perm<0xb1>(lo));  // quad_perm 1,0,3,2 and 2,3,0,1
+    hi = fmax(hi, dpp_perm<0xb1>(hi));
+    lo = fmin(lo, dpp_perm<0x4e>(lo));
+    hi = fmax(hi, dpp_perm<0x4e>(hi));
+    if ((threadIdx.x & 3) == 0) {
+      rmin[row] = lo;
+      rmax[row] = hi;
     }
-    const bool ok = mx > 0.0 && mx <= 1.7976931348623157e308 && rmin[best] >= kPairMinRel2 * mx;
-    pick = ok ? best : -1;
-    if (wg == 0) handled[b] = ok ? 1 : 0;
   }
   __syncthreads();
-  const int r = pick;
-  if (r < 0) return;  // uniform over the workgroup
-  if (r != 0 && threadIdx.x < N) {
-    const cpx<double> t = Ms[threadIdx.x];
-    Ms[threadIdx.x] = Ms[r * N + threadIdx.x];
-    Ms[r * N + threadIdx.x] = t;
+  const int lane = threadIdx.x & 63;
+  const double mn = lane < N ? rmin[lane] : -1.0, mx = lane < N ? rmax[lane] : 0.0;
+  const double top = wave_allmax(mx), best = wave_allmax(mn);
+  if (!(top > 0.0 && top <= 1.7976931348623157e308 && best >= kPairMinRel2 * top)) return -1;
+  return __ffsll((unsigned long long)__ballot(mn == best)) - 1;  // the first such row
+}
+
+// Wave 0: swaps row r with row 0, whose old entries go to row r, and leaves the reciprocals
+// of the new row 0 in inv0 (scaled by a power of two so that the square stays in range) and
+// K = prod_j M[0][j] / 2 as Km 2^Ke. Row 0 itself is not written back.
+template <int N>
+__device__ __forceinline__ void pair_divisors(cd *Ms, int r, cd *inv0, cd *Km, int *Ke) {
+  const int lane = threadIdx.x;
+  cd m = {1.0, 0.0};
+  double e = 0.0;
+  if (lane < N) {
+    const cd v = Ms[r * N + lane];
+    if (r != 0) Ms[r * N + lane] = Ms[lane];
+    const int ex = ilogb(fmax(fabs(v.re), fabs(v.im)));
+    m = {ldexp(v.re, -ex), ldexp(v.im, -ex)};
+    const double d = fma(m.re, m.re, m.im * m.im);
+    inv0[lane] = {ldexp(m.re / d, -ex), ldexp(-m.im / d, -ex)};
+    e = (double)ex;
   }
-  __syncthreads();
-  if (threadIdx.x < N) inv0[threadIdx.x] = cinv_scaled(cd{Ms[threadIdx.x].re, Ms[threadIdx.x].im});
-  if (threadIdx.x == 64) {  // K = prod_j M[0][j] / 2 as mantissa x 2^Ke
-    cd k;
-    int ke;
-    prod_half_scaled((const cd *)Ms, N, k, ke);
-    Km = k;
-    Ke = ke;
+  const cd k = wave_prod(m);  // below 2^60: each mantissa is at most 2 sqrt 2
+  const double ke = wave_allsum(e);
+  if (lane == 0) {
+    *Km = k;
+    *Ke = (int)ke - N;
   }
+}
+
+// PAIRED WIDE kernel: grid, chunks and partial layout of glynn_wide_kernel with C Gray
+// bits per chunk of codes (C - 1 super-step bits). A matrix without a pair row takes the
+// plain walk (U0 static bits) in the same workgroups.
+template <int N, int U, int B, int U0, int R0>
+__global__ __launch_bounds__(256) TB_WIDE_ATTR(N) void glynn_pair_kernel(
+    const cd *__restrict__ A, int64_t mstride, int C, int wpm, int iters, cd *__restrict__ partial,
+    cd *__restrict__ out) {
+  __shared__ cd Ms[N * N];
+  __shared__ cd inv0[N];
+  __shared__ double rmin[N], rmax[N];
+  __shared__ int Ke;
+  __shared__ cd Km;
+  __shared__ cd sums[4];
+  const int lane = threadIdx.x & 63;
+  const int wgs_per_matrix = wpm >> 2;
+  const int b = blockIdx.x / wgs_per_matrix;
+  const int wq = (blockIdx.x - b * wgs_per_matrix) * 4 + wave_in_block();
+  const cd *src = A + (size_t)b * mstride;
+  for (int e = threadIdx.x; e < N * N; e += 256) Ms[e] = src[e];
   __syncthreads();
-  for (int e = threadIdx.x; e < (N - 1) * N; e += 256) {
-    const int i = 1 + e / N, j = e - (i - 1) * N;
-    const cd v = cmul(cd{Ms[i * N + j].re, Ms[i * N + j].im}, inv0[j]);
-    Ms[i * N + j] = {2.0 * v.re, 2.0 * v.im};
-  }
-  __syncthreads();
+  const int r = pair_row<N>(Ms, rmin, rmax);
   double are = 0.0, aim = 0.0;
-  glynn_pair_lane<N, U, B>(Ms, C - 1, (uint64_t)wq * 64 + lane, (uint64_t)wpm * 64, iters, are, aim);
+  if (r < 0) {  // uniform over the workgroup
+    glynn_wide_walk<N, U0, R0, double>((const cpx<double> *)Ms, C, wq, wpm, iters, are, aim);
+    glynn_store(wave_sum(are), wave_sum(aim), b, wq, wpm, sums, partial, out);
+    return;
+  }
+  if (threadIdx.x < 64) pair_divisors<N>(Ms, r, inv0, &Km, &Ke);
+  __syncthreads();
+  for (int e = N + threadIdx.x; e < N * N; e += 256) {
+    const cd v = cmul(Ms[e], inv0[e % N]);
+    Ms[e] = {2.0 * v.re, 2.0 * v.im};
+  }
+  __syncthreads();
+  glynn_pair_lane<N, U, B>((const cpx<double> *)Ms, C - 1, (uint64_t)wq * 64 + lane,
+                           (uint64_t)wpm * 64, iters, are, aim);
   are = wave_sum(are);
   aim = wave_sum(aim);
-  if (lane == 0) {
-    const cd k = Km;
-    partial[(size_t)b * wpm + wq] = {ldexp(k.re * are - k.im * aim, Ke),
-                                     ldexp(k.re * aim + k.im * are, Ke)};
-  }
+  const cd k = Km;
+  glynn_store(ldexp(k.re * are - k.im * aim, Ke), ldexp(k.re * aim + k.im * are, Ke), b, wq, wpm,
+              sums, partial, out);
 }
 
 // ------------------------------------------------------------------------------------
@@ -705,81 +756,44 @@ __device__ __forceinline__ void glynn_pair_lane_f32(const cpx<float> *S2, int C,
 }
 
 // PAIRED WIDE kernel, FP32 column sums: reads the FP64 matrices (the quotients and the
-// row-0 product are formed in FP64), writes partials and handled[] like glynn_pair_kernel.
+// row-0 product are formed in FP64). A matrix without a pair row is left to the plain kernel
+// (handled[b] = 0, else 1), whose rows need more registers than this kernel's waves have.
 template <int N, int U, int SR, int S2P, int WPE>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE))) void glynn_pair_kernel_f32(
     const cd *__restrict__ A, int64_t mstride, int C, int wpm, int iters,
-    cd *__restrict__ partial, int *__restrict__ handled) {
+    cd *__restrict__ partial, int *__restrict__ handled, cd *__restrict__ out) {
   __shared__ cd Ms[N * N];
   __shared__ cpx<float> Sf[N * N];
   __shared__ cd inv0[N];
   __shared__ double rmin[N], rmax[N];
-  __shared__ int pick, Ke;
+  __shared__ int Ke;
   __shared__ cd Km;
+  __shared__ cd sums[4];
   const int lane = threadIdx.x & 63;
   const int wgs_per_matrix = wpm >> 2;
   const int b = blockIdx.x / wgs_per_matrix;
   const int wg = blockIdx.x - b * wgs_per_matrix;
-  const int wq = wg * 4 + (threadIdx.x >> 6);
+  const int wq = wg * 4 + wave_in_block();
   const cd *src = A + (size_t)b * mstride;
   for (int e = threadIdx.x; e < N * N; e += 256) Ms[e] = src[e];
   __syncthreads();
-  if (threadIdx.x < N) {
-    double lo = INFINITY, hi = 0.0;
-    for (int j = 0; j < N; ++j) {
-      const cd v = Ms[threadIdx.x * N + j];
-      const double a = fma(v.re, v.re, v.im * v.im);
-      lo = fmin(lo, a);
-      hi = fmax(hi, a);
-    }
-    rmin[threadIdx.x] = lo;
-    rmax[threadIdx.x] = hi;
-  }
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    int best = 0;
-    double mx = 0.0;
-    for (int i = 0; i < N; ++i) {
-      if (rmin[i] > rmin[best]) best = i;
-      mx = fmax(mx, rmax[i]);
-    }
-    const bool ok = mx > 0.0 && mx <= 1.7976931348623157e308 && rmin[best] >= kPairMinRel2 * mx;
-    pick = ok ? best : -1;
-    if (wg == 0) handled[b] = ok ? 1 : 0;
-  }
-  __syncthreads();
-  const int r = pick;
+  const int r = pair_row<N>(Ms, rmin, rmax);
+  if (wg == 0 && threadIdx.x == 0) handled[b] = r < 0 ? 0 : 1;
   if (r < 0) return;  // uniform over the workgroup
-  if (r != 0 && threadIdx.x < N) {
-    const cd t = Ms[threadIdx.x];
-    Ms[threadIdx.x] = Ms[r * N + threadIdx.x];
-    Ms[r * N + threadIdx.x] = t;
-  }
+  if (threadIdx.x < 64) pair_divisors<N>(Ms, r, inv0, &Km, &Ke);
   __syncthreads();
-  if (threadIdx.x < N) inv0[threadIdx.x] = cinv_scaled(Ms[threadIdx.x]);
-  if (threadIdx.x == 64) {
-    cd k;
-    int ke;
-    prod_half_scaled(Ms, N, k, ke);
-    Km = k;
-    Ke = ke;
-  }
-  __syncthreads();
-  for (int e = threadIdx.x; e < (N - 1) * N; e += 256) {
-    const int i = 1 + e / N, j = e - (i - 1) * N;
-    const cd v = cmul(Ms[i * N + j], inv0[j]);
-    Sf[i * N + j] = {(float)(2.0 * v.re), (float)(2.0 * v.im)};
+  for (int e = N + threadIdx.x; e < N * N; e += 256) {
+    const cd v = cmul(Ms[e], inv0[e % N]);
+    Sf[e] = {(float)(2.0 * v.re), (float)(2.0 * v.im)};
   }
   __syncthreads();
   double are = 0.0, aim = 0.0;
   glynn_pair_lane_f32<N, U, SR, S2P>(Sf, C - 1, (uint64_t)wq * 64 + lane, (uint64_t)wpm * 64, iters, are, aim);
   are = wave_sum(are);
   aim = wave_sum(aim);
-  if (lane == 0) {
-    const cd k = Km;
-    partial[(size_t)b * wpm + wq] = {ldexp(k.re * are - k.im * aim, Ke),
-                                     ldexp(k.re * aim + k.im * are, Ke)};
-  }
+  const cd k = Km;
+  glynn_store(ldexp(k.re * are - k.im * aim, Ke), ldexp(k.re * aim + k.im * are, Ke), b, wq, wpm,
+              sums, partial, out);
 }
 
 // One row of a matrix in LDS in broadcast form, each 16-lane row of the wave from its own M.
@@ -951,17 +965,6 @@ __global__ void copy_scalar_kernel(const cd *A, int64_t mstride, int batch, cd *
   if (b < batch) out[b] = A[(size_t)b * mstride];
 }
 
-// FP32 copy of the matrices (row store for the FP32 column-sum variant).
-__global__ void to_fp32_kernel(const cd *A, int64_t mstride, int n, int batch, float *dst) {
-  const int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const int64_t per = (int64_t)n * n;
-  if (idx >= per * batch) return;
-  const int64_t b = idx / per, e = idx - b * per;
-  const cd v = A[b * mstride + e];
-  dst[2 * idx] = (float)v.re;
-  dst[2 * idx + 1] = (float)v.im;
-}
-
 }  // namespace
 
 }  // namespace tb
@@ -1036,7 +1039,7 @@ inline int glynn_u_max(int n) {
 
 constexpr int kWideMinN = 14;  // below this the SMALL kernel
 
-// FP64 sizes that run the paired walk first (the plain WIDE kernel then takes the
+// FP64 sizes that run the paired walk (matrices it cannot take walk plainly in the same
 // matrices it left): from where a chunk holds the static block plus one bit up to the
 // largest n that fits 256 VGPRs without spills (n = 40 spills).
 #ifndef TB_GLYNN_PAIR_MIN_N
@@ -1072,7 +1075,7 @@ constexpr int glynn_pair_u_of() {
   return sizeof(F) == 8 ? glynn_pair_u<N>() : TB_GLYNN_F32_PAIR_U;
 }
 // Values of row 2 the paired FP32 kernel also keeps in SGPRs, so that it fits 4 waves
-// per SIMD (<= 128 VGPRs): about 6n + 17 VGPRs without them, 2 fewer per value; up to 11
+// per SIMD (<= 128 VGPRs): about 6n + 15 VGPRs without them, 2 fewer per value; up to 11
 // values (row 1 takes 2n SGPRs; n = 23 would need 14 and exceed the 102 SGPRs).
 #ifndef TB_GLYNN_F32_PAIR_S2_MAX
 #define TB_GLYNN_F32_PAIR_S2_MAX 11
@@ -1080,20 +1083,26 @@ constexpr int glynn_pair_u_of() {
 template <int N>
 constexpr int glynn_f32_pair_s2() {
   if (TB_GLYNN_F32_PAIR_SR != 1 || TB_GLYNN_F32_PAIR_U < 2) return 0;
-  constexpr int over = 6 * N + 17 - 128;
+  constexpr int over = 6 * N + 15 - 128;
   constexpr int need = over <= 0 ? 0 : (over + 1) / 2 + 1;  // one value of margin
   return (over <= 0 || need > TB_GLYNN_F32_PAIR_S2_MAX) ? 0 : need;
 }
-// Waves per SIMD the launch is resident at (the plan's round size).
+// Waves per SIMD the launch is resident at.
 template <int N, typename F>
 constexpr int glynn_wave_slots() {
   if constexpr (sizeof(F) == 4 && glynn_paired<N, F>()) {
     if constexpr (TB_GLYNN_F32_PAIR_SR == 1)
-      return (6 * N + 17 <= 128 || glynn_f32_pair_s2<N>() > 0) ? 4 : TB_GLYNN_F32_PAIR_WPE;
+      return (6 * N + 15 <= 128 || glynn_f32_pair_s2<N>() > 0) ? 4 : TB_GLYNN_F32_PAIR_WPE;
     if constexpr (TB_GLYNN_F32_PAIR_SR == 2) return 4;
     return TB_GLYNN_F32_PAIR_WPE;
   }
   return 2;
+}
+// Waves per SIMD of the plan's bound on C: the residency, but 3 at n = 22, which with 4 takes
+// C = 6 instead of 7 for 100 matrices (547 us instead of 482).
+template <int N, typename F>
+constexpr int glynn_plan_slots() {
+  return N == 22 ? std::min(glynn_wave_slots<N, F>(), 3) : glynn_wave_slots<N, F>();
 }
 template <int N, typename F>
 constexpr int glynn_min_c() {
@@ -1109,61 +1118,65 @@ struct GlynnPlan {
   int C, wpm, iters;
 };
 
-// WIDE plan: chunks of 2^C ranks. Built in: C shrinks (down to 7) until the batch
-// provides at least ~8192 waves (4 rounds of 2 waves on every SIMD), so small batches of
-// mid-size matrices still fill the GPU; C <= 12 bounds a lane's walk between re-seeds.
-// A tuned C (c_pref > 0) replaces that choice. Always: C >= U and a matrix gets at
-// least 4 waves (one workgroup). Re-seeding costs n^2 per 2^C steps.
-// Kernels resident at more than 2 waves per SIMD (wave_slots) compare the built-in C with
-// C - 1 and C - 2: the waves run in rounds of wave_slots x 1024 SIMDs (256 CUs), and a
-// smaller chunk can fill the last round better (16384 waves are 5.33 rounds of 3072 but
-// 10.67 rounds at twice the waves), against twice the re-seeding per code.
+// WIDE plan: chunks of 2^C ranks, one per lane.
+//
+// Upper bound: the sums drift with the length of a chunk (FP32 sums at n = 20 are off by 5e-6
+// with C = 8 and 1.1e-5 with C = 10), so C is at most what gives the batch ~8192 waves, or 7,
+// moved by up to two towards fuller rounds of waves: kernels resident at more than 2 waves per
+// SIMD (wave_slots) compare it with C - 1 and C - 2, FP64 ones with C + 1 and C + 2 (grow), by
+// how full the last round of wave_slots x 1024 waves is, times the share of a chunk left after
+// seeding ((n - 2) 2 / (5 2^C) of its instructions). Ties keep the candidate tried first.
+//
+// Below that bound the plan takes the C with the least ceil(waves / 1024) (2^C + 1.1 n): a
+// launch lasts as long as the SIMD with the most waves, and a wave costs its chunk and a fixed
+// part (staging the matrix, the quotients, seeding the sums) worth about 1.1 n ranks. One FP64
+// wave alone on a SIMD issues 2% slower than two, one FP32 wave at half the rate (dual issue
+// takes two). FP64, C = 4, 5, 6, 7, 8 and the rule's choice, with the bound taken before:
+//   one matrix of n = 20      15.2   16.5   21.5   33.5   57.1 us    4   (C = 7)
+//   16 of n = 20                67     48     39     36     56       7   (C = 7)
+//   16 of n = 22               249    178    146    132    125       8   (C = 8)
+// and FP32, 16 of n = 22: 178, 129, 100, 94 us, choice 7.
+//
+// A tuned C (c_pref > 0) replaces the choice. Always: U <= C <= 12 and a matrix gets at least 4
+// waves (one workgroup).
 constexpr int kPlanSimds = 1024;
 inline int glynn_plan_clamp(int C, int nb, int u) {
   return std::min(std::max(std::min(C, kMaxC), u), nb - 8);
 }
-// grow: how many chunk sizes above the ~8192-wave choice a 2-wave kernel may try (the
-// FP64 kernels: 2; the FP32 ones keep their chunks, whose length bounds how far their FP32
-// column sums drift between re-seeds).
 inline GlynnPlan glynn_plan(int n, int batch, int c_pref, int u = 2, int wave_slots = 2,
                             int grow = 0) {
   GlynnPlan p{};
   const int nb = n - 1;
+  const auto waves = [&](int c) { return (double)batch * std::ldexp(1.0, nb - c - 6); };
   int C;
   if (c_pref > 0) {
-    C = c_pref;
+    C = glynn_plan_clamp(c_pref, nb, u);
   } else {
     int want_bits = 0;  // log2(waves per matrix needed for ~8192 waves in total)
     while (((int64_t)batch << want_bits) < 8192 && want_bits < 30) ++want_bits;
-    C = nb - 6 - want_bits;
-    C = std::max(C, std::min(7, nb - 8));
-  }
-  C = glynn_plan_clamp(C, nb, u);
-  if (c_pref <= 0 && (wave_slots > 2 || grow > 0)) {
-    // Score chunk sizes near C by how full their last round of wave_slots x kPlanSimds
-    // waves is, times the share of a chunk left after seeding its column sums
-    // ((n - 2) 2 / (5 2^c) of its instructions). Kernels of 3-4 waves per SIMD try
-    // smaller chunks (more waves to fill their rounds); the FP64 kernels (2 waves) try up
-    // to `grow` larger ones (less seeding while the rounds stay full: 2-10% faster for
-    // batches of up to a few hundred matrices at n = 18..26, never slower in the batches
-    // measured). Ties keep the candidate tried first.
-    const int step = wave_slots > 2 ? -1 : 1;
-    const int count = wave_slots > 2 ? 3 : 1 + grow;
+    C = glynn_plan_clamp(std::max(nb - 6 - want_bits, std::min(7, nb - 8)), nb, u);
+    const int step = wave_slots > 2 ? -1 : 1, count = wave_slots > 2 ? 3 : 1 + grow;
     double best = -1.0;
-    int best_c = C;
-    for (int k = 0, c = C; k < count; ++k, c += step) {
+    for (int k = 0, c = C, c0 = C; k < count; ++k, c = c0 + k * step) {
       if (glynn_plan_clamp(c, nb, u) != c) continue;
-      const double waves = (double)batch * std::ldexp(1.0, nb - c - 6);
-      const double rounds = waves / ((double)kPlanSimds * wave_slots);
-      const double fill = rounds / std::ceil(rounds);
+      const double rounds = waves(c) / ((double)kPlanSimds * wave_slots);
       const double seed = (double)(n - 2) * 2.0 / (5.0 * std::ldexp(1.0, c));
-      const double score = fill * (1.0 - seed);
+      const double score = rounds / std::ceil(rounds) * (1.0 - seed);
       if (score > best + 1e-9) {
         best = score;
-        best_c = c;
+        C = c;
       }
     }
-    C = best_c;
+    const double alone = grow > 0 ? 1.02 : 2.0;
+    double least = INFINITY;
+    for (int c = C, low = glynn_plan_clamp(0, nb, u); c >= low; --c) {
+      const double cost =
+          std::max(std::ceil(waves(c) / kPlanSimds), alone) * (std::ldexp(1.0, c) + 1.1 * n);
+      if (cost < least) {
+        least = cost;
+        C = c;
+      }
+    }
   }
   p.C = C;
   const int wave_bits = nb - p.C - 6;  // log2(waves needed at one chunk per lane), >= 2
@@ -1194,61 +1207,48 @@ inline int glynn_small_plan(int n, int batch, int c_pref, int u, size_t elem) {
   return C;
 }
 
-// A: the matrices in the kernel's precision; A64 / mstride64: the same matrices in FP64
-// (the paired FP32 kernel forms its quotients from them).
 // wpm_cap: partials per matrix the workspace holds; a plan that needs more fails with
 // TB_EWORKSPACE instead of writing past them.
 template <int N, typename F>
-inline int32_t launch_glynn_n(const tb::cpx<F> *A, int64_t mstride, const tb::cd *A64,
-                              int64_t mstride64, int batch, tb::cd *out, tb::cd *partial,
-                              int *handled, int wpm_cap, int c_pref, hipStream_t s) {
+inline int32_t launch_glynn_n(const tb::cd *A, int64_t mstride, int batch, tb::cd *out,
+                              tb::cd *partial, int *handled, int wpm_cap, int c_pref,
+                              hipStream_t s) {
   if constexpr (N < kWideMinN) {
     constexpr int U = (N - 1) < 2 ? (N - 1) : 2;
     const int C = glynn_small_plan(N, batch, c_pref, U, sizeof(tb::cpx<F>));
     const int mats = 256 >> (N - 1 - C);
     hipLaunchKernelGGL((tb::glynn_small_kernel<N, U, F>), dim3((batch + mats - 1) / mats), dim3(256),
-                       glynn_small_lds(N, C, sizeof(tb::cpx<F>)), s, A64, mstride64, batch, C, out);
-    (void)A;
-    (void)mstride;
+                       glynn_small_lds(N, C, sizeof(tb::cpx<F>)), s, A, mstride, batch, C, out);
     (void)partial;
     (void)handled;
     (void)wpm_cap;
     return tbh::check_hip(hipGetLastError(), "glynn_small_kernel");
   } else {
-    constexpr int U = glynn_u<N, F>();
+    constexpr int U = glynn_u<N, F>(), R0 = glynn_reg_rows<N, F>();
     constexpr int CMIN = glynn_min_c<N, F>();
+    constexpr bool paired = glynn_paired<N, F>(), fp32 = sizeof(F) == 4;
     static_assert(CMIN <= N - 9, "the static block must fit the smallest chunk (C <= n - 9)");
-    const GlynnPlan p =
-        glynn_plan(N, batch, c_pref, CMIN, glynn_wave_slots<N, F>(), sizeof(F) == 8 ? 2 : 0);
+    const GlynnPlan p = glynn_plan(N, batch, c_pref, CMIN, glynn_plan_slots<N, F>(), fp32 ? 0 : 2);
     if (p.wpm > wpm_cap)
       return tbh::fail(TB_EWORKSPACE,
                        "glynn: the plan for n=%d batch=%d needs %d partials per matrix, the "
                        "workspace holds %d", N, batch, p.wpm, wpm_cap);
-    const unsigned blocks = (unsigned)batch * (unsigned)(p.wpm / 4);
-    const int *skip = nullptr;
-    if constexpr (glynn_paired<N, F>()) {
-      if constexpr (sizeof(F) == 8)
-        hipLaunchKernelGGL((tb::glynn_pair_kernel<N, glynn_pair_u<N>(), glynn_pair_b<N>()>),
-                           dim3(blocks), dim3(256), 0, s, (const tb::cpx<double> *)A64, mstride64,
-                           p.C, p.wpm, p.iters, partial, handled);
-      else
-        hipLaunchKernelGGL((tb::glynn_pair_kernel_f32<N, TB_GLYNN_F32_PAIR_U, TB_GLYNN_F32_PAIR_SR,
-                                                      glynn_f32_pair_s2<N>(),
-                                                      glynn_wave_slots<N, F>()>),
-                           dim3(blocks), dim3(256),
-                           0, s, A64, mstride64, p.C, p.wpm, p.iters, partial, handled);
-      int32_t rc = tbh::check_hip(hipGetLastError(), "glynn_pair_kernel");
-      if (rc) return rc;
-      skip = handled;
-    } else {
-      (void)handled;
-      (void)A64;
-      (void)mstride64;
+    const dim3 blocks((unsigned)batch * (unsigned)(p.wpm / 4));
+    if constexpr (paired && fp32) {
+      hipLaunchKernelGGL((tb::glynn_pair_kernel_f32<N, TB_GLYNN_F32_PAIR_U, TB_GLYNN_F32_PAIR_SR,
+                                                    glynn_f32_pair_s2<N>(), glynn_wave_slots<N, F>()>),
+                         blocks, dim3(256), 0, s, A, mstride, p.C, p.wpm, p.iters, partial, handled,
+                         out);
+      if (const int32_t rc = tbh::check_hip(hipGetLastError(), "glynn_pair_kernel_f32")) return rc;
     }
-    hipLaunchKernelGGL((tb::glynn_wide_kernel<N, U, glynn_reg_rows<N, F>(), F>), dim3(blocks), dim3(256), 0, s,
-                       A, mstride, p.C, p.wpm, p.iters, partial, skip);
-    int32_t rc = tbh::check_hip(hipGetLastError(), "glynn_wide_kernel");
-    if (rc) return rc;
+    if constexpr (paired && !fp32)
+      hipLaunchKernelGGL((tb::glynn_pair_kernel<N, glynn_pair_u<N>(), glynn_pair_b<N>(), U, R0>),
+                         blocks, dim3(256), 0, s, A, mstride, p.C, p.wpm, p.iters, partial, out);
+    else
+      hipLaunchKernelGGL((tb::glynn_wide_kernel<N, U, R0, F>), blocks, dim3(256), 0, s, A, mstride,
+                         p.C, p.wpm, p.iters, partial, paired ? handled : nullptr, out);
+    const int32_t rc = tbh::check_hip(hipGetLastError(), "glynn walk");
+    if (rc || p.wpm == 4) return rc;
     hipLaunchKernelGGL(tb::glynn_finish_kernel, dim3((batch + 3) / 4), dim3(256), 0, s, partial,
                        p.wpm, batch, out);
     return tbh::check_hip(hipGetLastError(), "glynn_finish_kernel");
@@ -1256,27 +1256,23 @@ inline int32_t launch_glynn_n(const tb::cpx<F> *A, int64_t mstride, const tb::cd
 }
 
 template <typename F, int N = 2>
-inline int32_t dispatch_glynn(int n, const tb::cpx<F> *A, int64_t mstride, const tb::cd *A64,
-                              int64_t mstride64, int batch, tb::cd *out, tb::cd *partial,
-                              int *handled, int wpm_cap, int c_pref, hipStream_t s) {
+inline int32_t dispatch_glynn(int n, const tb::cd *A, int64_t mstride, int batch, tb::cd *out,
+                              tb::cd *partial, int *handled, int wpm_cap, int c_pref,
+                              hipStream_t s) {
   if constexpr (N > TB_GLYNN_MAX_N) {
     return tbh::fail(TB_ERANGE, "glynn: n=%d exceeds TB_GLYNN_MAX_N=%d", n, TB_GLYNN_MAX_N);
   } else {
     if (n == N)
-      return launch_glynn_n<N, F>(A, mstride, A64, mstride64, batch, out, partial, handled,
-                                  wpm_cap, c_pref, s);
-    return dispatch_glynn<F, N + 1>(n, A, mstride, A64, mstride64, batch, out, partial, handled,
-                                    wpm_cap, c_pref, s);
+      return launch_glynn_n<N, F>(A, mstride, batch, out, partial, handled, wpm_cap, c_pref, s);
+    return dispatch_glynn<F, N + 1>(n, A, mstride, batch, out, partial, handled, wpm_cap, c_pref, s);
   }
 }
 
-// `handled`: batch ints of workspace for the paired walks; `wpm_cap`: partials per matrix
-// after them. The FP32 dispatch takes the FP32 copy (A) and the FP64 originals (A64).
-int32_t glynn_dispatch_f64(int n, const tb::cpx<double> *A, int64_t mstride, int batch,
-                           tb::cd *out, tb::cd *partial, int *handled, int wpm_cap, int c_pref,
-                           hipStream_t s);
-int32_t glynn_dispatch_f32(int n, const tb::cpx<float> *A, int64_t mstride, const tb::cd *A64,
-                           int64_t mstride64, int batch, tb::cd *out, tb::cd *partial,
-                           int *handled, int wpm_cap, int c_pref, hipStream_t s);
+// `handled`: batch ints of workspace for the paired FP32 walk; `wpm_cap`: partials per matrix
+// after them. Both take the FP64 matrices.
+int32_t glynn_dispatch_f64(int n, const tb::cd *A, int64_t mstride, int batch, tb::cd *out,
+                           tb::cd *partial, int *handled, int wpm_cap, int c_pref, hipStream_t s);
+int32_t glynn_dispatch_f32(int n, const tb::cd *A, int64_t mstride, int batch, tb::cd *out,
+                           tb::cd *partial, int *handled, int wpm_cap, int c_pref, hipStream_t s);
 
 }  // namespace tbgl
