@@ -93,6 +93,8 @@ def sweep_builtin(k: int, items: int) -> int:
     while (max(items, 1) << want) < 4096 and want < 30:
         want += 1
     c = max(min(11, nb - 6 - want), min(5, nb - 6))
+    while 3 < c < nb - 6 and nb - c - 5 <= 8 and max(items, 1) << (nb - c - 5) <= 1024:
+        c -= 1
     return min(max(c, min(3, nb)), nb, 16)
 
 

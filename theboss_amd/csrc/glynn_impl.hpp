@@ -1039,8 +1039,8 @@ inline int glynn_u_max(int n) {
 
 constexpr int kWideMinN = 14;  // below this the SMALL kernel
 
-// FP64 sizes that run the paired walk (matrices it cannot take walk plainly in the same
-// matrices it left): from where a chunk holds the static block plus one bit up to the
+// Sizes that run the paired walk (FP64: matrices it cannot take walk plainly in the same
+// kernel; FP32: in a second one): from where a chunk holds the static block plus one bit up to the
 // largest n that fits 256 VGPRs without spills (n = 40 spills).
 #ifndef TB_GLYNN_PAIR_MIN_N
 #define TB_GLYNN_PAIR_MIN_N 14

@@ -52,9 +52,26 @@ __device__ __forceinline__ void sweep_stage(const SweepSource &src, int item, cd
   }
 }
 
+// The tasks of a workgroup. Workgroups go round-robin over the XCDs; an XCD takes consecutive
+// tasks, as many as its share of the workgroups, so with a workgroup for every task each has
+// one (an eighth of the tasks, rounded up, gave some workgroups two and others none where 8 does
+// not divide them: 500 k = 12 items in 500 workgroups 11.6 us instead of 19.7).
+struct SweepTasks {
+  int64_t first, end;
+  int step;
+  __device__ __forceinline__ explicit SweepTasks(int64_t total) {
+    constexpr int kXcd = 8;
+    const int G = gridDim.x, x = blockIdx.x % kXcd;
+    const int before = x * (G / kXcd) + min(x, G % kXcd);  // workgroups of the XCDs before
+    step = G / kXcd + (x < G % kXcd ? 1 : 0);
+    first = total * before / G + blockIdx.x / kXcd;
+    end = total * (before + step) / G;
+  }
+};
+
 // Persistent grid: G one-wave blocks loop over the tasks (slot, w), slot < active
 // items, w < wpi. Blocks are dispatched round-robin over the 8 XCDs (each with its own
-// L2); XCD x takes the contiguous task range [x T/8, (x+1) T/8) so that the waves of one
+// L2); each XCD takes a contiguous task range (SweepTasks) so that the waves of one
 // item run on one XCD and its columns are fetched into one L2 only. The active item
 // count may come from device memory, so a captured graph launches the same grid for
 // any number of active items and idle tasks cost nothing.
@@ -70,15 +87,8 @@ __global__ __launch_bounds__(64) TB_SWEEP_ATTR(K) void sweep_kernel(
   const int lane = threadIdx.x;
   int nitems = items;
   if (item_count) nitems = min(items, *item_count);
-  constexpr int kXcd = 8;
-  const int G = gridDim.x, p = blockIdx.x;
-  const int x = p % kXcd, bi = p / kXcd;
-  const int nblk_x = G / kXcd + (x < G % kXcd ? 1 : 0);
-  const int64_t total = (int64_t)nitems * wpi;
-  const int64_t per_x = (total + kXcd - 1) / kXcd;
-  const int64_t lo = (int64_t)x * per_x;
-  const int64_t hi = min(total, lo + per_x);
-  for (int64_t task = lo + bi; task < hi; task += nblk_x) {
+  const SweepTasks own((int64_t)nitems * wpi);
+  for (int64_t task = own.first; task < own.end; task += own.step) {
     const int slot = (int)(task / wpi);
     const int w = (int)(task - (int64_t)slot * wpi);
     __syncthreads();  // previous task's reads of Vs are done
@@ -117,15 +127,8 @@ __global__ __launch_bounds__(64) TB_SWEEP_PAIR_ATTR(K) void sweep_pair_kernel(
   const int lane = threadIdx.x;
   int nitems = items;
   if (item_count) nitems = min(items, *item_count);
-  constexpr int kXcd = 8;
-  const int G = gridDim.x, p = blockIdx.x;
-  const int x = p % kXcd, bi = p / kXcd;
-  const int nblk_x = G / kXcd + (x < G % kXcd ? 1 : 0);
-  const int64_t total = (int64_t)nitems * wpi;
-  const int64_t per_x = (total + kXcd - 1) / kXcd;
-  const int64_t lo = (int64_t)x * per_x;
-  const int64_t hi = min(total, lo + per_x);
-  for (int64_t task = lo + bi; task < hi; task += nblk_x) {
+  const SweepTasks own((int64_t)nitems * wpi);
+  for (int64_t task = own.first; task < own.end; task += own.step) {
     const int slot = (int)(task / wpi);
     const int w = (int)(task - (int64_t)slot * wpi);
     __syncthreads();  // previous task's reads of LDS are done
@@ -288,7 +291,11 @@ constexpr int64_t kSweepWaveTarget = 4096;
 // Built-in chunk: the longest walk (at most 2^11 Gray steps per lane) that still gives the
 // launch kSweepWaveTarget waves, but not below 2^5 steps. A batch of 4096 k = 20 items
 // keeps 2^11 (4 waves per item); one k = 20 item gets 2^5 (256 waves) instead of a
-// 4-wave launch. The tuner may choose otherwise per (k, batch bucket).
+// 4-wave launch. A launch that would leave SIMDs idle all the same goes on down to 2^3 steps,
+// up to 1024 waves and 256 partials per item to add (us at 2^5, 2^4, 2^3: one k = 14 item 17.5,
+// 15.5, 15.0; one k = 18 item 23.4, 21.3, 20.1; 16 k = 16 items 20.8, 19.7, 17.2; past the lines
+// 100 k = 16 items 28, 41, 52 and one k = 20 item 28.5, 28.1, 30.4), unless one wave is an item. The tuner may choose
+// otherwise per (k, batch bucket).
 inline SweepPlan sweep_plan(int k, int64_t items, int c_override) {
   SweepPlan p{};
   const int nb = k - 1;                      // Gray bits (particle 0 is fixed)
@@ -302,6 +309,8 @@ inline SweepPlan sweep_plan(int k, int64_t items, int c_override) {
       ++want_bits;
     c = std::min(TB_SWEEP_BUILTIN_MAX_C, nb - 6 - want_bits);
     c = std::max(c, std::min(TB_SWEEP_BUILTIN_MIN_C, nb - 6));
+    const auto wpi = [&](int bits) { return (int64_t)1 << std::max(0, nb - bits - 6); };
+    while (c > u && wpi(c) > 1 && wpi(c - 1) <= 256 && items * wpi(c - 1) <= 1024) --c;
   }
   c = std::max(c, u);
   c = std::min(c, std::min(nb, tb::kSweepMaxC));
@@ -412,9 +421,12 @@ constexpr int kReduceInOrder = 32;
 int32_t run_sweep(int k, const tb::SweepSource &src, int items, int c_override, tb::cd *partial,
                   const int *in_mult, int in_max, tb::cd *minors, hipStream_t s) {
   const SweepPlan p = sweep_plan(k, items, c_override);
-  int32_t rc = dispatch_sweep(k, src, nullptr, nullptr, items, p, partial, s);
-  if (rc) return rc;
   const int outs = in_mult ? in_max : k;
+  // One wave per item and no empty slot: the sums are the minors, with nothing to add or place
+  // (one launch of two saved: 14.6 us a call instead of 17.4 up to k = 12).
+  const bool direct = p.wpi == 1 && outs == k;
+  int32_t rc = dispatch_sweep(k, src, nullptr, nullptr, items, p, direct ? minors : partial, s);
+  if (rc || direct) return rc;
   if (p.wpi > kReduceInOrder) {
     hipLaunchKernelGGL(tb::sweep_reduce_wide_kernel, dim3(items), dim3(256), 0, s, partial, k, p.wpi,
                        in_mult, outs, minors);
