@@ -345,6 +345,61 @@ __device__ __forceinline__ double vgpr_one() {
   return one;
 }
 
+// Two wait states between whatever wrote a broadcast-form row's registers and its DPP reads.
+template <int N>
+__device__ __forceinline__ void bcast_settle(Bcast<N> &b) {
+#pragma unroll
+  for (int p = 0; p < Bcast<N>::P; ++p) asm volatile("s_nop 1" : "+v"(b.v[p]));
+}
+
+// The half sums at the start of a chunk of 2^c ranks, h = (fixed + sum_b d_b row_b) / 2 with
+// d_b = -1 where bit b of g0 is set, row b at rows + 2 N b, for lanes on consecutive chunks:
+// only bits c - 1 .. c + 5 differ between the lanes of a wave. The rows of the other bits are
+// added up once per wave, each lane keeping the components it holds in broadcast form, and the
+// sum and the seven others enter every lane's sums from there by DPP: at n = 20, 16 N FMAs and
+// 3 reads per row instead of 2 N FMAs and N 16-byte reads for each of 19 rows. That took the
+// fixed cost of a wave of the k = 20 sweep from about 38 codes to 20 (one item 28.7 -> 18.8 us,
+// 16 items 67 -> 47), of a Glynn wave at n = 20 from 22 to 17 (20 matrices 53 -> 48 us). Reading
+// the seven rows ahead of their use gains nothing more, and FP32 sums, which issue two FMAs in
+// the time of one of these, are 1-20% slower this way.
+template <int N>
+__device__ __forceinline__ void seed_half_sums(double (&hr)[N], double (&hi)[N], const double *fixed,
+                                               const double *rows, int bits, int c, uint64_t g0) {
+  constexpr int P = Bcast<N>::P;
+  int lane = threadIdx.x;
+  asm volatile("" : "+v"(lane));  // the slots are worked out here, not kept from chunk to chunk
+  const uint64_t g = (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)g0) |
+                     (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(g0 >> 32)) << 32;
+  int at[P];
+#pragma unroll
+  for (int p = 0; p < P; ++p) at[p] = min(16 * p + (lane & 15), 2 * N - 1);
+  Bcast<N> sum;
+#pragma unroll
+  for (int p = 0; p < P; ++p) sum.v[p] = 0.5 * fixed[at[p]];
+  const int lo = max(c - 1, 0), end = min(c + 6, bits);
+  const auto add = [&](int b) {
+    const double d = ((g >> b) & 1ull) ? -0.5 : 0.5;
+#pragma unroll
+    for (int p = 0; p < P; ++p) sum.v[p] = fma(d, rows[2 * N * b + at[p]], sum.v[p]);
+  };
+#pragma unroll 2
+  for (int b = 0; b < lo; ++b) add(b);
+#pragma unroll 2
+  for (int b = end; b < bits; ++b) add(b);
+#pragma unroll
+  for (int j = 0; j < N; ++j) hr[j] = hi[j] = 0.0;
+  bcast_settle(sum);
+  flip_bcast<0, N, 1>(hr, hi, sum, vgpr_one());
+#pragma unroll 1
+  for (int b = lo; b < end; ++b) {
+    Bcast<N> row;
+#pragma unroll
+    for (int p = 0; p < P; ++p) row.v[p] = rows[2 * N * b + at[p]];
+    bcast_settle(row);
+    flip_bcast<0, N, 0>(hr, hi, row, ((g0 >> b) & 1ull) ? -0.5 : 0.5);
+  }
+}
+
 // Largest of one value per lane, in every lane.
 __device__ __forceinline__ double wave_allmax(double v) {
   const uint64_t u = __builtin_bit_cast(uint64_t, v);

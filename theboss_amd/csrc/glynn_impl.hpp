@@ -122,26 +122,30 @@ __device__ __forceinline__ void glynn_lane(P M, int C, uint64_t q0, uint64_t qst
     const uint64_t t0 = q << C;
     const uint64_t g0 = t0 ^ (t0 >> 1);
     F hr[N], hi[N];
-#pragma unroll
-    for (int j = 0; j < N; ++j) {
-      const cpx<F> v = M[(size_t)(N - 1) * N + j];
-      hr[j] = v.re;
-      hi[j] = v.im;
-    }
-#pragma unroll 1
-    for (int i = 0; i < NB; ++i) {
-      const F sg = ((g0 >> i) & 1ull) ? F(-1) : F(1);
+    if constexpr (B > 0) {
+      seed_half_sums<N>(hr, hi, (const double *)(M + (size_t)(N - 1) * N), (const double *)M, NB, C, g0);
+    } else {
 #pragma unroll
       for (int j = 0; j < N; ++j) {
-        const cpx<F> v = M[(size_t)i * N + j];
-        hr[j] = fma(sg, v.re, hr[j]);
-        hi[j] = fma(sg, v.im, hi[j]);
+        const cpx<F> v = M[(size_t)(N - 1) * N + j];
+        hr[j] = v.re;
+        hi[j] = v.im;
       }
-    }
+#pragma unroll 1
+      for (int i = 0; i < NB; ++i) {
+        const F sg = ((g0 >> i) & 1ull) ? F(-1) : F(1);
 #pragma unroll
-    for (int j = 0; j < N; ++j) {
-      hr[j] *= F(0.5);
-      hi[j] *= F(0.5);
+        for (int j = 0; j < N; ++j) {
+          const cpx<F> v = M[(size_t)i * N + j];
+          hr[j] = fma(sg, v.re, hr[j]);
+          hi[j] = fma(sg, v.im, hi[j]);
+        }
+      }
+#pragma unroll
+      for (int j = 0; j < N; ++j) {
+        hr[j] *= F(0.5);
+        hi[j] *= F(0.5);
+      }
     }
     const bool q_odd = (q & 1ull) != 0;
     double cre, cim;
@@ -346,27 +350,8 @@ __device__ __forceinline__ void glynn_pair_lane(const cpx<double> *S2, int C, ui
     const uint64_t t0 = q << C;
     const uint64_t g0 = t0 ^ (t0 >> 1);
     double ur[N], ui[N];
-#pragma unroll
-    for (int j = 0; j < N; ++j) {
-      const cpx<double> v = S2[(size_t)(N - 1) * N + j];
-      ur[j] = v.re;
-      ui[j] = v.im;
-    }
-#pragma unroll 1
-    for (int i = 0; i < NB; ++i) {
-      const double sg = ((g0 >> i) & 1ull) ? -1.0 : 1.0;
-#pragma unroll
-      for (int j = 0; j < N; ++j) {
-        const cpx<double> v = S2[(size_t)(i + 1) * N + j];
-        ur[j] = fma(sg, v.re, ur[j]);
-        ui[j] = fma(sg, v.im, ui[j]);
-      }
-    }
-#pragma unroll
-    for (int j = 0; j < N; ++j) {
-      ur[j] *= 0.5;
-      ui[j] *= 0.5;
-    }
+    seed_half_sums<N>(ur, ui, (const double *)(S2 + (size_t)(N - 1) * N), (const double *)(S2 + N), NB,
+                      C, g0);
     const bool q_odd = (q & 1ull) != 0;
     double cre = 0.0, cim = 0.0;
     pair_acc<1>(cre, cim, ur, ui);
@@ -1129,7 +1114,8 @@ struct GlynnPlan {
 //
 // Below that bound the plan takes the C with the least ceil(waves / 1024) (2^C + 1.1 n): a
 // launch lasts as long as the SIMD with the most waves, and a wave costs its chunk and a fixed
-// part (staging the matrix, the quotients, seeding the sums) worth about 1.1 n ranks. One FP64
+// part (staging the matrix, the quotients, seeding the sums) worth about 1.1 n ranks (0.85 n with
+// the FP64 seeds of seed_half_sums, which moves no choice below). One FP64
 // wave alone on a SIMD issues 2% slower than two, one FP32 wave at half the rate (dual issue
 // takes two). FP64, C = 4, 5, 6, 7, 8 and the rule's choice, with the bound taken before:
 //   one matrix of n = 20      15.2   16.5   21.5   33.5   57.1 us    4   (C = 7)

@@ -292,9 +292,10 @@ constexpr int64_t kSweepWaveTarget = 4096;
 // launch kSweepWaveTarget waves, but not below 2^5 steps. A batch of 4096 k = 20 items
 // keeps 2^11 (4 waves per item); one k = 20 item gets 2^5 (256 waves) instead of a
 // 4-wave launch. A launch that would leave SIMDs idle all the same goes on down to 2^3 steps,
-// up to 1024 waves and 256 partials per item to add (us at 2^5, 2^4, 2^3: one k = 14 item 17.5,
-// 15.5, 15.0; one k = 18 item 23.4, 21.3, 20.1; 16 k = 16 items 20.8, 19.7, 17.2; past the lines
-// 100 k = 16 items 28, 41, 52 and one k = 20 item 28.5, 28.1, 30.4), unless one wave is an item. The tuner may choose
+// up to 1024 waves and 256 partials per item to add (us at 2^5, 2^4, 2^3, with the seeds as they
+// were: one k = 14 item 17.5, 15.5, 15.0; one k = 18 item 23.4, 21.3, 20.1; 16 k = 16 items 20.8,
+// 19.7, 17.2; past the lines 100 k = 16 items 28, 41, 52 and one k = 20 item 28.5, 28.1, 30.4),
+// unless one wave is an item. The tuner may choose
 // otherwise per (k, batch bucket).
 inline SweepPlan sweep_plan(int k, int64_t items, int c_override) {
   SweepPlan p{};

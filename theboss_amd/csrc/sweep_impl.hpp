@@ -172,19 +172,23 @@ __device__ __forceinline__ void sweep_chunk(const cd *Vs, const Col0<K - 1, R0> 
   const uint64_t g0 = t0 ^ (t0 >> 1);
   // Half sums h_j = (1/2) sum_nu delta_nu V[nu][j], delta_0 = +1, delta_{b+1} = (-1)^{g_b}.
   double hr[R], hi[R];
-#pragma unroll
-  for (int j = 0; j < R; ++j) {
-    hr[j] = 0.5 * Vs[j].re;
-    hi[j] = 0.5 * Vs[j].im;
-  }
-#pragma unroll 1
-  for (int b = 0; b < NB; ++b) {
-    const double d = ((g0 >> b) & 1ull) ? -0.5 : 0.5;
-    const cd *col = Vs + (b + 1) * R;
+  if constexpr (R0 == 3) {
+    seed_half_sums<R>(hr, hi, (const double *)Vs, (const double *)(Vs + R), NB, c, g0);
+  } else {
 #pragma unroll
     for (int j = 0; j < R; ++j) {
-      hr[j] = fma(d, col[j].re, hr[j]);
-      hi[j] = fma(d, col[j].im, hi[j]);
+      hr[j] = 0.5 * Vs[j].re;
+      hi[j] = 0.5 * Vs[j].im;
+    }
+#pragma unroll 1
+    for (int b = 0; b < NB; ++b) {
+      const double d = ((g0 >> b) & 1ull) ? -0.5 : 0.5;
+      const cd *col = Vs + (b + 1) * R;
+#pragma unroll
+      for (int j = 0; j < R; ++j) {
+        hr[j] = fma(d, col[j].re, hr[j]);
+        hi[j] = fma(d, col[j].im, hi[j]);
+      }
     }
   }
   double Tr, Ti;
@@ -412,21 +416,7 @@ __device__ __forceinline__ void sweep_pair_chunk(const cd *S2, const ColP<K - 1>
   const uint64_t t0 = q << c;
   const uint64_t g0 = t0 ^ (t0 >> 1);
   double ur[R], ui[R];
-#pragma unroll
-  for (int j = 0; j < R; ++j) {
-    ur[j] = 0.5 * S2[j].re;
-    ui[j] = 0.5 * S2[j].im;
-  }
-#pragma unroll 1
-  for (int b = 0; b < NB; ++b) {
-    const double d = ((g0 >> b) & 1ull) ? -0.5 : 0.5;
-    const cd *col = S2 + (b + 2) * R;
-#pragma unroll
-    for (int j = 0; j < R; ++j) {
-      ur[j] = fma(d, col[j].re, ur[j]);
-      ui[j] = fma(d, col[j].im, ui[j]);
-    }
-  }
+  seed_half_sums<R>(ur, ui, (const double *)S2, (const double *)(S2 + 2 * R), NB, c, g0);
   double Xr = 0.0, Xi = 0.0, Yr = 0.0, Yi = 0.0;
   if (t0 & 1ull)
     pair_acc2<-1>(Xr, Xi, Yr, Yi, ur, ui);
