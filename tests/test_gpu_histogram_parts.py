@@ -112,3 +112,17 @@ def test_histogram_in_several_slabs(T):
     _lib.check(lib.tb_outcome_histogram(smp.data_ptr(), m, S, m, n, 1, ref.data_ptr(), None,
                                         T.cuda.current_stream().cuda_stream))
     assert outside == 0 and int(counts.sum()) == S and T.equal(counts, ref.to(T.int64))
+
+
+# the partition's tiles: as many modes as are loaded ahead, one fewer and one more; a last tile
+# whose values are no multiple of four; and tiles smaller than a chunk's sorted offsets
+@pytest.mark.parametrize("m,n,S", [(31, 4, (1 << 19) + 3), (32, 4, (1 << 20) + 1),
+                                   (33, 4, (1 << 20) + 513), (5, 40, (1 << 21) + 77)])
+def test_histogram_partition_tiles(T, m, n, S):
+    from theboss_amd import _lib, ops
+
+    assert _lib.load().tb_outcome_histogram64_workspace_size(S, m, n, 0) > 0
+    smp = _samples(np.random.default_rng(m), S, m, n, False)
+    counts, outside = ops.outcome_histogram(T.from_numpy(smp).cuda(), n)
+    ref, ref_out = _host_counts(smp, n, False, ops.outcome_count(n, m, False))
+    assert np.array_equal(counts.cpu().numpy(), ref) and outside == ref_out

@@ -42,62 +42,113 @@ __device__ __forceinline__ void hist_table(unsigned *T, const HistShape &h) {
   }
 }
 
-// The `rows` samples from `src` on. Rows that follow each other without a gap and start on
-// 16 bytes (a tile's first row is a multiple of 256 rows from the samples' first) are read
-// four values per lane: 62 us for 2^22 samples of 20 modes, 5.4 TB/s, where one value per
-// lane, and the lanes then walking rows of stride m, took 172. Any other stride or start
-// is read value by value.
+// Four values of a tile whose rows follow each other, from value 4 e on, which is of row r and
+// mode c.
+__device__ __forceinline__ void hist_put(int *tile, int e, int r, int c, int4 q, int m) {
+  int *d = tile + 4 * e;
+  if (!(m & 1)) d += r;  // the stride is m + 1
+  d[0] = q.x, d[1] = q.y;
+  if (!(m & 1)) d += c + 2 >= m;  // a row may end after the first two values, and only there
+  d[2] = q.z, d[3] = q.w;
+}
+
+// The values `from` on of `rows` samples, one by one: rows of any stride and start.
 template <int TH>
-__device__ __forceinline__ void hist_stage(int *tile, const int *__restrict__ src, int rows,
-                                           const HistShape &h) {
+__device__ __forceinline__ void hist_stage_each(int *tile, const int *__restrict__ src, int from,
+                                                int rows, const HistShape &h) {
   const int m = h.m, pad = m | 1;
-  int from = 0;
-  const int total = rows * m;
-  if (h.ld == m && ((uintptr_t)src & 15) == 0) {
-    const int4 *s4 = (const int4 *)src;
-    from = total & ~3;
-    if (m & 1) {
-      for (int e = threadIdx.x; e < total / 4; e += TH) {
-        const int4 v = s4[e];
-        int *d = tile + 4 * e;
-        d[0] = v.x, d[1] = v.y, d[2] = v.z, d[3] = v.w;
-      }
-    } else {  // a row may end after the first two values, and only there
-      for (int e = threadIdx.x; e < total / 4; e += TH) {
-        const int4 v = s4[e];
-        const int r = 4 * e / m, c = 4 * e - r * m;
-        int *d = tile + 4 * e + r;
-        d[0] = v.x, d[1] = v.y;
-        d += c + 2 >= m;
-        d[2] = v.z, d[3] = v.w;
-      }
-    }
-  }
-  for (int e = from + threadIdx.x; e < total; e += TH) {
+  for (int e = from + threadIdx.x; e < rows * m; e += TH) {
     const int r = e / m, c = e - r * m;
     tile[r * pad + c] = src[(int64_t)r * h.ld + c];
   }
 }
 
+// Whether rows follow each other without a gap and start on 16 bytes (a tile's first row is a
+// multiple of 256 rows from the samples' first). Those are read four values per lane: 62 us for
+// 2^22 samples of 20 modes, 5.4 TB/s, where one value per lane, and the lanes then walking
+// rows of stride m, took 172.
+__device__ __forceinline__ bool hist_wide(const int *src, const HistShape &h) {
+  return h.ld == h.m && ((uintptr_t)src & 15) == 0;
+}
+
+// The `rows` samples from `src` on.
+template <int TH>
+__device__ __forceinline__ void hist_stage(int *tile, const int *__restrict__ src, int rows,
+                                           const HistShape &h) {
+  const int n4 = hist_wide(src, h) ? rows * h.m / 4 : 0;
+  for (int e = threadIdx.x; e < n4; e += TH) {
+    const int r = 4 * e / h.m;
+    hist_put(tile, e, r, 4 * e - r * h.m, ((const int4 *)src)[e], h.m);
+  }
+  hist_stage_each<TH>(tile, src, 4 * n4, rows, h);
+}
+
+// The same a tile ahead: the next tile's loads are in flight while one is ranked. Up to
+// 4 kHistAhead modes, what the registers hold beside a chunk's ranks.
+constexpr int kHistAhead = 8;
+template <int TH>
+struct HistTile {
+  int4 v[kHistAhead];
+  bool ahead;
+  int r0, c0, dr, dc;  // row and mode of the lane's first value, and of TH lanes further on
+
+  __device__ __forceinline__ void init(const int *samples, const HistShape &h) {
+    ahead = hist_wide(samples, h) && h.m <= 4 * kHistAhead;
+    r0 = 4 * (int)threadIdx.x / h.m;
+    c0 = 4 * (int)threadIdx.x - r0 * h.m;
+    dr = 4 * TH / h.m;
+    dc = 4 * TH - dr * h.m;
+  }
+  __device__ __forceinline__ void load(const int *__restrict__ src, int rows, const HistShape &h) {
+    if (!ahead) return;
+    const int n4 = rows * h.m / 4;
+#pragma unroll
+    for (int k = 0; k < kHistAhead; ++k) {
+      const int e = k * TH + (int)threadIdx.x;
+      if (e < n4) v[k] = ((const int4 *)src)[e];
+    }
+  }
+  __device__ __forceinline__ void stage(int *tile, const int *__restrict__ src, int rows,
+                                        const HistShape &h) const {
+    if (!ahead) {
+      hist_stage<TH>(tile, src, rows, h);
+      return;
+    }
+    const int n4 = rows * h.m / 4;
+    int r = r0, c = c0;
+#pragma unroll
+    for (int k = 0; k < kHistAhead; ++k) {
+      const int e = k * TH + (int)threadIdx.x;
+      if (e < n4) hist_put(tile, e, r, c, v[k], h.m);
+      r += dr;
+      c += dc;
+      if (c >= h.m) {
+        c -= h.m;
+        ++r;
+      }
+    }
+    hist_stage_each<TH>(tile, src, 4 * n4, rows, h);
+  }
+};
+
 constexpr unsigned kHistOutside = ~0u;
 
 // Rank of the sample in `row`, or kHistOutside. The modes are taken from the last, so the
-// particles after a mode are a running sum; entries are checked against 0..n, so the sum
-// stays within m n, and the table's index is held to its row.
+// particles after a mode are a running sum, and the table's index is held to its row. Entries
+// all of 0..n sum up to m n at most; with any other the sample is outside, whatever the sum.
 __device__ __forceinline__ unsigned hist_rank(const int *row, const unsigned *T,
                                               const HistShape &h) {
   const int W = h.n + 1;
-  int after = 0;
-  bool bad = false;
-  unsigned rank = 0;
+  unsigned after = 0, most = 0, rank = 0;
   const unsigned *t = T;
   for (int i = h.m - 1; i >= 0; --i, t += W) {
-    rank += t[min((unsigned)after, (unsigned)h.n)];
-    const int v = row[i];
-    bad |= (unsigned)v > (unsigned)h.n;
-    after += bad ? 0 : v;
+    rank += t[min(after, (unsigned)h.n)];
+    const unsigned v = (unsigned)row[i];
+    most = max(most, v);
+    after += v;
   }
-  if (bad || after > h.n || (!h.losses && after != h.n)) return kHistOutside;
+  if (most > (unsigned)h.n || after > (unsigned)h.n || (!h.losses && after != (unsigned)h.n))
+    return kHistOutside;
   return rank + (h.losses ? t[after] : 0u);  // row m: where the block begins
 }
 
@@ -151,15 +202,18 @@ __global__ __launch_bounds__(TH) void outcome_histogram_kernel(
 // each bucket's run begins in each chunk; a second kernel counts one bucket per workgroup in
 // LDS, over its run of every chunk, and writes the counters once, so they need no clearing.
 //
-// The sample loads bound the first kernel and the counters' stores the second. 2^22 samples of
-// 20 modes: 154 us with 20 million counters (the direct kernel 212, and 350 with a clear and
-// a widening pass of 75 more for the 32-bit counters and ranks of before), 117 with 177100
-// (200).
+// The sample loads bound the first kernel and the counters' stores the second. 2^22 samples,
+// per call: 160 us of 20 modes with 20 million counters, 96 of 18 modes with 100947; 178 and 134
+// when a tile was loaded only after the one before it had been ranked and the offsets went from
+// registers to their places in memory, two bytes each, instead of through LDS. (The direct kernel
+// took 35% longer, and the 32-bit counters with a clearing and a widening pass 446.) The direct
+// kernel gains nothing from loads a tile ahead: 286 counters in LDS 62 us against 49, as the
+// registers cost it a workgroup per CU.
 //
 // Rows per thread, so samples per chunk: about 512 chunks are two workgroups per CU; fewer
 // leave CUs without loads in flight (2^20 samples of 20 modes into 20 million counters in 128,
-// 256 and 512 chunks: 92, 69 and 63 us), more cut the runs short (2^22 in 512, 1024 and 2048:
-// 154, 170 and 180).
+// 256 and 512 chunks, before the loads ahead: 92, 69 and 63 us), more cut the runs short (2^22 in
+// 512, 1024 and 2048: 154, 170 and 180).
 constexpr int kHistPartThreads = 512;
 constexpr int kHistMaxShift = 14, kHistMaxBuckets = 4096;
 
@@ -171,17 +225,25 @@ __global__ __launch_bounds__(kHistPartThreads) void hist_partition_kernel(
   extern __shared__ unsigned hist_lds[];
   unsigned *T = hist_lds;
   int *tile = (int *)(T + (h.m + 1) * (h.n + 1));
-  unsigned *fill = (unsigned *)(tile + TH * (h.m | 1));  // [buckets]
-  unsigned *wave_sum = fill + buckets;                   // [WAVES]
+  uint16_t *sorted = (uint16_t *)tile;                                 // [ROWS * TH], at the end
+  unsigned *fill = (unsigned *)(tile + TH * max(h.m | 1, ROWS / 2));  // [buckets]
+  unsigned *wave_sum = fill + buckets;                                 // [WAVES]
   for (int e = threadIdx.x; e < buckets; e += TH) fill[e] = 0;
-  hist_table<TH>(T, h);
   const int64_t first = (int64_t)blockIdx.x * (ROWS * TH);
+  const auto rows_at = [&](int it) {
+    return (int)max((int64_t)0, min((int64_t)TH, (int64_t)S - first - it * TH));
+  };
+  HistTile<TH> in;
+  in.init(samples, h);
+  in.load(samples + first * h.ld, rows_at(0), h);
+  hist_table<TH>(T, h);
   unsigned rank[ROWS], slot[ROWS];
 #pragma unroll
   for (int it = 0; it < ROWS; ++it) {
     const int64_t base = first + it * TH;
-    const int rows = (int)max((int64_t)0, min((int64_t)TH, (int64_t)S - base));
-    if (rows) hist_stage<TH>(tile, samples + base * h.ld, rows, h);
+    const int rows = rows_at(it);
+    in.stage(tile, samples + base * h.ld, rows, h);
+    if (it + 1 < ROWS) in.load(samples + (base + TH) * h.ld, rows_at(it + 1), h);
     __syncthreads();
     rank[it] = kHistOutside;
     slot[it] = 0;
@@ -214,17 +276,18 @@ __global__ __launch_bounds__(kHistPartThreads) void hist_partition_kernel(
     col[(int64_t)b * gridDim.x] = (uint16_t)at;
     at += c;
   }
-  if (threadIdx.x == TH - 1) {  // the last piece ends at the chunk's total
-    unsigned total = 0;
-    for (int w = 0; w < WAVES; ++w) total += wave_sum[w];
-    col[(int64_t)buckets * gridDim.x] = (uint16_t)total;
-  }
+  unsigned total = 0;
+  for (int w = 0; w < WAVES; ++w) total += wave_sum[w];
+  if (threadIdx.x == TH - 1) col[(int64_t)buckets * gridDim.x] = (uint16_t)total;
   __syncthreads();
-  uint16_t *out = offsets + first;
 #pragma unroll
   for (int it = 0; it < ROWS; ++it)
     if (rank[it] != kHistOutside)
-      out[fill[rank[it] >> shift] + slot[it]] = (uint16_t)(rank[it] & ((1u << shift) - 1));
+      sorted[fill[rank[it] >> shift] + slot[it]] = (uint16_t)(rank[it] & ((1u << shift) - 1));
+  __syncthreads();
+  // two at a time; past an odd total one more of the chunk's own, which nothing reads
+  unsigned *out = (unsigned *)(offsets + first);
+  for (unsigned e = threadIdx.x; 2 * e < total; e += TH) out[e] = ((const unsigned *)sorted)[e];
 }
 
 constexpr int kHistCountThreads = 1024, kHistRunLanes = 8;
@@ -303,6 +366,13 @@ size_t hist_lds_bytes(const tb::HistShape &h, int threads, int64_t words) {
          sizeof(unsigned);
 }
 
+// The partition's tile also holds a chunk's sorted offsets.
+size_t hist_part_lds(const tb::HistShape &h, int rows, int64_t buckets) {
+  const int tile = std::max(h.m | 1, rows / 2);
+  return ((size_t)(h.m + 1) * (h.n + 1) + (size_t)tb::kHistPartThreads * tile +
+          (size_t)buckets + tb::kHistPartThreads / 64) * sizeof(unsigned);
+}
+
 template <typename K>
 int32_t hist_allow_lds(K kernel, size_t lds) {
   if (lds <= 64 * 1024) return TB_OK;
@@ -363,12 +433,10 @@ HistParts hist_parts(const tb::HistShape &h, int64_t bins, int S) {
   if (S < kHistPartMinSamples || hist_lds_threads(h, bins, S)) return p;
   while (p.shift < tb::kHistMaxShift && (bins >> p.shift) >= 1024) ++p.shift;
   const int64_t buckets = ((bins - 1) >> p.shift) + 1;
-  if (buckets > tb::kHistMaxBuckets ||
-      hist_lds_bytes(h, tb::kHistPartThreads, buckets + 8) > kHistLds)
-    return p;
+  p.rows = S <= 1 << 20 ? 4 : S <= 1 << 21 ? 8 : 16;
+  if (buckets > tb::kHistMaxBuckets || hist_part_lds(h, p.rows, buckets) > kHistLds) return p;
   p.use = true;
   p.buckets = (int)buckets;
-  p.rows = S <= 1 << 20 ? 4 : S <= 1 << 21 ? 8 : 16;
   p.chunk = p.rows * tb::kHistPartThreads;
   const int64_t most = std::min<int64_t>(S, kHistSlab);
   p.slab_chunks = (int)((most + p.chunk - 1) / p.chunk);
@@ -415,7 +483,8 @@ extern "C" int32_t tb_outcome_histogram64(const int32_t *samples, int32_t ld, in
   if (!counts) return tbh::fail(TB_EINVAL, "histogram: NULL pointer");
   const tb::HistShape h{m, n, ld, losses ? 1 : 0};
   const HistParts p = hist_parts(h, bins, samples_n);
-  const bool parts = p.use && workspace && workspace_bytes >= p.bytes;
+  const bool parts =
+      p.use && workspace && ((uintptr_t)workspace & 3) == 0 && workspace_bytes >= p.bytes;
   const int64_t clear = parts ? 0 : bins;
   hipLaunchKernelGGL(tb::hist_clear_kernel,
                      dim3((int)std::min<int64_t>(std::max<int64_t>((clear + 255) / 256, 1), 4096)),
@@ -426,7 +495,7 @@ extern "C" int32_t tb_outcome_histogram64(const int32_t *samples, int32_t ld, in
     return hist_count(samples, samples_n, h, bins, (unsigned *)counts, 2, (unsigned *)outside, s);
   uint16_t *offsets = (uint16_t *)workspace;
   uint16_t *starts = (uint16_t *)((char *)workspace + p.starts_at);
-  const size_t lds = hist_lds_bytes(h, tb::kHistPartThreads, p.buckets + 8);
+  const size_t lds = hist_part_lds(h, p.rows, p.buckets);
   const size_t lds_count = sizeof(unsigned) << p.shift;
   auto partition = p.rows == 4   ? &tb::hist_partition_kernel<4>
                    : p.rows == 8 ? &tb::hist_partition_kernel<8>
