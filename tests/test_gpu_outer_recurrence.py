@@ -136,3 +136,20 @@ def test_op_takes_both_routes_and_the_calculator_says_which(T, oracle):
     for how in (True, None):
         for formula in (0, 1):
             assert close(ops.guan_perm_outer(U, *o, *i, formula, how).cpu().numpy(), walk)
+
+
+def test_walk_of_the_rows_left_in_a_large_call(T, oracle):
+    """More than 64 turns of the walk that follows the recurrence; rows left to it here and there."""
+    n_out, m = 120001, 12
+    U = T.from_numpy(oracle.haar_unitary(m, 4)).cuda()
+    ins = np.zeros((36, m), dtype=np.int64)
+    ins[:, :9] = substates((1,) * 9, 2)
+    rng = np.random.default_rng(8)
+    modes = rng.integers(0, m, (n_out, 2)).astype(np.int32)
+    mult = np.ones((n_out, 2), dtype=np.int32)
+    left = np.array([0, 3000, 3001, 60000, n_out - 1])
+    mult[left] = 2
+    outs = [T.from_numpy(modes).cuda(), T.from_numpy(mult).cuda()]
+    got, walk = both(T, U, outs, rows_to_device(T, ins))
+    assert np.array_equal(got[left], walk[left])
+    assert close(np.delete(got, left, 0), np.delete(walk, left, 0))

@@ -375,7 +375,8 @@ __global__ __launch_bounds__(64) void guan_kernel(const cd *__restrict__ U, int 
 }
 
 // All-pairs form. AFTER: the launch follows the subset recurrence, which has usually done every
-// row, so its grid is bounded and each block loops over its share of the items.
+// row, so its grid is bounded and each block loops over its share of the items; it reads the
+// flags of 64 turns at once, a lane each, and skips the turns whose rows are all done.
 template <int JB, int IPW, bool AFTER>
 __global__ __launch_bounds__(64) void guan_outer_kernel(
     const cd *__restrict__ U, int ldu, const int *__restrict__ out_modes,
@@ -387,9 +388,28 @@ __global__ __launch_bounds__(64) void guan_outer_kernel(
     guan_items<JB, IPW, true>(U, ldu, out_modes, out_mult, out_max, in_modes, in_mult, in_max,
                               batch, n_in, formula, 0, (int)blockIdx.x * IPW, nullptr, smem, out);
   } else {
-    for (int64_t b0 = (int64_t)blockIdx.x * IPW; b0 < batch; b0 += (int64_t)gridDim.x * IPW) {
+    const int64_t stride = (int64_t)gridDim.x * IPW;
+    uint64_t todo = 0, whole = 0;  // of 64 turns: any, and every row is left
+    int64_t b0 = (int64_t)blockIdx.x * IPW;
+    for (int turn = 0; b0 < batch; b0 += stride, ++turn) {
+      if ((turn & 63) == 0) {
+        const int64_t own = b0 + threadIdx.x * stride;
+        bool left = false, all = true;
+        if (own < batch) {
+          const int j1 = (int)(min(own + IPW, (int64_t)batch) - 1) / n_in;
+          for (int j = (int)own / n_in; j <= j1; ++j) {
+            const bool l = done[j] == 0;
+            left |= l;
+            all &= l;
+          }
+        }
+        todo = __ballot(left);
+        whole = __ballot(all);
+      }
+      if (!((todo >> (turn & 63)) & 1)) continue;
       guan_items<JB, IPW, true>(U, ldu, out_modes, out_mult, out_max, in_modes, in_mult, in_max,
-                                batch, n_in, formula, 0, (int)b0, done, smem, out);
+                                batch, n_in, formula, 0, (int)b0,
+                                (whole >> (turn & 63)) & 1 ? nullptr : done, smem, out);
       __syncthreads();  // the next items reuse the LDS blocks
     }
   }
@@ -412,9 +432,10 @@ size_t guan_lds_bytes(int out_max, int in_max, int mode, int ipw) {
 
 // n_in > 0: the all-pairs form over batch = n_out * n_in items (mode 0 only); done (may be
 // null): output rows already written. Those launches use a bounded grid, since the walk is
-// then the exception (1.0M pairs all done: 126,000 one-wave blocks that only read their flag
-// take 15 us longer than 4096; nothing done: the bounded grid takes 350 us instead of 356).
-constexpr int kGuanAfterRecurrenceBlocks = 4096;
+// then the exception. 1.0M pairs all done: 5 us, 12 when each turn read its own flags and 27 as
+// 126,000 one-wave blocks. Nothing done, 90,000 pairs of k = 8 after an attempt in vain: 201 us,
+// 232 with half the blocks, 192 without the attempt.
+constexpr int kGuanAfterRecurrenceBlocks = 8192;
 int32_t run_guan(const tb::cd *U, int ldu, const int *out_modes, const int *out_mult, int out_max,
                  const int *in_modes, const int *in_mult, int in_max, int batch, int formula,
                  int mode, tb::cd *out, hipStream_t s, int n_in = 0, const int *done = nullptr) {

@@ -13,12 +13,16 @@
 // multiplies: n = 10, k = 5: 2560 against 40,000. No term cancels another by construction, so the
 // result is at least as accurate as the alternating sums.
 //
-// What bounds it: latency (GCC-A layer of 200 prefixes x 20 outputs x C(10, 5) inputs, 1.0M
-// pairs: 42 us, 4 of them the 16 MB written; the walk 351). A workgroup first builds the lattice from the input rows (in LDS, for
-// itself: a plan kernel with predecessor lists in global memory took 20 us more per call),
-// then a wave per output row walks the levels (the whole workgroup where the levels are wide
-// or the rows few). The Guan walk follows in stream order over the rows whose done flag is 0:
-// all of them when the lattice is too large, or a row whose particle number differs.
+// What bounds it (GCC-A layer of 200 prefixes x 20 outputs x C(10, 5) inputs, 1.0M pairs: 32 us a
+// call, 4 of them the 16 MB written; the walk 351): a workgroup first builds the lattice from
+// the input rows, 19,000 cycles of latency (in LDS, for itself: a plan kernel with predecessor
+// lists in global memory took 20 us more per call); then a wave per output row walks the levels
+// (the whole workgroup where the levels are wide or the rows few), 17,000 cycles a row with the
+// eight waves of a CU sharing its LDS reads. Slots loaded all at once and a row ahead, levels
+// unrolled, and ranks that share their low bits: 42 us before, with the walk's flags (below); 12
+// modes, k = 6, 1200 rows: 77 -> 54. The Guan walk follows in stream order over the rows whose
+// done flag is 0: all of them when the lattice is too large, or a row whose particle number
+// differs.
 #include <algorithm>
 
 #include "tb_common.hpp"
@@ -55,6 +59,26 @@ struct SubsetLds {
   SubsetPlan p;
 };
 
+// An input row in registers, all its slots loaded at once (in_max <= kSubModes); slots past
+// in_max are empty. Slot by slot the loads of the plan came one latency after the other.
+struct SubsetIn {
+  int d[kSubModes], m[kSubModes];
+};
+__device__ __forceinline__ SubsetIn subset_in(const int *__restrict__ in_modes,
+                                              const int *__restrict__ in_mult, int in_max, int i) {
+  SubsetIn r;
+  const int *sm = in_modes + (size_t)i * in_max, *su = in_mult + (size_t)i * in_max;
+#pragma unroll
+  for (int q = 0; q < kSubModes; ++q) {
+    const int at = min(q, in_max - 1);
+    r.d[q] = sm[at];
+    r.m[q] = su[at];
+  }
+#pragma unroll
+  for (int q = 0; q < kSubModes; ++q) r.m[q] = q < in_max ? max(r.m[q], 0) : 0;
+  return r;
+}
+
 // Fills S.p, S.order, S.pos and S.in_pos; S.p.ok = 0 when the rows have no small lattice.
 __device__ __forceinline__ void subset_plan(SubsetLds &S, const int *__restrict__ in_modes,
                                             const int *__restrict__ in_mult, int in_max, int n_in,
@@ -72,23 +96,27 @@ __device__ __forceinline__ void subset_plan(SubsetLds &S, const int *__restrict_
   if (tid == 0) S.bad = 0;
   // multiplicities above kSubK are refused below, so capped sums cannot wrap
   int k = 0;
-  for (int q = 0; q < in_max; ++q) k += min(max(in_mult[q], 0), kSubK + 1);
+  const SubsetIn first = subset_in(in_modes, in_mult, in_max, 0);
+  SubsetIn in = subset_in(in_modes, in_mult, in_max, min(tid, n_in - 1));
+#pragma unroll
+  for (int q = 0; q < kSubModes; ++q) k += min(first.m[q], kSubK + 1);
   __syncthreads();
   for (int i = tid; i < n_in; i += 256) {
-    const int *sm = in_modes + (size_t)i * in_max, *su = in_mult + (size_t)i * in_max;
+    if (i != tid) in = subset_in(in_modes, in_mult, in_max, i);
     int sum = 0;
     bool refuse = false;
-    for (int q = 0; q < in_max; ++q) {
-      const int m = su[q], d = sm[q];
-      if (m <= 0) continue;
+#pragma unroll
+    for (int q = 0; q < kSubModes; ++q) {
+      const int m = in.m[q], d = in.d[q];
+      if (m == 0) continue;
       sum += min(m, kSubK + 1);
       if (d < 0 || d >= ldu || m > kSubK) {
         refuse = true;
         continue;
       }
       int all = m;  // a mode may fill several slots
-      for (int r = 0; r < q; ++r)
-        if (su[r] > 0 && sm[r] == d) all += min(su[r], kSubK + 1);
+#pragma unroll
+      for (int r = 0; r < q; ++r) all += in.d[r] == d ? min(in.m[r], kSubK + 1) : 0;
       atomicMax(&S.top[d], all);
     }
     if (refuse || sum != k) S.bad = 1;
@@ -129,10 +157,11 @@ __device__ __forceinline__ void subset_plan(SubsetLds &S, const int *__restrict_
   if (tid < p.D) S.top[p.modes[tid]] = tid;
   __syncthreads();
   for (int i = tid; i < n_in; i += 256) {
-    const int *sm = in_modes + (size_t)i * in_max, *su = in_mult + (size_t)i * in_max;
+    if (n_in > 256) in = subset_in(in_modes, in_mult, in_max, i);
     int code = 0;
-    for (int q = 0; q < in_max; ++q)
-      if (su[q] > 0) code += su[q] * p.stride[S.top[sm[q]]];
+#pragma unroll
+    for (int q = 0; q < kSubModes; ++q)
+      if (in.m[q] > 0) code += in.m[q] * p.stride[S.top[in.d[q]]];
     S.in_pos[i] = (unsigned short)code;
   }
   if (p.multi) {
@@ -143,9 +172,11 @@ __device__ __forceinline__ void subset_plan(SubsetLds &S, const int *__restrict_
     }
   } else {  // one particle per mode: the rank among the subsets of the same size
     if (tid <= min(p.k, p.D)) p.cnt[tid] = S.binom[p.D][tid];
+    int low = 0, n_low = 0;  // of the eight bits that a thread's points share
+    for (int m = min(tid, p.total - 1); m; m &= m - 1) low += S.binom[__ffs(m) - 1][++n_low];
     for (int c = tid; c < p.total; c += 256) {
-      int r = 0, i = 1;
-      for (int m = c; m; m &= m - 1, ++i) r += S.binom[__ffs(m) - 1][i];
+      int r = low, i = n_low;
+      for (int m = c >> 8; m; m &= m - 1) r += S.binom[7 + __ffs(m)][++i];
       S.pos[c] = (unsigned short)r;
     }
   }
@@ -181,44 +212,90 @@ __device__ __forceinline__ void cfma(double &re, double &im, cd a, cd b) {
   im = fma(a.im, b.re, im);
 }
 
-// Level l from level l - 1 by the T threads of a group (t inside it).
-template <int T, bool MULTI>
-__device__ __forceinline__ void subset_level(const SubsetLds &S, const cd *src, cd *dst, const cd *u,
-                                             int l, int t) {
+// Level L from level L - 1 by the T threads of a group (t inside it), one particle per mode:
+// every point of the level has L bits. Unrolled, so that the reads of a point are all in flight.
+template <int T, int L>
+__device__ __forceinline__ void subset_level_bits(const SubsetLds &S, const cd *src, cd *dst,
+                                                  const cd *u, int t) {
+  const int cnt = S.p.cnt[L];
+  const unsigned short *order = S.order + S.p.off[L];
+  for (int i = t; i < cnt; i += T) {
+    const int c = order[i];
+    double re = 0.0, im = 0.0;
+    int m = c;
+#pragma unroll
+    for (int j = 0; j < L; ++j) {
+      const int bit = m & -m;
+      m ^= bit;
+      cfma(re, im, u[__ffs(bit) - 1], src[S.pos[c ^ bit]]);
+    }
+    dst[i] = {re, im};
+  }
+}
+
+// The same with several particles per mode.
+template <int T>
+__device__ __forceinline__ void subset_level_multi(const SubsetLds &S, const cd *src, cd *dst,
+                                                   const cd *u, int l, int t) {
   const SubsetPlan &p = S.p;
   const int cnt = p.cnt[l];
   const unsigned short *order = S.order + p.off[l];
   for (int i = t; i < cnt; i += T) {
     const int c = order[i];
     double re = 0.0, im = 0.0;
-    if constexpr (MULTI) {
-      for (int d = 0; d < p.D; ++d) {
-        const int st = p.stride[d];
-        const int s = (c / st) % p.radix[d];
-        if (s == 0) continue;
-        const cd w = u[d];
-        cfma(re, im, {(double)s * w.re, (double)s * w.im}, src[S.pos[c - st]]);
-      }
-    } else {
-      int m = c;
-#pragma unroll 4
-      for (int j = 0; j < l; ++j) {  // every point of level l has l bits
-        const int bit = m & -m;
-        m ^= bit;
-        cfma(re, im, u[__ffs(bit) - 1], src[S.pos[c ^ bit]]);
-      }
+    for (int d = 0; d < p.D; ++d) {
+      const int st = p.stride[d];
+      const int s = (c / st) % p.radix[d];
+      if (s == 0) continue;
+      const cd w = u[d];
+      cfma(re, im, {(double)s * w.re, (double)s * w.im}, src[S.pos[c - st]]);
     }
     dst[i] = {re, im};
   }
 }
 
-// Output row j by the T threads of a group; F holds two levels of p.width values.
+template <int T>
+__device__ __forceinline__ void subset_level(const SubsetLds &S, const cd *src, cd *dst, const cd *u,
+                                             int l, int t) {
+  if (S.p.multi) {
+    subset_level_multi<T>(S, src, dst, u, l, t);
+    return;
+  }
+  static_assert(kSubK == 12, "a case for each level");
+  switch (l) {
+    case 1: subset_level_bits<T, 1>(S, src, dst, u, t); break;
+    case 2: subset_level_bits<T, 2>(S, src, dst, u, t); break;
+    case 3: subset_level_bits<T, 3>(S, src, dst, u, t); break;
+    case 4: subset_level_bits<T, 4>(S, src, dst, u, t); break;
+    case 5: subset_level_bits<T, 5>(S, src, dst, u, t); break;
+    case 6: subset_level_bits<T, 6>(S, src, dst, u, t); break;
+    case 7: subset_level_bits<T, 7>(S, src, dst, u, t); break;
+    case 8: subset_level_bits<T, 8>(S, src, dst, u, t); break;
+    case 9: subset_level_bits<T, 9>(S, src, dst, u, t); break;
+    case 10: subset_level_bits<T, 10>(S, src, dst, u, t); break;
+    case 11: subset_level_bits<T, 11>(S, src, dst, u, t); break;
+    case 12: subset_level_bits<T, 12>(S, src, dst, u, t); break;
+  }
+}
+
+// A lane's slot of an output row (out_max <= 64); empty past the row's slots and past the rows.
+struct SubsetSlot {
+  int m, d;
+};
+__device__ __forceinline__ SubsetSlot subset_slot(const int *__restrict__ out_modes,
+                                                  const int *__restrict__ out_mult, int out_max,
+                                                  int n_out, int64_t j) {
+  const int lane = threadIdx.x & 63;
+  if (lane >= out_max || j >= n_out) return {0, 0};
+  return {max(out_mult[j * out_max + lane], 0), out_modes[j * out_max + lane]};
+}
+
+// Output row j, of these slots, by the T threads of a group; F holds two levels of p.width
+// values.
 template <int T>
 __device__ __forceinline__ void subset_row(SubsetLds &S, const cd *__restrict__ U, int ldu,
-                                           const int *__restrict__ out_modes,
-                                           const int *__restrict__ out_mult, int out_max, int j,
-                                           int n_in, cd *F, cd *Ul, int *rl, int *__restrict__ done,
-                                           cd *__restrict__ out) {
+                                           SubsetSlot slot, int j, int n_in, cd *F, cd *Ul, int *rl,
+                                           int *__restrict__ done, cd *__restrict__ out) {
   const SubsetPlan &p = S.p;
   const int lane = threadIdx.x & 63, t = T == 64 ? lane : (int)threadIdx.x;
   auto wave_sync = [] {
@@ -231,12 +308,8 @@ __device__ __forceinline__ void subset_row(SubsetLds &S, const cd *__restrict__ 
     else
       __syncthreads();
   };
-  // The row's particles, one after the other: a lane per slot (out_max <= 64).
-  int m = 0, md = 0;
-  if (lane < out_max) {
-    m = max(out_mult[(size_t)j * out_max + lane], 0);
-    md = out_modes[(size_t)j * out_max + lane];
-  }
+  // The row's particles, one after the other.
+  const int m = slot.m, md = slot.d;
   int incl = m;
 #pragma unroll
   for (int off = 1; off < 64; off <<= 1) {
@@ -258,10 +331,7 @@ __device__ __forceinline__ void subset_row(SubsetLds &S, const cd *__restrict__ 
   for (int l = 1; l <= p.k; ++l) {
     const cd *src = F + ((l & 1) ? 0 : p.width);
     cd *dst = F + ((l & 1) ? p.width : 0);
-    if (p.multi)
-      subset_level<T, true>(S, src, dst, Ul + (l - 1) * p.D, l, t);
-    else
-      subset_level<T, false>(S, src, dst, Ul + (l - 1) * p.D, l, t);
+    subset_level<T>(S, src, dst, Ul + (l - 1) * p.D, l, t);
     sync();
   }
   const cd *last = F + ((p.k & 1) ? p.width : 0);
@@ -275,20 +345,31 @@ __global__ __launch_bounds__(256) void subset_rows_kernel(
     const int *__restrict__ out_mult, int out_max, int n_out, int *__restrict__ done,
     cd *__restrict__ out) {
   __shared__ SubsetLds S;
-  subset_plan(S, in_modes, in_mult, in_max, n_in, ldu);
   const int wave = threadIdx.x >> 6;
+  // A row per wave or per workgroup, its slots loaded while the plan is made or the row before
+  // it is done; which of the two is known for most calls before the plan.
+  const bool many = n_out >= kSubWaveRows;
+  int64_t j = many ? blockIdx.x * 4 + wave : blockIdx.x;
+  SubsetSlot slot = subset_slot(out_modes, out_mult, out_max, n_out, j);
+  subset_plan(S, in_modes, in_mult, in_max, n_in, ldu);
   if (!S.p.ok) {
-    for (int j = blockIdx.x * 256 + threadIdx.x; j < n_out; j += gridDim.x * 256) done[j] = 0;
+    for (int e = blockIdx.x * 256 + threadIdx.x; e < n_out; e += gridDim.x * 256) done[e] = 0;
     return;
   }
-  if (n_out >= kSubWaveRows && 2 * S.p.width <= kSubWaveEntries) {
-    for (int j = blockIdx.x * 4 + wave; j < n_out; j += gridDim.x * 4)
-      subset_row<64>(S, U, ldu, out_modes, out_mult, out_max, j, n_in,
-                     S.F + wave * kSubWaveEntries, S.Ul[wave], S.rl[wave], done, out);
-  } else {
-    for (int j = blockIdx.x; j < n_out; j += gridDim.x)
-      subset_row<256>(S, U, ldu, out_modes, out_mult, out_max, j, n_in, S.F, S.Ul[wave],
-                      S.rl[wave], done, out);
+  const bool waves = many && 2 * S.p.width <= kSubWaveEntries;
+  if (many && !waves) {
+    j = blockIdx.x;
+    slot = subset_slot(out_modes, out_mult, out_max, n_out, j);
+  }
+  const int64_t step = (int64_t)gridDim.x * (waves ? 4 : 1);
+  for (; j < n_out; j += step) {
+    const SubsetSlot next = subset_slot(out_modes, out_mult, out_max, n_out, j + step);
+    if (waves)
+      subset_row<64>(S, U, ldu, slot, (int)j, n_in, S.F + wave * kSubWaveEntries, S.Ul[wave],
+                     S.rl[wave], done, out);
+    else
+      subset_row<256>(S, U, ldu, slot, (int)j, n_in, S.F, S.Ul[wave], S.rl[wave], done, out);
+    slot = next;
   }
 }
 
@@ -300,7 +381,7 @@ namespace tbsub {
 // large enough to gain: pairs times the 2^in_max codes of a pair's walk of at least 2^20. The
 // recurrence takes 14-28 us plus its share of the rows, the walk 9 us plus its pairs; they cross
 // near that line (20 modes, 10 photons: k = 3, 24,000 pairs 9 us walked, 15 by recurrence;
-// k = 4, 42,000: 16, 16; k = 6, 42,000: 40, 20; k = 8, 9000: 39, 26; k = 5, 1,008,000: 351, 42).
+// k = 4, 42,000: 16, 16; k = 6, 42,000: 40, 19; k = 8, 9000: 39, 26; k = 5, 1,008,000: 351, 32).
 constexpr int64_t kSubMinCodes = 1 << 20;
 bool attempt(int ldu, int out_max, int n_out, int in_max, int n_in) {
   if (n_out < 1 || n_in < 1 || in_max < 1 || out_max < 1 || ldu < 1) return false;
