@@ -71,8 +71,8 @@ def clock_during(fn, seconds):
 
 class GuanFlops:
     """Counts, inside the with-block, the multiplicity-aware algorithmic flops of every
-    tb_guan_perm_batch and tb_guan_perm_outer launch the calculators make: per item (pair)
-    prod_d (e_d + 1) Guan codes, each costing 2|T| + 6(sum t - 1) + 2 (|T| complex adds
+    tb_guan_perm_batch, tb_guan_perm_outer and tb_gcca_layer_pmfs call the calculators make:
+    per item (pair) prod_d (e_d + 1) Guan codes, each costing 2|T| + 6(sum t - 1) + 2 (|T| complex adds
     into the sums of the product side's distinct modes, sum t - 1 complex multiplies, the
     accumulation), with e the enumerated side's multiplicities and t the product side's. Calls
     that take the subset recurrence are charged the same, the walk they replace.
@@ -94,10 +94,7 @@ class GuanFlops:
             self.items += int(in_mult.shape[0])
             return self._orig(U, out_modes, out_mult, in_modes, in_mult, formula)
 
-        self._orig_outer = ops.guan_perm_outer
-
-        def counted_outer(U, out_modes, out_mult, in_modes, in_mult, formula=L.TB_FORMULA_RYSER,
-                          common=None):
+        def add_pairs(out_mult, in_mult):
             # pair (j, i) enumerates the T row j when it has fewer codes than the S row i
             f64 = T.float64
             codes_t, codes_s = (out_mult.to(f64) + 1).prod(dim=1), (in_mult.to(f64) + 1).prod(dim=1)
@@ -108,15 +105,27 @@ class GuanFlops:
             self._acc += T.where(codes_t[:, None] < codes_s[None, :], enum_t, enum_s).sum()
             self.launches += 1
             self.items += int(out_mult.shape[0]) * int(in_mult.shape[0])
-            return self._orig_outer(U, out_modes, out_mult, in_modes, in_mult, formula, common)
+
+        self._orig_outer, self._orig_layer = ops.guan_perm_outer, ops.gcca_layer_pmfs
+
+        def counted_outer(U, out_modes, out_mult, in_modes, in_mult, *args, **kw):
+            add_pairs(out_mult, in_mult)
+            return self._orig_outer(U, out_modes, out_mult, in_modes, in_mult, *args, **kw)
+
+        def counted_layer(U, prefixes, width, in_modes, in_mult, *args, **kw):
+            one = T.eye(prefixes.shape[1], dtype=prefixes.dtype, device=prefixes.device)
+            add_pairs((prefixes[:, None, :] + one).flatten(0, 1), in_mult)
+            return self._orig_layer(U, prefixes, width, in_modes, in_mult, *args, **kw)
 
         ops.guan_perm_batch = counted
         ops.guan_perm_outer = counted_outer
+        ops.gcca_layer_pmfs = counted_layer
         return self
 
     def __exit__(self, *exc):
         ops.guan_perm_batch = self._orig
         ops.guan_perm_outer = self._orig_outer
+        ops.gcca_layer_pmfs = self._orig_layer
         self.flops = float(self._acc.item())
         return False
 
@@ -124,7 +133,7 @@ class GuanFlops:
 def sweep_small(checker):
     """The C&C minors sweep as the drop-in submatrices calculator and the plain GCC-B path
     launch it: one item, and small batches, at k = 20 (the batch-aware built-in plan cuts
-    the chunks until the launch has ~4096 waves, not below 2^5 Gray steps per lane)."""
+    the chunks until the launch has ~4096 waves, or 1024 below 2^5 Gray steps per lane)."""
     T = D.torch()
     lib = L.load()
     k = 20
