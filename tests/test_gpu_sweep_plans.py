@@ -65,3 +65,10 @@ def test_plans_and_tasks(T, k, items):
     got = ops.cc_submatrices_batch(Ud, om, ou, dev(wide_m), dev(wide_u), k, True)
     assert not got[:, 0].abs().any()
     close(got[:, 1:])
+
+
+# waves that walk several chunks: one wave per item (written directly) and several, with the wide
+# reduction too, and batches just past a round of waves
+@pytest.mark.parametrize("k,items", [(13, 1025), (14, 1501), (16, 301), (18, 70), (20, 17)])
+def test_several_chunks_per_wave(T, k, items):
+    test_plans_and_tasks(T, k, items)

@@ -288,6 +288,9 @@ constexpr int64_t kSweepMaxBlocks = 8192;  // 4 one-wave blocks per SIMD of 256 
 // per SIMD (one-wave blocks, 2 resident per SIMD, so two rounds and a short tail).
 constexpr int64_t kSweepWaveTarget = 4096;
 
+// What a wave of the sweep costs besides walking, in codes: seeding a chunk; staging and the sums.
+constexpr int64_t kSweepSeedCodes = 10, kSweepWaveCodes = 10;
+
 // Built-in chunk: the longest walk (at most 2^11 Gray steps per lane) that still gives the
 // launch kSweepWaveTarget waves, but not below 2^5 steps. A batch of 4096 k = 20 items
 // keeps 2^11 (4 waves per item); one k = 20 item gets 2^5 (256 waves) instead of a
@@ -297,7 +300,16 @@ constexpr int64_t kSweepWaveTarget = 4096;
 // 19.7, 17.2; past the lines 100 k = 16 items 28, 41, 52 and one k = 20 item 28.5, 28.1, 30.4),
 // unless one wave is an item. The tuner may choose
 // otherwise per (k, batch bucket).
-inline SweepPlan sweep_plan(int k, int64_t items, int c_override) {
+//
+// all_items: the launch sweeps all `items`, not a part of them that only the device knows, so its
+// waves share the SIMDs evenly and a launch lasts as long as the SIMD with the most waves. A wave
+// then walks as many chunks as make ceil(waves / 1024) times its cost least, where that is less by
+// a tenth (fewer waves per SIMD hide less latency: 200 k = 15 items, less by 0.096, took 26 us
+// instead of 24), or a twentieth where it saves the reduction: 2000 k = 14 items 71 -> 57 us, 1000 of
+// k = 15 76 -> 65, 4 of k = 22 67 -> 60. Longer chunks in place of more of them gain up to twice that, but
+// the half sums drift: 200 k = 18 items from 4e-15 to 2e-14. The partials are never more than the
+// workspace, which is sized without this, holds.
+inline SweepPlan sweep_plan(int k, int64_t items, int c_override, bool all_items = false) {
   SweepPlan p{};
   const int nb = k - 1;                      // Gray bits (particle 0 is fixed)
   const int u = std::min(tb::kSweepU, nb);   // static bits of the kernel for this k
@@ -318,7 +330,15 @@ inline SweepPlan sweep_plan(int k, int64_t items, int c_override) {
   p.c = c;
   const int chunk_bits = nb - c;                      // log2(chunks per item)
   const int wave_bits = std::max(0, chunk_bits - 6);  // log2(waves at one chunk per lane)
-  const int wpi_bits = std::min(wave_bits, 13);
+  int wpi_bits = std::min(wave_bits, 13);
+  if (all_items && c_override <= 0) {
+    const auto cost = [&](int bits) {
+      return ((items << bits) + 1023) / 1024 *
+             ((((int64_t)1 << c) + kSweepSeedCodes) * ((int64_t)1 << (wave_bits - bits)) + kSweepWaveCodes);
+    };
+    for (int bits = wpi_bits - 1; bits >= 0; --bits)
+      if (100 * cost(bits) < (bits == 0 ? 95 : 90) * cost(wpi_bits)) wpi_bits = bits;
+  }
   p.wpi = 1 << wpi_bits;
   p.iters = 1 << (wave_bits - wpi_bits);
   return p;
@@ -407,7 +427,8 @@ tb::SweepSource gathered(const tb::cd *Vt, int ldv, int64_t item_stride) {
 }
 
 // Partial sums only: partial[(item * wpi + w) * k + nu], w < *wpi. A consumer that sums
-// them in w order gets the same minors as run_sweep with up to kReduceInOrder of them.
+// them in w order gets the same minors as run_sweep with the same plan and up to kReduceInOrder
+// of them.
 int32_t run_sweep_partial(int k, const tb::cd *Vt, int ldv, int64_t item_stride,
                           const int *item_map, const int *item_count, int items, int c_override,
                           tb::cd *partial, int *wpi, hipStream_t s) {
@@ -421,7 +442,7 @@ int32_t run_sweep_partial(int k, const tb::cd *Vt, int ldv, int64_t item_stride,
 constexpr int kReduceInOrder = 32;
 int32_t run_sweep(int k, const tb::SweepSource &src, int items, int c_override, tb::cd *partial,
                   const int *in_mult, int in_max, tb::cd *minors, hipStream_t s) {
-  const SweepPlan p = sweep_plan(k, items, c_override);
+  const SweepPlan p = sweep_plan(k, items, c_override, true);
   const int outs = in_mult ? in_max : k;
   // One wave per item and no empty slot: the sums are the minors, with nothing to add or place
   // (one launch of two saved: 14.6 us a call instead of 17.4 up to k = 12).
