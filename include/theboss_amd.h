@@ -319,7 +319,8 @@ int32_t tb_gccb_status(const void *workspace, void *stream);
  * tb_outcome_histogram64 sets 64-bit counts and outside (optional) instead; they need no
  * clearing. The workspace, of tb_outcome_histogram64_workspace_size bytes (0: none needed;
  * at most 32 MiB of ranks and the table of their runs), lets a large call count without
- * atomics on memory; without it (NULL, or fewer bytes) the counts are the same, slower.
+ * atomics on memory; without it (NULL, fewer bytes, or not on a multiple of 4 bytes) the
+ * counts are the same, slower.
  * ------------------------------------------------------------------------------- */
 int64_t tb_outcome_count(int32_t n, int32_t m, int32_t losses);
 int32_t tb_outcome_histogram(const int32_t *samples, int32_t ld, int32_t samples_n, int32_t m,
