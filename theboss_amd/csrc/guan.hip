@@ -231,11 +231,10 @@ __device__ __forceinline__ void guan_items(const cd *__restrict__ U, int ldu,
                                            const int *__restrict__ out_mult, int out_max,
                                            const int *__restrict__ in_modes,
                                            const int *__restrict__ in_mult, int in_max, int batch,
-                                           int n_in, int formula, int mode, int b0,
+                                           int n_in, int formula, int mode, int b0, int lane,
                                            const int *__restrict__ done, char *smem,
                                            cd *__restrict__ out) {
   constexpr int W = 64 / IPW;  // lanes per item in a packed wave
-  const int lane = threadIdx.x;
   const int g = lane / W, l = lane % W;
   const int b = b0 + g;
   bool live = b < batch;
@@ -371,47 +370,85 @@ __global__ __launch_bounds__(64) void guan_kernel(const cd *__restrict__ U, int 
                                                   cd *__restrict__ out) {
   extern __shared__ char smem[];
   guan_items<JB, IPW, false>(U, ldu, out_modes, out_mult, out_max, in_modes, in_mult, in_max, batch,
-                             1, formula, mode, (int)blockIdx.x * IPW, nullptr, smem, out);
+                             1, formula, mode, (int)blockIdx.x * IPW, threadIdx.x, nullptr, smem, out);
 }
 
-// All-pairs form. AFTER: the launch follows the subset recurrence, which has usually done every
-// row, so its grid is bounded and each block loops over its share of the items; it reads the
-// flags of 64 turns at once, a lane each, and skips the turns whose rows are all done.
-template <int JB, int IPW, bool AFTER>
+// All-pairs form.
+template <int JB, int IPW>
 __global__ __launch_bounds__(64) void guan_outer_kernel(
     const cd *__restrict__ U, int ldu, const int *__restrict__ out_modes,
     const int *__restrict__ out_mult, int out_max, const int *__restrict__ in_modes,
     const int *__restrict__ in_mult, int in_max, int batch, int n_in, int formula,
-    const int *__restrict__ done, cd *__restrict__ out) {
+    cd *__restrict__ out) {
   extern __shared__ char smem[];
-  if constexpr (!AFTER) {
-    guan_items<JB, IPW, true>(U, ldu, out_modes, out_mult, out_max, in_modes, in_mult, in_max,
-                              batch, n_in, formula, 0, (int)blockIdx.x * IPW, nullptr, smem, out);
-  } else {
-    const int64_t stride = (int64_t)gridDim.x * IPW;
-    uint64_t todo = 0, whole = 0;  // of 64 turns: any, and every row is left
-    int64_t b0 = (int64_t)blockIdx.x * IPW;
-    for (int turn = 0; b0 < batch; b0 += stride, ++turn) {
-      if ((turn & 63) == 0) {
-        const int64_t own = b0 + threadIdx.x * stride;
-        bool left = false, all = true;
-        if (own < batch) {
-          const int j1 = (int)(min(own + IPW, (int64_t)batch) - 1) / n_in;
-          for (int j = (int)own / n_in; j <= j1; ++j) {
-            const bool l = done[j] == 0;
-            left |= l;
-            all &= l;
-          }
-        }
-        todo = __ballot(left);
-        whole = __ballot(all);
+  guan_items<JB, IPW, true>(U, ldu, out_modes, out_mult, out_max, in_modes, in_mult, in_max, batch,
+                            n_in, formula, 0, (int)blockIdx.x * IPW, threadIdx.x, nullptr, smem, out);
+}
+
+struct GuanAfterArgs {
+  const cd *U;
+  int ldu, out_max;
+  const int *out_modes, *out_mult, *in_modes, *in_mult;
+  int in_max, batch, n_in, formula;
+  int *done;
+  int classes, grab;  // the counters, and how many turns to take from one at once
+  cd *out;
+};
+
+// All-pairs form after the subset recurrence, which has usually done every row, so the grid is
+// bounded and each block looks at its share of the turns (IPW items each), 64 at once, a lane each,
+// and walks those with a row left. Where the recurrence had no lattice and did nothing
+// (subset_rows_kernel then leaves counters in place of the flags), the blocks take a few turns at a
+// time from the counter of their class: with a fixed share each, some were still walking when most
+// had nothing left (8M pairs of k = 8 on 13 modes: 14.0 ms walked at once, 17.9 ms with 8192 blocks
+// of a fixed share, 10.8M pairs now 19.1 ms against 19.0).
+//
+// The walk needs nearly all SGPRs, so nothing of the loop stays in one while a turn is walked: the
+// arguments are read again from the kernel's argument segment, the turns stay with their lanes.
+// With the loop's state and the arguments held there, 19 to 57 of them went through VGPR lanes in
+// the walk, and the launch that finds 1.0M pairs done took 5 us instead of 3.
+template <int JB, int IPW>
+__global__ __launch_bounds__(64) void guan_after_kernel(GuanAfterArgs) {
+  extern __shared__ char smem[];
+  using ArgsPtr = const __attribute__((address_space(4))) GuanAfterArgs *;
+  int base = 0;            // turns of this block's share that are behind it
+  int own = 0, flags = 0;  // the lane's turn: first item; 1 a row of it is left, 2 all are
+  for (;;) {
+    ArgsPtr a = (ArgsPtr)__builtin_amdgcn_kernarg_segment_ptr();
+    int lane = threadIdx.x;
+    asm volatile("" : "+s"(a), "+v"(base), "+v"(lane));
+    const int n_in = a->n_in, batch = a->batch;
+    uint64_t left = __ballot(flags & 1);
+    if (left == 0) {
+      int *done = a->done;
+      const int in_vain = uniform_int(done[0]) < 0;
+      int64_t t = blockIdx.x + (int64_t)(base + lane) * gridDim.x;
+      base += 64;
+      if (in_vain) {
+        const int classes = a->classes, grab = a->grab, mine = blockIdx.x % classes;
+        int next = 0;
+        if (lane == 0) next = atomicAdd(done + mine * kSubCounterStride, grab) - INT32_MIN;
+        t = lane < grab ? mine + (int64_t)classes * (uniform_int(next) + lane) : (int64_t)batch;
       }
-      if (!((todo >> (turn & 63)) & 1)) continue;
-      guan_items<JB, IPW, true>(U, ldu, out_modes, out_mult, out_max, in_modes, in_mult, in_max,
-                                batch, n_in, formula, 0, (int)b0,
-                                (whole >> (turn & 63)) & 1 ? nullptr : done, smem, out);
-      __syncthreads();  // the next items reuse the LDS blocks
+      own = (int)min(t * IPW, (int64_t)batch);
+      if (uniform_int(own) >= batch) break;  // lane 0 has the first of them
+      flags = 0;
+      if (own < batch && in_vain) flags = 3;
+      if (own < batch && !in_vain) {
+        const int j1 = (int)(min((int64_t)own + IPW, (int64_t)batch) - 1) / n_in;
+        flags = 2;
+        for (int j = own / n_in; j <= j1; ++j) flags = done[j] == 0 ? flags | 1 : flags & ~2;
+      }
+      left = __ballot(flags & 1);
+      if (left == 0) continue;
     }
+    const int at = __ffsll((unsigned long long)left) - 1;
+    const int f = __builtin_amdgcn_readlane(flags, at), b0 = __builtin_amdgcn_readlane(own, at);
+    if (lane == at) flags = 0;
+    guan_items<JB, IPW, true>(a->U, a->ldu, a->out_modes, a->out_mult, a->out_max, a->in_modes,
+                              a->in_mult, a->in_max, batch, n_in, a->formula, 0, b0, lane,
+                              f & 2 ? nullptr : a->done, smem, a->out);
+    __syncthreads();  // the next items reuse the LDS blocks
   }
 }
 
@@ -431,14 +468,19 @@ size_t guan_lds_bytes(int out_max, int in_max, int mode, int ipw) {
 }
 
 // n_in > 0: the all-pairs form over batch = n_out * n_in items (mode 0 only); done (may be
-// null): output rows already written. Those launches use a bounded grid, since the walk is
-// then the exception. 1.0M pairs all done: 5 us, 12 when each turn read its own flags and 27 as
-// 126,000 one-wave blocks. Nothing done, 90,000 pairs of k = 8 after an attempt in vain: 201 us,
-// 232 with half the blocks, 192 without the attempt.
-constexpr int kGuanAfterRecurrenceBlocks = 8192;
+// null): output rows already written, or the counters of a recurrence that did nothing. Those
+// launches use a bounded grid, no fewer waves than the CUs hold at once (1.0M pairs all done took
+// 27 us as 126,000 one-wave blocks). An attempt in vain costs 7 to 30 us in all: 90,000 pairs of
+// k = 6 60 -> 70 us, of k = 8 201 -> 210, 1.0M of k = 3 168 -> 192, of k = 8 1805 -> 1830.
+constexpr int kGuanAfterBlocks = 4096;
+// Turns of short items that a block takes at once: 64 counters pass one block every 30 ns each.
+int guan_grab(int turns, int slots) {
+  return slots > 6 ? 1 : std::min(std::max(turns >> 15, 1), 8);
+}
 int32_t run_guan(const tb::cd *U, int ldu, const int *out_modes, const int *out_mult, int out_max,
                  const int *in_modes, const int *in_mult, int in_max, int batch, int formula,
-                 int mode, tb::cd *out, hipStream_t s, int n_in = 0, const int *done = nullptr) {
+                 int mode, tb::cd *out, hipStream_t s, int n_in = 0, int *done = nullptr,
+                 int counters = 0) {
   const bool outer = n_in > 0;
   // slot capacities: an all-pairs item may enumerate either side
   const int ecap = outer ? std::max(in_max, out_max) : in_max;
@@ -461,14 +503,15 @@ int32_t run_guan(const tb::cd *U, int ldu, const int *out_modes, const int *out_
   do {                                                                                        \
     const int blocks = (batch + IPW - 1) / IPW;                                               \
     if (outer && done)                                                                        \
-      hipLaunchKernelGGL((tb::guan_outer_kernel<JB, IPW, true>),                              \
-                         dim3(std::min(blocks, kGuanAfterRecurrenceBlocks)), dim3(64), LDS, s, \
-                         U, ldu, out_modes, out_mult, out_max, in_modes, in_mult, in_max,     \
-                         batch, n_in, formula, done, out);                                    \
+      hipLaunchKernelGGL((tb::guan_after_kernel<JB, IPW>),                                    \
+                         dim3(std::min(blocks, kGuanAfterBlocks)), dim3(64), LDS, s,          \
+                         tb::GuanAfterArgs{U, ldu, out_max, out_modes, out_mult, in_modes,    \
+                                           in_mult, in_max, batch, n_in, formula, done,          \
+                                           std::min(blocks, counters), guan_grab(blocks, ecap), out}); \
     else if (outer)                                                                           \
-      hipLaunchKernelGGL((tb::guan_outer_kernel<JB, IPW, false>), dim3(blocks), dim3(64),     \
-                         LDS, s, U, ldu, out_modes, out_mult, out_max, in_modes, in_mult,     \
-                         in_max, batch, n_in, formula, nullptr, out);                         \
+      hipLaunchKernelGGL((tb::guan_outer_kernel<JB, IPW>), dim3(blocks), dim3(64), LDS, s, U, \
+                         ldu, out_modes, out_mult, out_max, in_modes, in_mult, in_max, batch, \
+                         n_in, formula, out);                                                 \
     else                                                                                      \
       hipLaunchKernelGGL((tb::guan_kernel<JB, IPW>), dim3(blocks), dim3(64), LDS, s, U, ldu,  \
                          out_modes, out_mult, out_max, in_modes, in_mult, in_max, batch,      \
@@ -521,10 +564,11 @@ extern "C" int32_t tb_guan_perm_batch(const tb_complex128 *U, int32_t ldu,
 
 namespace tbsub {
 bool attempt(int ldu, int out_max, int n_out, int in_max, int n_in);
+size_t flag_bytes(int n_out);
 size_t workspace(int n_out);
 int32_t run(const tb::cd *U, int ldu, const int *out_modes, const int *out_mult, int out_max,
             int n_out, const int *in_modes, const int *in_mult, int in_max, int n_in, int *done,
-            tb::cd *out, hipStream_t s);
+            int counters, tb::cd *out, hipStream_t s);
 }  // namespace tbsub
 
 extern "C" size_t tb_guan_outer_workspace_size(int32_t ldu, int32_t out_max, int32_t n_out,
@@ -564,19 +608,21 @@ extern "C" int32_t tb_guan_perm_outer_ws(const tb_complex128 *U, int32_t ldu,
     return tbh::fail(TB_ERANGE, "guan_outer: out_max=%d, in_max=%d: either side may be "
                      "enumerated, so both must be <= %d", out_max, in_max,
                      std::min(TB_GUAN_MAX_ROWS, TB_GUAN_MAX_COLS));
-  int *done = nullptr;
+  int *done = nullptr, counters = 0;
   if (workspace != nullptr && tbsub::attempt(ldu, out_max, n_out, in_max, n_in)) {
-    const size_t need = tbsub::workspace(n_out);
+    const size_t need = tbsub::flag_bytes(n_out);
     if (workspace_bytes < need)
       return tbh::fail(TB_EWORKSPACE, "guan_outer: workspace %zu bytes < required %zu",
                        workspace_bytes, need);
     done = (int *)workspace;
+    counters = (int)std::min<size_t>(tb::kSubCounters,
+                                     workspace_bytes / (sizeof(int) * tb::kSubCounterStride));
     const int32_t rc = tbsub::run((const tb::cd *)U, ldu, out_modes, out_mult, out_max, n_out,
-                                  in_modes, in_mult, in_max, n_in, done, (tb::cd *)out,
+                                  in_modes, in_mult, in_max, n_in, done, counters, (tb::cd *)out,
                                   (hipStream_t)stream);
     if (rc) return rc;
   }
   return tbg::run_guan((const tb::cd *)U, ldu, out_modes, out_mult, out_max, in_modes, in_mult,
                        in_max, n_out * n_in, formula, 0, (tb::cd *)out, (hipStream_t)stream, n_in,
-                       done);
+                       done, counters);
 }

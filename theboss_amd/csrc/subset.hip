@@ -342,7 +342,7 @@ __device__ __forceinline__ void subset_row(SubsetLds &S, const cd *__restrict__ 
 __global__ __launch_bounds__(256) void subset_rows_kernel(
     const int *__restrict__ in_modes, const int *__restrict__ in_mult, int in_max, int n_in,
     const cd *__restrict__ U, int ldu, const int *__restrict__ out_modes,
-    const int *__restrict__ out_mult, int out_max, int n_out, int *__restrict__ done,
+    const int *__restrict__ out_mult, int out_max, int n_out, int *__restrict__ done, int counters,
     cd *__restrict__ out) {
   __shared__ SubsetLds S;
   const int wave = threadIdx.x >> 6;
@@ -352,8 +352,9 @@ __global__ __launch_bounds__(256) void subset_rows_kernel(
   int64_t j = many ? blockIdx.x * 4 + wave : blockIdx.x;
   SubsetSlot slot = subset_slot(out_modes, out_mult, out_max, n_out, j);
   subset_plan(S, in_modes, in_mult, in_max, n_in, ldu);
-  if (!S.p.ok) {
-    for (int e = blockIdx.x * 256 + threadIdx.x; e < n_out; e += gridDim.x * 256) done[e] = 0;
+  if (!S.p.ok) {  // nothing is done: counters for the walk that follows, in place of the flags
+    if (blockIdx.x == 0 && (int)threadIdx.x < counters)
+      done[threadIdx.x * kSubCounterStride] = INT32_MIN;
     return;
   }
   const bool waves = many && 2 * S.p.width <= kSubWaveEntries;
@@ -390,14 +391,18 @@ bool attempt(int ldu, int out_max, int n_out, int in_max, int n_in) {
   return ((int64_t)n_out * n_in) << in_max >= kSubMinCodes;
 }
 
-size_t workspace(int n_out) { return (sizeof(int) * (size_t)n_out + 255) & ~(size_t)255; }
+// Bytes of the flags, the least a workspace may hold, and with all the counters.
+size_t flag_bytes(int n_out) { return (sizeof(int) * (size_t)n_out + 255) & ~(size_t)255; }
+size_t workspace(int n_out) {
+  return std::max(flag_bytes(n_out), sizeof(int) * tb::kSubCounters * tb::kSubCounterStride);
+}
 
 // 512 workgroups: two per CU, what their LDS allows.
 int32_t run(const tb::cd *U, int ldu, const int *out_modes, const int *out_mult, int out_max,
             int n_out, const int *in_modes, const int *in_mult, int in_max, int n_in, int *done,
-            tb::cd *out, hipStream_t s) {
+            int counters, tb::cd *out, hipStream_t s) {
   hipLaunchKernelGGL(tb::subset_rows_kernel, dim3(std::min(n_out, 512)), dim3(256), 0, s, in_modes,
-                     in_mult, in_max, n_in, U, ldu, out_modes, out_mult, out_max, n_out, done, out);
+                     in_mult, in_max, n_in, U, ldu, out_modes, out_mult, out_max, n_out, done, counters, out);
   return tbh::check_hip(hipGetLastError(), "subset_rows_kernel");
 }
 

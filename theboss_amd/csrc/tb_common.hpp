@@ -118,6 +118,11 @@ __device__ __forceinline__ double wave_allsum(double v) {
 
 __device__ __forceinline__ int uniform_int(int v) { return __builtin_amdgcn_readfirstlane(v); }
 
+// Counters that an all-pairs recurrence which did nothing leaves in place of the rows' flags, each
+// on a cache line of its own (in ints) and from INT32_MIN on: the walk that follows takes its work
+// from them.
+constexpr int kSubCounters = 64, kSubCounterStride = 32;
+
 }  // namespace tb
 
 // Host-side error channel (defined in capi.hip).
