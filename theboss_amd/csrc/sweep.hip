@@ -6,7 +6,9 @@ namespace tb {
 
 // Stages item `item` as Vs[nu][j] = V[nu][j]: copied from gathered columns, or gathered from U
 // by the item's slots (particles: the occupied input slots in order; rows: the output slots,
-// repeated by multiplicity; entries past either list are 0). lists: 2K - 1 ints of LDS.
+// repeated by multiplicity; entries past either list are 0). With fewer than K particles every
+// minor has a column of zeros, so the item is all 0: its minors are then exactly 0 at whatever slot
+// they are written. lists: 2K - 1 ints of LDS.
 template <int K>
 __device__ __forceinline__ void sweep_stage(const SweepSource &src, int item, cd *Vs, int *lists,
                                             int lane) {
@@ -31,6 +33,7 @@ __device__ __forceinline__ void sweep_stage(const SweepSource &src, int item, cd
     if (on && at < K) cols[at] = src.in_modes[q];
     base += __popcll(bal);
   }
+  const bool enough = base >= K;
   base = 0;
   for (int q0 = 0; q0 < src.out_max; q0 += 64) {
     const size_t q = (size_t)item * src.out_max + q0 + lane;
@@ -48,7 +51,7 @@ __device__ __forceinline__ void sweep_stage(const SweepSource &src, int item, cd
   for (int e = lane; e < K * R; e += 64) {
     const int nu = e / R, j = e - nu * R;
     const int row = rows[j], col = cols[nu];
-    Vs[e] = row >= 0 && col >= 0 ? src.U[(size_t)row * src.ldu + col] : cd{0.0, 0.0};
+    Vs[e] = enough && row >= 0 && col >= 0 ? src.U[(size_t)row * src.ldu + col] : cd{0.0, 0.0};
   }
 }
 
@@ -444,7 +447,8 @@ int32_t run_sweep(int k, const tb::SweepSource &src, int items, int c_override, 
                   const int *in_mult, int in_max, tb::cd *minors, hipStream_t s) {
   const SweepPlan p = sweep_plan(k, items, c_override, true);
   const int outs = in_mult ? in_max : k;
-  // One wave per item and no empty slot: the sums are the minors, with nothing to add or place
+  // One wave per item and no more slots than particles: the sums are the minors, with nothing to
+  // add or place (an item with an empty slot after all is short of a particle, so all 0)
   // (one launch of two saved: 14.6 us a call instead of 17.4 up to k = 12).
   const bool direct = p.wpi == 1 && outs == k;
   int32_t rc = dispatch_sweep(k, src, nullptr, nullptr, items, p, direct ? minors : partial, s);
