@@ -43,12 +43,16 @@ bool runs_fp32(int n, int precision) {
          (precision == TB_PREC_FP32_COLSUM && n <= TB_FP32_COLSUM_MAX_N);
 }
 
+// What the launches use: flags and partial sums.
+size_t glynn_launch_bytes(int n, int batch, int c_pref) {
+  return n <= 1 || batch <= 0 || n > TB_GLYNN_MAX_N ? 0 : tbgl_partial_bytes(n, batch, c_pref);
+}
+
+// What a caller's workspace has: room for an FP32 copy of the matrices as well, which the kernels
+// do without (they convert as they stage).
 size_t glynn_workspace_bytes(int n, int batch, int precision, int c_pref) {
-  if (n <= 1 || batch <= 0 || n > TB_GLYNN_MAX_N) return 0;
-  size_t bytes = tbgl_partial_bytes(n, batch, c_pref);
-  // room for an FP32 copy of the matrices, which callers may rely on; the kernels convert as
-  // they stage
-  if (n >= tbgl::kWideMinN && runs_fp32(n, precision))
+  size_t bytes = glynn_launch_bytes(n, batch, c_pref);
+  if (bytes > 0 && n >= tbgl::kWideMinN && runs_fp32(n, precision))
     bytes += align256((size_t)batch * n * n * sizeof(tb::cpx<float>));
   return bytes;
 }
@@ -58,9 +62,11 @@ extern "C" size_t tb_glynn_workspace_size(int32_t n, int32_t batch, int32_t prec
   return glynn_workspace_bytes(n, batch, precision, tbh::tuned(TB_TUNE_GLYNN, n, batch));
 }
 
-extern "C" int32_t tb_glynn_batch(const tb_complex128 *A, int32_t n, int32_t batch,
-                                  int64_t matrix_stride, int32_t precision, tb_complex128 *out,
-                                  void *workspace, size_t workspace_bytes, void *stream) {
+namespace {
+// copy_room: the workspace has to hold glynn_workspace_bytes, else what the launches use.
+int32_t glynn_batch(const tb_complex128 *A, int32_t n, int32_t batch, int64_t matrix_stride,
+                    int32_t precision, tb_complex128 *out, void *workspace, size_t workspace_bytes,
+                    bool copy_room, void *stream) {
   hipStream_t s = (hipStream_t)stream;
   if (batch < 0) return tbh::fail(TB_EINVAL, "glynn: batch=%d < 0", batch);
   if (batch == 0) return TB_OK;
@@ -81,7 +87,8 @@ extern "C" int32_t tb_glynn_batch(const tb_complex128 *A, int32_t n, int32_t bat
     return tbh::fail(TB_EINVAL, "glynn: matrix_stride=%lld < n*n=%d", (long long)matrix_stride,
                      n * n);
   const int c_pref = tbh::tuned(TB_TUNE_GLYNN, n, batch);  // read once: size check and launch agree
-  const size_t need = glynn_workspace_bytes(n, batch, precision, c_pref);
+  const size_t need = copy_room ? glynn_workspace_bytes(n, batch, precision, c_pref)
+                                : glynn_launch_bytes(n, batch, c_pref);
   if (need > 0 && (workspace == nullptr || workspace_bytes < need))
     return tbh::fail(TB_EWORKSPACE, "glynn: workspace %zu bytes < required %zu", workspace_bytes,
                      need);
@@ -98,11 +105,19 @@ extern "C" int32_t tb_glynn_batch(const tb_complex128 *A, int32_t n, int32_t bat
       runs_fp32(n, precision) ? tbgl::glynn_dispatch_f32 : tbgl::glynn_dispatch_f64;
   return dispatch(n, (const tb::cd *)A, matrix_stride, batch, o, partial, handled, wpm_cap, c_pref, s);
 }
+}  // namespace
+
+extern "C" int32_t tb_glynn_batch(const tb_complex128 *A, int32_t n, int32_t batch,
+                                  int64_t matrix_stride, int32_t precision, tb_complex128 *out,
+                                  void *workspace, size_t workspace_bytes, void *stream) {
+  return glynn_batch(A, n, batch, matrix_stride, precision, out, workspace, workspace_bytes, true,
+                     stream);
+}
 
 // ------------------------------------------------------------------------------------
-// tb_glynn_batch_noalloc: the same launches with their scratch memory (per-wave partial
-// sums, flags) in a static device array instead of a caller's
-// workspace, for callers that cannot allocate. `scratch` is the array's host-side name
+// tb_glynn_batch_noalloc: the same launches with their scratch memory (flags, per-wave partial
+// sums) in a static device array instead of a caller's workspace, for callers that cannot
+// allocate. `scratch` is the array's host-side name
 // only; its address on a device comes from hipGetSymbolAddress, taken once per device
 // with that device current, and that address is what the launches receive.
 // ------------------------------------------------------------------------------------
@@ -138,7 +153,7 @@ extern "C" int32_t tb_glynn_batch_noalloc(const tb_complex128 *A, int32_t n, int
   if (n > TB_GLYNN_MAX_N)
     return tbh::fail(TB_ERANGE, "glynn_noalloc: n=%d exceeds TB_GLYNN_MAX_N=%d", n, TB_GLYNN_MAX_N);
   const size_t need =
-      n < 0 ? 0 : glynn_workspace_bytes(n, batch, precision, tbh::tuned(TB_TUNE_GLYNN, n, batch));
+      n < 0 ? 0 : glynn_launch_bytes(n, batch, tbh::tuned(TB_TUNE_GLYNN, n, batch));
   if (need > (size_t)TB_GLYNN_NOALLOC_SCRATCH_BYTES)
     return tbh::fail(TB_ERANGE,
                      "glynn_noalloc: n=%d batch=%d needs %zu bytes of scratch, more than the "
@@ -149,8 +164,8 @@ extern "C" int32_t tb_glynn_batch_noalloc(const tb_complex128 *A, int32_t n, int
     const int32_t rc = scratch_on_current_device(&ws);
     if (rc) return rc;
   }
-  // The workspace entry point re-validates every argument and re-checks the size against
-  // the whole array, so a tuning entry changed in between cannot overrun it.
-  return tb_glynn_batch(A, n, batch, matrix_stride, precision, out, ws,
-                        ws ? (size_t)TB_GLYNN_NOALLOC_SCRATCH_BYTES : 0, stream);
+  // The common part validates every argument and re-checks the size against the whole array, so a
+  // tuning entry changed in between cannot overrun it.
+  return glynn_batch(A, n, batch, matrix_stride, precision, out, ws,
+                     ws ? (size_t)TB_GLYNN_NOALLOC_SCRATCH_BYTES : 0, false, stream);
 }
