@@ -127,3 +127,36 @@ def test_op_leaves_the_choice_to_the_device(T, oracle):
             assert np.max(np.abs(got - walk)) <= REL * np.max(np.abs(walk))
         same = np.array_equal(ops.guan_perm_outer(U, *outs, *ins).cpu().numpy(), walk)
         assert same == (len(top) == 13)  # the walk's values exactly, or the recurrence's
+
+
+@pytest.mark.parametrize("modes", [8, 13])
+def test_op_shares_no_scratch_between_calls(T, oracle, monkeypatch, modes):
+    """The scratch of a call is its own: threads share a stream, and a graph outlives the call."""
+    from theboss_amd import _device as D
+    from theboss_amd import ops
+
+    m, k = 14, 4
+    U = T.from_numpy(oracle.haar_unitary(m, 3)).cuda()
+    outs = on_device(T, random_rows(np.random.default_rng(1), 4200, m, k))
+    ins = on_device(T, substates((1,) * modes, k, m))
+    walk = ops.guan_perm_outer(U, *outs, *ins, common=False)
+    monkeypatch.setattr(D, "workspace", lambda *a: pytest.fail("the stream's workspace"))
+    want = ops.guan_perm_outer(U, *outs, *ins)
+    assert T.max(T.abs(want - walk)) <= REL * T.max(T.abs(walk))
+    side = T.cuda.Stream()
+    side.wait_stream(T.cuda.current_stream())
+    with T.cuda.stream(side):
+        ops.guan_perm_outer(U, *outs, *ins)
+        T.cuda.synchronize()
+        graph = T.cuda.CUDAGraph()
+        with T.cuda.graph(graph, stream=side):
+            got = ops.guan_perm_outer(U, *outs, *ins)
+    T.cuda.current_stream().wait_stream(side)
+    more = on_device(T, random_rows(np.random.default_rng(2), 9000, m, k))
+    for _ in range(3):
+        got.zero_()
+        ops.guan_perm_outer(U, *more, *ins)
+        graph.replay()
+        ops.guan_perm_outer(U, *more, *ins)
+        T.cuda.synchronize()
+        assert T.equal(got, want)

@@ -82,7 +82,9 @@ def guan_perm_outer(U, out_modes, out_mult, in_modes, in_mult, formula: int = L.
     need = 0
     if common or (common is None and (n_out * n_in) << min(in_max, 32) >= _OUTER_TRY_CODES):
         need = lib.tb_guan_outer_workspace_size(ldu, out_max, n_out, in_max, n_in)
-    ws = D.workspace(need, U.device) if need else None
+    # Of this call alone: what one launch leaves in it the next one reads, and another thread's call
+    # on the same stream may come between the two; a captured graph keeps it.
+    ws = T.empty(need, dtype=T.uint8, device=U.device) if need else None
     L.check(lib.tb_guan_perm_outer_ws(
         D.ptr(U), ldu, D.ptr(out_modes), D.ptr(out_mult), out_max, n_out,
         D.ptr(in_modes), D.ptr(in_mult), in_max, n_in, formula, D.ptr(out),
