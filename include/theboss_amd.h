@@ -185,7 +185,7 @@ int32_t tb_guan_perm_outer_ws(const tb_complex128 *U, int32_t ldu, const int32_t
  * over the n_in input rows (in_modes, in_mult) of tb_guan_perm_outer_ws, each of one particle
  * more than the prefixes; U is m x m.
  *   width      at least the most modes a prefix occupies, >= 1 (width + 1 and in_max as
- *              out_max and in_max of tb_guan_perm_outer)
+ *              out_max and in_max of tb_guan_perm_outer); a prefix that occupies more gets NaN
  *   common     nonzero: the input rows are known to have a small common state (as above)
  *   workspace  tb_gcca_layer_workspace_size bytes (holds the permanents; 0 = sizes refused) */
 size_t tb_gcca_layer_workspace_size(int32_t m, int32_t prefixes_n, int32_t width, int32_t in_max,

@@ -13,13 +13,15 @@
 namespace tb {
 
 // Row p m + o in compact form: the prefix's modes in mode order, one more particle where the
-// mode is o; a last slot for o itself, of multiplicity 0 where the prefix holds it. One
+// mode is o; a last slot for o itself, of multiplicity 0 where the prefix holds it. pmf[row] is
+// left 0, or NaN where the prefix occupies more modes than width and the row is not whole. One
 // thread per row; 4000 rows of 20 modes take 5 us, less than the copy of the rows (they were
 // formed on the host, 160 us, and uploaded).
 __global__ __launch_bounds__(256) void gcca_rows_kernel(const int *__restrict__ prefixes, int m,
                                                         int64_t rows, int width,
                                                         int *__restrict__ modes,
-                                                        int *__restrict__ mult) {
+                                                        int *__restrict__ mult,
+                                                        double *__restrict__ pmf) {
   const int64_t row = (int64_t)blockIdx.x * 256 + threadIdx.x;
   if (row >= rows) return;
   const int64_t p = row / m;
@@ -29,17 +31,21 @@ __global__ __launch_bounds__(256) void gcca_rows_kernel(const int *__restrict__ 
   int at = 0;
   for (int j = 0; j < m; ++j) {
     const int c = prefix[j];
-    if (c > 0 && at < width) {
-      mo[at] = j;
-      mu[at++] = c + (j == o);
+    if (c > 0) {
+      if (at < width) {
+        mo[at] = j;
+        mu[at] = c + (j == o);
+      }
+      ++at;
     }
   }
+  pmf[row] = at > width ? NAN : 0.0;
   for (; at < width; ++at) mo[at] = mu[at] = 0;
   mo[width] = o;
   mu[width] = prefix[o] > 0 ? 0 : 1;
 }
 
-// pmf[row] = sum_i w_i |perms[row][i]|^2, one wave per row; bound by the read of the
+// pmf[row] += sum_i w_i |perms[row][i]|^2, one wave per row; bound by the read of the
 // permanents.
 __global__ __launch_bounds__(256) void gcca_pmf_kernel(const cd *__restrict__ perms,
                                                        const double *__restrict__ weights,
@@ -54,7 +60,7 @@ __global__ __launch_bounds__(256) void gcca_pmf_kernel(const cd *__restrict__ pe
     sum = fma(weights[i], fma(v.re, v.re, v.im * v.im), sum);
   }
   sum = wave_sum(sum);
-  if ((threadIdx.x & 63) == 0) pmf[row] = sum;
+  if ((threadIdx.x & 63) == 0) pmf[row] += sum;
 }
 
 }  // namespace tb
@@ -114,7 +120,7 @@ extern "C" int32_t tb_gcca_layer_pmfs(const tb_complex128 *U, int32_t m, const i
   tb_complex128 *perms = (tb_complex128 *)ws;
   int *modes = (int *)(ws + g.modes), *mult = (int *)(ws + g.mult);
   hipLaunchKernelGGL(tb::gcca_rows_kernel, dim3((unsigned)((rows + 255) / 256)), dim3(256), 0, s,
-                     prefixes, m, rows, width, modes, mult);
+                     prefixes, m, rows, width, modes, mult, pmf);
   if (const int32_t rc = tbh::check_hip(hipGetLastError(), "gcca_rows_kernel")) return rc;
   if (const int32_t rc = tb_guan_perm_outer_ws(U, m, modes, mult, width + 1, (int32_t)rows, in_modes,
                                                in_mult, in_max, n_in, formula, perms,

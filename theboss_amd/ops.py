@@ -96,8 +96,8 @@ def gcca_layer_pmfs(U, prefixes, width: int, in_modes, in_mult, weights,
                     formula: int = L.TB_FORMULA_RYSER, common: bool = False):
     """The layers of P prefixes (P x m occupations, int32) on the m x m matrix U: a (P, m)
     tensor of sum_i weights[i] |perm(U[prefix_p + e_o, s_i])|^2 over the input rows s_i of
-    guan_perm_outer. `width` is the most modes a prefix occupies (at least 1); `common` as in
-    guan_perm_outer."""
+    guan_perm_outer. `width` is the most modes a prefix occupies (at least 1; the layers of a
+    prefix that occupies more are NaN); `common` as in guan_perm_outer."""
     T = D.require_gpu()
     U, prefixes = _c128(U, "U"), _i32(prefixes, "prefixes")
     in_modes, in_mult = _i32(in_modes, "in_modes"), _i32(in_mult, "in_mult")
