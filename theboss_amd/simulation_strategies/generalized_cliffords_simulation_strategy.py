@@ -191,10 +191,11 @@ class GeneralizedCliffordsSimulationStrategy(SimulationStrategyInterface):
         calc = self._bs_permanent_calculator
         sums = perms = None
         if hasattr(calc, "compute_layer_pmfs"):
-            if k not in self._layer_inputs:   # uploaded once per k
-                self._layer_inputs[k] = calc.layer_inputs(S, weights / norm)
-            if self._layer_inputs[k] is not None:
-                sums = calc.compute_layer_pmfs(self._layer_inputs[k], prefixes)
+            key = (k, D.device())
+            if key not in self._layer_inputs:   # uploaded once per k and device
+                self._layer_inputs[key] = calc.layer_inputs(S, weights / norm)
+            if self._layer_inputs[key] is not None:
+                sums = calc.compute_layer_pmfs(self._layer_inputs[key], prefixes)
         outputs = prefixes[:, None, :] + np.eye(m, dtype=np.int64)[None, :, :]   # P x m x m
         if sums is not None:    # device tensor P x m
             return outputs, sums.cpu().numpy()
