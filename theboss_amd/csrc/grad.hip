@@ -492,6 +492,11 @@ struct GradPlan {
 // (measured: 0.83 with one, 0.97 with two) and the share of a chunk left after its seed and
 // its end, which cost about 10 steps (n = 20, 64 matrices: 2^6 443 us, 2^7 411, 2^8 398,
 // 2^9 396, 2^10 405, 2^11 474). A tuned c (c_pref > 0) replaces that choice.
+//
+// A workgroup writes n^2 partial sums, so with many of them the groups walk several chunks each and
+// the partials stay below 2^16 n^2 (n = 30, 1000 matrices: 0.9 GB, not 110). That many groups are
+// 64 rounds or more of the resident waves.
+constexpr int64_t kGradMaxGroups = 1 << 16;
 inline GradPlan grad_plan(int n, int batch, int c_pref) {
   GradPlan p{};
   const int nb = n - 1, lb = tb::grad_lb(n), u = tb::grad_u(n), wfull = tb::grad_wbits(n);
@@ -515,7 +520,8 @@ inline GradPlan grad_plan(int n, int batch, int c_pref) {
   p.c = c;
   const int wave_bits = nb - c - lb;  // log2 of the waves per matrix at one chunk per lane group
   p.wb = std::min(wave_bits, wfull);
-  const int wg_bits = std::min(wave_bits - p.wb, 13);
+  int wg_bits = std::min(wave_bits - p.wb, 13);
+  while (wg_bits > 0 && ((int64_t)batch << wg_bits) > kGradMaxGroups) --wg_bits;
   p.wpi = 1 << wg_bits;
   p.iters = 1 << (wave_bits - p.wb - wg_bits);
   return p;
