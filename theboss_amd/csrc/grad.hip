@@ -40,6 +40,10 @@
 // kept per wave: at such a flip the wave sums T_j over its code lanes (transposed, so
 // that each lane ends with one value) and adds it to the row's sums in LDS. Bits above the
 // chunk contribute delta_i T_j at the chunk end.
+//
+// Infinities and NaN. Row i of the result does not depend on row i of the matrix, but every
+// column sum holds it. Rows with such an entry are walked as zeros, and the other rows of the
+// result, which depend on them, are NaN.
 #include <algorithm>
 #include <cmath>
 
@@ -167,6 +171,22 @@ __device__ __forceinline__ void dpp_ready(Bcast<C> &b) {
     asm volatile("s_nop 1" : "+v"(b.v[0]), "+v"(b.v[Bcast<C>::P - 1]));
 }
 
+// The rows of the matrix in Ms with an infinite or NaN entry, a bit each, and zeros in their place.
+// Called by the workgroup where there is one.
+template <int N, int NP>
+__device__ __attribute__((noinline)) void grad_clear_rows(cd *Ms, uint64_t *bad) {
+  if (threadIdx.x == 0) {
+    uint64_t rows = 0;
+    for (int e = 0; e < N * NP; ++e)
+      if (!isfinite(Ms[e].re) || !isfinite(Ms[e].im)) rows |= 1ull << (e / NP);
+    *bad = rows;
+  }
+  __syncthreads();
+  for (int e = threadIdx.x; e < N * N; e += blockDim.x)
+    if ((*bad >> (e / N)) & 1ull) Ms[e / N * NP + e % N] = {0.0, 0.0};
+  __syncthreads();
+}
+
 // Workgroup = 2^wb waves of one matrix: chunk q = ((it wpi + wg) 2^wb + wave) 2^lb + code
 // lane. wpi workgroups per matrix; direct: wpi == 1 and the results go to grad and perm,
 // otherwise to partial[(b wpi + wg)][n][n].
@@ -184,13 +204,25 @@ __attribute__((amdgpu_waves_per_eu(2))) void grad_kernel(
   const int b = blockIdx.x / wpi, wg = blockIdx.x - b * wpi;
   cd *acc = smem + (size_t)N * NP * (1 + wave);  // this wave's sums, [N][NP]
   const cd *src = A + (size_t)b * mstride;
+  __shared__ uint64_t bad;  // set where `odd` is, per wave: an entry that is not finite
+  __shared__ int odd[4];
+  bool finite = true;
   for (int e = threadIdx.x; e < N * NP; e += blockDim.x) {
     const int i = e / NP, j = e - i * NP;
     // a padding column's half sum is 1: 2 in the fixed row, 0 in the others
-    Ms[e] = j < N ? src[i * N + j] : cd{i == NB ? 2.0 : 0.0, 0.0};
+    const cd v = j < N ? src[i * N + j] : cd{i == NB ? 2.0 : 0.0, 0.0};
+    Ms[e] = v;
+    finite &= isfinite(v.re) && isfinite(v.im);
   }
   for (int e = lane; e < N * NP; e += 64) acc[e] = {0.0, 0.0};
+  odd[wave] = __any(!finite);
   __syncthreads();
+  const auto any_odd = [&] {
+    int any = odd[0];
+    for (int w = 1; w < waves; ++w) any |= odd[w];
+    return uniform_int(any) != 0;
+  };
+  if (any_odd()) grad_clear_rows<N, NP>(Ms, &bad);
   const int far = (lane ^ 32) << 2;         // ds_bpermute address of lane ^ 32
   const int blk_col = (lane >> LB) * C;     // first column of the lane's block
   const cd *M = Ms + blk_col;
@@ -369,13 +401,15 @@ __attribute__((amdgpu_waves_per_eu(2))) void grad_kernel(
   __syncthreads();
   const cd *sums = smem + (size_t)N * NP;
   const bool direct = wpi == 1;
+  const uint64_t cleared = any_odd() ? bad : 0;
   cd *dst = direct ? grad + (size_t)b * N * N : partial + (size_t)blockIdx.x * N * N;
   for (int e = threadIdx.x; e < N * N; e += blockDim.x) {
     const int i = e / N, j = e - i * N;
     cd v = sums[i * NP + j];
     for (int w = 1; w < waves; ++w) v = cadd(v, sums[(size_t)w * N * NP + i * NP + j]);
+    if (cleared != 0 && cleared != 1ull << i) v = {NAN, NAN};
     if (direct && i == 0) {  // perm: the Laplace expansion along row 0
-      const cd t = cmul(Ms[j], v);
+      const cd t = cmul((cleared & 1ull) != 0 ? src[j] : Ms[j], v);
       Ms[j] = t;
     }
     if (direct && conj) v.im = -v.im;
