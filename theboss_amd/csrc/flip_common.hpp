@@ -233,36 +233,9 @@ __device__ __forceinline__ void pair_acc2(double &xr, double &xi, double &yr, do
   cmul_acc<SIGN>(yr, yi, fold_chain<-1, 0, H>(ur, ui), fold_chain<-1, H, N>(ur, ui));
 }
 
-// 1 / c for c != 0, with c scaled by a power of two so that |c|^2 stays in range.
-__device__ __forceinline__ cd cinv_scaled(cd c) {
-  const int e = ilogb(fmax(fabs(c.re), fabs(c.im)));
-  const double cr = ldexp(c.re, -e), ci = ldexp(c.im, -e);
-  const double d = fma(cr, cr, ci * ci);
-  return {ldexp(cr / d, -e), ldexp(-ci / d, -e)};
-}
-
 // A pair row must have every entry above 2^-16 of the matrix's largest entry (squared
 // magnitudes compared): far from zero, its quotients stay in range and well rounded.
 constexpr double kPairMinRel2 = 0x1p-32;
-
-// c = prod_j v[j] * 2^-J (J values) as a mantissa and a power of two, renormalised after
-// every factor so that no partial product over- or underflows.
-__device__ __forceinline__ void prod_half_scaled(const cd *v, int J, cd &mant, int &e2) {
-  cd k = {1.0, 0.0};
-  int ke = -J;
-  for (int j = 0; j < J; ++j) {
-    k = cmul(k, v[j]);
-    const double a = fmax(fabs(k.re), fabs(k.im));
-    if (a > 0.0) {
-      const int e = ilogb(a);
-      k.re = ldexp(k.re, -e);
-      k.im = ldexp(k.im, -e);
-      ke += e;
-    }
-  }
-  mant = k;
-  e2 = ke;
-}
 
 // ------------------------------------------------------------------------------------
 // Sums of several values over 2^LB lanes (LB = 4: each row of 16 lanes; 5: the rows 0, 1 and
