@@ -997,8 +997,8 @@ constexpr int glynn_reg_rows() {
 // The paired FP32 kernel: 2 static Gray bits, static row SR in SGPRs (row 1 by default)
 // and the other in VGPRs. A SIMD issues two FP32 instructions per 4-cycle slot only from
 // two different waves, so the kernel wants 4 resident waves (<= 128 VGPRs): row 1 in
-// SGPRs and, at n = 19..21, the first values of row 2 too (glynn_f32_pair_s2) give 4 waves
-// up to n = 21 and 3 at n = 22, 23. 3 static bits with every row in VGPRs need 217 VGPRs
+// SGPRs and, at n = 19..22, the first values of row 2 too (glynn_f32_pair_s2) give 4 waves
+// up to n = 22 and 3 at n = 23. 3 static bits with every row in VGPRs need 217 VGPRs
 // (2 waves) at n = 20. SR = 2 (row 2 in SGPRs, so the row-1 flips dual-issue) fits 4
 // waves at every n and measured the same time at n = 20 and 5% slower at n = 23: at
 // n = 20 the launch runs the clock down to 1.9 GHz whichever rows dual-issue.
@@ -1042,8 +1042,9 @@ constexpr bool glynn_paired() {
 }
 // Static super-step bits of the paired walk and its rows in broadcast form (rows 1..B).
 // Static super-step bits: 3 at every paired n (a block of 8 pairs between block-start
-// flips; 166..256 VGPRs, no spills). Measured against 2 bits below n = 25: 3.7% faster at
-// n = 16 and 3.6-4% at n = 20..24.
+// flips; 172..256 VGPRs; n = 23 and 24 spill 1 and 10 values, of which the walk reloads one a
+// block, and are 1-7% faster than the three launches without spills were). Measured against
+// 2 bits below n = 25: 3.7% faster at n = 16 and 3.6-4% at n = 20..24.
 template <int N>
 constexpr int glynn_pair_u() {
   return 3;
@@ -1083,8 +1084,11 @@ constexpr int glynn_wave_slots() {
   }
   return 2;
 }
-// Waves per SIMD of the plan's bound on C: the residency, but 3 at n = 22, which with 4 takes
-// C = 6 instead of 7 for 100 matrices (547 us instead of 482).
+// Waves per SIMD of the plan's bound on C: the residency, but 3 at n = 22, the one size whose fourth
+// wave came with the present register count. With 3 no batch measured is slower than at 3 resident
+// waves. With 4 some are 5-20% faster (8, 16, 150, 500 matrices: 67 -> 54, 102 -> 88, 736 -> 685,
+// 2255 -> 2152 us) and some 12-23% slower (4, 24, 100: 31 -> 38, 126 -> 145, 493 -> 556), as the
+// plan's score takes 2^6 ranks for 2^7.
 template <int N, typename F>
 constexpr int glynn_plan_slots() {
   return N == 22 ? std::min(glynn_wave_slots<N, F>(), 3) : glynn_wave_slots<N, F>();

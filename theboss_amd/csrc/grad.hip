@@ -61,7 +61,8 @@ constexpr int grad_np(int n) { return grad_l(n) * grad_cols(n); }
 // log2 of the code lanes of a wave.
 constexpr int grad_lb(int n) { return grad_l(n) == 4 ? 4 : 5; }
 // Static Gray bits: the more, the fewer block starts and their code-lane sums, as far as the
-// 2C correctors of each fit 256 VGPRs (n = 20: 0.384 ms with 4, 0.396 with 3, 0.424 with 2).
+// 2C correctors of each fit 256 VGPRs, but for 2 to 12 values at n = 15..18 and 29..32 that are
+// reloaded once a chunk (n = 20: 0.384 ms with 4, 0.396 with 3, 0.424 with 2).
 // At n <= 8 a lane group walks 2^3 codes or fewer: 2 bits and 3 take the same time within 4%.
 constexpr int grad_u(int n) {
   const int u = grad_l(n) == 2 ? (n <= 16 ? 4 : 3) : n <= 8 ? 2 : n <= 32 ? 4 : 2;

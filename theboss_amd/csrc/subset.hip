@@ -10,8 +10,10 @@
 // loop of generalized_cliffords_simulation_strategy.py:162-171 over :224-247 calls
 // compute_permanent per pair). For n input modes of one particle each the lattice costs
 // sum_{l <= k} l C(n, l) complex multiply-adds per output row, against C(n, k) 2^k codes of k
-// multiplies: n = 10, k = 5: 2560 against 40,000. No term cancels another by construction, so the
-// result is at least as accurate as the alternating sums.
+// multiplies: n = 10, k = 5: 2560 against 40,000. No inclusion-exclusion signs enter: the terms
+// are products of entries, so the error is bounded by the permanent of the entries' moduli, where
+// the alternating sums start from terms up to 2^k times larger (not by |perm|: entries of any
+// phase still cancel). Measured on 200 prefixes of 10 modes, k = 5: 2.7e-16 against 2.8e-15.
 //
 // What bounds it (GCC-A layer of 200 prefixes x 20 outputs x C(10, 5) inputs, 1.0M pairs: 32 us a
 // call, 4 of them the 16 MB written; the walk 351): a workgroup first builds the lattice from
@@ -21,8 +23,7 @@
 // eight waves of a CU sharing its LDS reads. Slots loaded all at once and a row ahead, levels
 // unrolled, and ranks that share their low bits: 42 us before, with the walk's flags (below); 12
 // modes, k = 6, 1200 rows: 77 -> 54. The Guan walk follows in stream order over the rows whose
-// done flag is 0: all of them when the lattice is too large, or a row whose particle number
-// differs.
+// done flag is 0, whose particle number differs, or over all of them when the lattice is too large.
 #include <algorithm>
 
 #include "tb_common.hpp"

@@ -359,7 +359,9 @@ inline size_t sweep_pair_lds_bytes(int k, int c) {
 }
 // Sizes that run the paired sweep (with a chunk holding the static block plus the pair
 // bit), at 2 waves per SIMD: up to k = 21 with five particles in broadcast form, from
-// k = 22 with the three static ones (196..249 VGPRs, no spills). Five broadcast particles
+// k = 22 with the three static ones (206..256 VGPRs; 1, 3 and 4 values are spilled around the
+// walk at k = 21, 30 and 31, and the SGPRs that staging needs, 24 bytes a lane at every k; k = 30
+// and 31 are 3-7% faster than when nothing was spilled). Five broadcast particles
 // spill from k = 22, and at one wave per SIMD the compiler parks broadcast columns in
 // AGPRs and reloads them right before their DPP reads, a hazard that
 // tests/test_dpp_hazards.py looks for. k = 31 is the largest broadcast-column sweep.
