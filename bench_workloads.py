@@ -70,19 +70,19 @@ def clock_during(fn, seconds):
 
 
 class GuanFlops:
-    """Counts, inside the with-block, the multiplicity-aware algorithmic flops of every
+    """Counts, inside the with-block, the flops that a pair-by-pair Guan walk would take for every
     tb_guan_perm_batch, tb_guan_perm_outer and tb_gcca_layer_pmfs call the calculators make:
     per item (pair) prod_d (e_d + 1) Guan codes, each costing 2|T| + 6(sum t - 1) + 2 (|T| complex adds
     into the sums of the product side's distinct modes, sum t - 1 complex multiplies, the
     accumulation), with e the enumerated side's multiplicities and t the product side's. Calls
-    that take the subset recurrence are charged the same, the walk they replace.
+    that take the subset recurrence execute far fewer.
     The count is summed on the device and read once at the end."""
 
     def __enter__(self):
         T = D.torch()
         self._orig = ops.guan_perm_batch
         self._acc = T.zeros((), dtype=T.float64, device="cuda")
-        self.launches = 0
+        self.calls = 0
         self.items = 0
 
         def counted(U, out_modes, out_mult, in_modes, in_mult, formula=L.TB_FORMULA_RYSER):
@@ -90,7 +90,7 @@ class GuanFlops:
             distinct = (out_mult > 0).sum(dim=1).to(T.float64)
             parts = out_mult.sum(dim=1).to(T.float64)
             self._acc += (codes * (2 * distinct + 6 * (parts - 1) + 2)).sum()
-            self.launches += 1
+            self.calls += 1
             self.items += int(in_mult.shape[0])
             return self._orig(U, out_modes, out_mult, in_modes, in_mult, formula)
 
@@ -103,7 +103,7 @@ class GuanFlops:
             enum_s = codes_s[None, :] * (2 * dist_t[:, None] + 6 * (parts_t[:, None] - 1) + 2)
             enum_t = codes_t[:, None] * (2 * dist_s[None, :] + 6 * (parts_s[None, :] - 1) + 2)
             self._acc += T.where(codes_t[:, None] < codes_s[None, :], enum_t, enum_s).sum()
-            self.launches += 1
+            self.calls += 1
             self.items += int(out_mult.shape[0]) * int(in_mult.shape[0])
 
         self._orig_outer, self._orig_layer = ops.guan_perm_outer, ops.gcca_layer_pmfs
@@ -426,8 +426,8 @@ def exact(checker, m=12, n=6, eta=0.5):
         return np.asarray(calc.calculate_distribution())
 
     T = D.torch()
-    # warm-up run (library, workspaces), which also counts the launches' flops: the
-    # distribution is deterministic, so the timed run makes the same launches, uncounted
+    # warm-up run (library, workspaces), which also counts the calls' pairs: the
+    # distribution is deterministic, so the timed run makes the same calls, uncounted
     with GuanFlops() as gf:
         run()
     T.cuda.synchronize()
@@ -441,7 +441,8 @@ def exact(checker, m=12, n=6, eta=0.5):
     dt_cpu = time.perf_counter() - t0
     return {"workload": f"exact uniform-loss distribution, m={m}, n={n}, eta={eta}",
             "outcomes": len(dist), "permanents": perms, "seconds": dt,
-            "guan_launches": gf.launches, "guan_items": gf.items, "guan_flops": gf.flops,
+            "guan_calls": gf.calls, "guan_pairs": gf.items,
+            "walk_equivalent_flops": gf.flops,
             "permanents_per_s": perms / dt, "sum": float(dist.sum()),
             "max_abs_diff_vs_oracle": float(np.max(np.abs(dist - ref))),
             "cpu_baseline": {"value": perms / dt_cpu, "unit": "permanents/s", "cores": 1,
@@ -455,7 +456,7 @@ def exact(checker, m=12, n=6, eta=0.5):
 
 def gcca(checker):
     """GCC-A, m=20, n=10 photons in modes 0..9, 200 samples, Ryser on the GPU (the
-    samples advance in lock-step: one all-pairs launch per particle number); plus one
+    samples advance in lock-step: one layer call per particle number); plus one
     10x10 permanent by Ryser and Glynn."""
     from theboss_amd.permanent_calculators import GPUGlynnGrayPermanentCalculator, GPURyserPermanentCalculator
     from theboss_amd.simulation_strategies import GeneralizedCliffordsSimulationStrategy
@@ -475,8 +476,8 @@ def gcca(checker):
     samples = strat.simulate(inp, S)
     D.torch().cuda.synchronize()
     dt = time.perf_counter() - t0
-    # the flop count, outside the timed run: the same draws again (same seed, so the same
-    # layers and launches) with the counter on every launch
+    # the count of pairs, outside the timed run: the same draws again (same seed, so the same
+    # layers and calls) with the counter on every call
     with GuanFlops() as gf:
         again = GeneralizedCliffordsSimulationStrategy(GPURyserPermanentCalculator(U),
                                                        rng=np.random.default_rng(0)).simulate(inp, S)
@@ -507,7 +508,8 @@ def gcca(checker):
                      f"{spent:.1f} s, scaled by this run's {len(strat.pmfs)} layers"}
     return {"workload": "GCC-A m=20 n=10, 200 samples (Ryser, lock-step layers)",
             "samples_per_s": S / dt, "seconds": dt, "layers_computed": len(strat.pmfs),
-            "guan_launches": gf.launches, "guan_items": gf.items, "guan_flops": gf.flops,
+            "guan_calls": gf.calls, "guan_pairs": gf.items,
+            "walk_equivalent_flops": gf.flops,
             "cpu_python_baseline": cpu, "gpu_vs_cpu_python": (S / dt) / cpu["value"],
             "ryser_vs_glynn_10x10_rel": abs(r - g) / abs(g),
             "all_samples_have_n_photons": all(sum(s_) == n for s_ in samples)}
@@ -605,16 +607,18 @@ def hist(checker):
     chunk = 1 << 20
     for i in range(S // chunk):
         ops.gccb_sample(U, parts, chunk, 100 + i, out=samples[i * chunk:(i + 1) * chunk])
-    # Reference result through the tensor wrapper, then the bare launch timed on
-    # preallocated counters (they accumulate over the repetitions).
+    # Reference result through the tensor wrapper, then the same entry timed on a preallocated
+    # workspace and counters.
     counts, outside = ops.outcome_histogram(samples, n)
     lib = L.load()
-    cnt = T.zeros(ops.outcome_count(n, m), dtype=T.int32, device=samples.device)
+    cnt = T.empty(ops.outcome_count(n, m), dtype=T.int64, device=samples.device)
+    need = lib.tb_outcome_histogram64_workspace_size(S, m, n, 0)
+    ws = T.empty(need, dtype=T.uint8, device=samples.device)
     stream = D.stream_ptr(samples.device)
-    t = _time(lambda: L.check(lib.tb_outcome_histogram(D.ptr(samples), m, S, m, n, 0, D.ptr(cnt),
-                                                       None, stream)), reps=3)
-    read = S * m * 4
-    algo = read + S * 4  # one 4-byte counter update per sample
+    t = _time(lambda: L.check(lib.tb_outcome_histogram64(D.ptr(samples), m, S, m, n, 0, D.ptr(cnt),
+                                                         None, D.ptr(ws), need, stream)), reps=3)
+    assert T.equal(cnt, counts)
+    algo = S * m * 4 + len(counts) * 8  # the samples read, the counters written
     cpu, cpu_py = _hist_cpu_lines(checker, samples[: 1 << 20].cpu().numpy(), counts, n, m, S)
     return {"workload": "outcome histogram, 2^24 samples, m=20, n=10 (20,030,010 outcomes)",
             "ms": t * 1e3, "samples_per_s": S / t,
