@@ -133,7 +133,8 @@ class GuanFlops:
 def sweep_small(checker):
     """The C&C minors sweep as the drop-in submatrices calculator and the plain GCC-B path
     launch it: one item, and small batches, at k = 20 (the batch-aware built-in plan cuts
-    the chunks until the launch has ~4096 waves, or 1024 below 2^5 Gray steps per lane)."""
+    the chunks until one a lane would make ~4096 waves, or 1024 below 2^5 Gray steps per lane;
+    a wave may walk several of them)."""
     T = D.torch()
     lib = L.load()
     k = 20
@@ -148,7 +149,7 @@ def sweep_small(checker):
         wpi = lib.tb_sweep_workspace_size(k, B) // (B * k * 16)
         fl = B * 2 ** (k - 1) * (10 * k - 12)
         got = out["m"].cpu().numpy()
-        rows.append({"batch": B, "waves_per_item": int(wpi), "waves": int(B * wpi),
+        rows.append({"batch": B, "waves_per_item_at_one_chunk": int(wpi),
                      "ms": t * 1e3, "tflops": fl / t / 1e12, "frac_fp64_peak": fl / t / FP64_PEAK,
                      "max_rel_diff_vs_one_item": float(np.max(np.abs(got - ref[None])) / np.max(np.abs(ref)))})
     return {"workload": "C&C minors sweep, k=20, batches 1..4096 (built-in plans)", "results": rows}
