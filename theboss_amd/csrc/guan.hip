@@ -406,7 +406,7 @@ struct GuanAfterArgs {
 // The walk needs nearly all SGPRs, so nothing of the loop stays in one while a turn is walked: the
 // arguments are read again from the kernel's argument segment, the turns stay with their lanes.
 // With the loop's state and the arguments held there, 19 to 57 of them went through VGPR lanes in
-// the walk, and the launch that finds 1.0M pairs done took 5 us instead of 3.
+// the walk, and the launch that finds 1.0M pairs done took 5.4 us instead of 4.0.
 template <int JB, int IPW>
 __global__ __launch_bounds__(64) void guan_after_kernel(GuanAfterArgs) {
   extern __shared__ char smem[];

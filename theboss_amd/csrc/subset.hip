@@ -15,7 +15,7 @@
 // the alternating sums start from terms up to 2^k times larger (not by |perm|: entries of any
 // phase still cancel). Measured on 200 prefixes of 10 modes, k = 5: 2.7e-16 against 2.8e-15.
 //
-// What bounds it (GCC-A layer of 200 prefixes x 20 outputs x C(10, 5) inputs, 1.0M pairs: 32 us a
+// What bounds it (GCC-A layer of 200 prefixes x 20 outputs x C(10, 5) inputs, 1.0M pairs: 30 us a
 // call, 4 of them the 16 MB written; the walk 351): a workgroup first builds the lattice from
 // the input rows, 19,000 cycles of latency (in LDS, for itself: a plan kernel with predecessor
 // lists in global memory took 20 us more per call); then a wave per output row walks the levels

@@ -33,7 +33,8 @@ __device__ __forceinline__ void sweep_stage(const SweepSource &src, int item, cd
     if (on && at < K) cols[at] = src.in_modes[q];
     base += __popcll(bal);
   }
-  const bool enough = base >= K;
+  if (base < K)
+    for (int e = lane; e < K; e += 64) cols[e] = -1;
   base = 0;
   for (int q0 = 0; q0 < src.out_max; q0 += 64) {
     const size_t q = (size_t)item * src.out_max + q0 + lane;
@@ -51,7 +52,7 @@ __device__ __forceinline__ void sweep_stage(const SweepSource &src, int item, cd
   for (int e = lane; e < K * R; e += 64) {
     const int nu = e / R, j = e - nu * R;
     const int row = rows[j], col = cols[nu];
-    Vs[e] = enough && row >= 0 && col >= 0 ? src.U[(size_t)row * src.ldu + col] : cd{0.0, 0.0};
+    Vs[e] = row >= 0 && col >= 0 ? src.U[(size_t)row * src.ldu + col] : cd{0.0, 0.0};
   }
 }
 
